@@ -312,6 +312,26 @@ int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], 
                         float scale, int32_t* status, void* stream);
 
 /*
+ * The same with device scratch (16-byte aligned, any contents) of at least
+ * prism_paged_prefill_workspace_bytes() bytes for the same geometry, which is
+ * 0 where none is used.  With it, few query blocks behind long contexts have
+ * their keys split over several workgroups, whose fp32 partials a second
+ * kernel merges; with less, or NULL, every block is one workgroup's.
+ */
+int64_t prism_paged_prefill_workspace_bytes(int batch, int total_q, int num_heads, int num_kv_heads, int page_size,
+                                            int width);
+
+int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,
+                           const void* v_cache, int cache_dtype, const int64_t k_strides[4],
+                           const int64_t v_strides[4], const float* k_scale, const float* v_scale,
+                           const int64_t ks_strides[3], const int64_t vs_strides[3],
+                           const int32_t* block_tables, const int64_t bt_strides[2],
+                           const int32_t* context_lens, const int32_t* cu_seqlens_q, void* out,
+                           const int64_t out_strides[3], int batch, int total_q, int num_heads,
+                           int num_kv_heads, int head_dim, int page_size, int num_blocks, int width,
+                           float scale, int32_t* status, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Test hook with no counterpart in the reference: converts n fp32 values to
  * E4M3FN bytes with the exact device routine the scaled store uses (native
  * gfx950 conversion plus the NaN rule), so the rounding can be checked

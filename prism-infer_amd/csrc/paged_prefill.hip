@@ -8,38 +8,58 @@
 // is fp32 (payload * scale applied to the fp32 scores and to P), as the
 // decode kernels do; the reference multiplies in q's dtype.
 //
-// Work layout.  A workgroup owns one kv head and one block of 32 query
-// tokens of one sequence; its G waves are the G query heads of the kv head,
-// so each K/V tile is read once into LDS for all of them.  Tiles of KT keys
-// (one page holds whole tiles) are double buffered through LDS: the next
-// tile's loads are in flight while the current one is computed.  Per
-// 16-key sub-block, a wave computes S^T = K Q^T (bf16 queries: the fp8 MFMA
-// 16x16x128 on the K bytes as they are, the query split into two fp8 terms
-// that hold it exactly, products exact in fp32; f16 queries:
-// v_mfma_f32_16x16x32_f16 on K converted to f16, exact; the key scale
-// multiplies the rows of S^T), runs the online softmax per query column
-// (log2 domain, lazy rescaling), and accumulates O^T += V^T P^T with
-// v_mfma_f32_16x16x32_bf16 (v_mfma_f32_16x16x16_bf16 for 16-key steps), V^T
-// coming from ds_read_b64_tr_b8 (fp8 -> bf16 is exact) and P * v_scale
-// entering as bf16, whose fp32 exponent range holds every v scale from the
-// 1e-6 floor up.  Only tiles on the diagonal apply the causal mask.
+// Work layout.  A workgroup owns one kv head and one block of query tokens of
+// one sequence; a wave owns 32 of the tokens and one of the G query heads of
+// the kv head, so each K/V tile is read once into LDS for all of them (4 waves:
+// 32 tokens for G = 4, 64 and 128 for G = 2 and 1; 8 waves for G = 8).  Tiles of 64 keys
+// are double buffered through LDS: the next tile's loads are in flight while
+// the current one is computed.  Per tile a wave computes S^T = K Q^T with
+// 32x32 MFMAs (bf16 queries: the fp8 MFMA 32x32x64 on the K bytes as they
+// are, the query split into two fp8 terms that hold it exactly, products
+// exact in fp32; f16 queries: v_mfma_f32_32x32x16_f16 on K converted to f16,
+// exact; the key scale multiplies the rows of S^T), runs the online softmax
+// per query column (log2 domain, lazy rescaling), and accumulates O^T += V^T
+// P^T with v_mfma_f32_32x32x16_bf16, V^T coming from ds_read_b64_tr_b8 (fp8
+// -> bf16 is exact) and P * v_scale entering as bf16, whose fp32 exponent
+// range holds every v scale from the 1e-6 floor up.  Only tiles on the
+// diagonal apply the causal mask.
+//
+// A query is one lane column from the scores to the output (S^T and O^T
+// share it), so the running max, the sum and the rescaling of the
+// accumulators are lane-local, and a column's max needs one lane swap.
+//
+// Few, long blocks (a short chunk behind a long prefix) leave most CUs idle:
+// the keys of a block are then split over several workgroups, which write
+// fp32 partials (max, sum, unnormalised output), merged by a second kernel
+// (330 tokens behind 12000-token prefixes, 32 / 8 heads: 371 us on 88
+// workgroups, 110 + 9.6 us on 440).
+//
+// Bound by VALU issue beside the MFMAs: per 32 x 32 scores of a wave the MFMAs
+// take 512 cycles (4 fp8 and 8 bf16) and the softmax, the
+// scales and the V conversion about 140 instructions.  With 16x16 MFMAs (four
+// lane groups per score column, outputs as query rows) the same work took
+// 193: 4 x 2048 tokens behind 8192, 32 / 8 heads, 1585 us against 1390 here
+// (890 TFLOP/s); 6 prompts of 61 to 1900 tokens, kernel 219 against 182 us.
 //
 // Metadata stays on the device: each workgroup finds its sequence and query
-// block from cu_seqlens_q with a wave scan.  Invalid lengths or block ids
-// record the lowest offending sequence in status[0] (atomicMin); the host
-// raises the reference's error for it.
+// block from cu_seqlens_q with wave reductions, longest blocks first.
+// Invalid lengths or block ids record the lowest offending sequence in
+// status[0] (atomicMin); the host raises the reference's error for it.
 #include "common.h"
 #include "fp8_mfma.h"
+
+#include <algorithm>
 
 namespace prism {
 namespace {
 
-constexpr int kPfD = 128;                      // head dim
-constexpr int kPfCols = 16;                    // query tokens per MFMA column block
-constexpr int kPfColBlocks = 2;                // column blocks per wave
-constexpr int kPfQTile = kPfCols * kPfColBlocks;  // query tokens per workgroup
-constexpr int kPfMaxWaves = 8;                 // GQA group size limit
-constexpr float kPfRescaleThreshold = 8.0f;    // log2 units
+constexpr int kPfD = 128;                    // head dim
+constexpr int kPfCols = 32;                  // query tokens per wave: the columns of a 32x32 MFMA
+constexpr int kPfKT = 64;                    // keys per tile
+constexpr int kPfMaxWaves = 8;               // GQA group size limit
+constexpr float kPfRescaleThreshold = 8.0f;  // log2 units
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 struct PrefillArgs {
   const void* q;
@@ -59,6 +79,10 @@ struct PrefillArgs {
   int batch, num_heads, groups, page, num_blocks, width;
   float scale_log2;
   int* status;
+  int out_vec;    // output rows can be stored 8 bytes at a time
+  int splits;     // workgroups per (block, kv head)
+  int total_q;
+  float* part;    // [splits][total_q][num_heads][kPfD] unnormalised outputs, then [..][2] (max, sum)
 };
 
 // 16-byte chunk swizzle of a key row in LDS, by the key's index t.  gfx950
@@ -67,12 +91,12 @@ struct PrefillArgs {
 // passes; ds_read_b128 serves 16 lanes per pass, the lanes whose bit 5 and
 // parity of bits 2..4 agree.  A 128-byte key row puts bit 7 of the address
 // at t & 1, so a row's 8 chunks cover one half of the banks and rows of
-// opposite parity the other half.  The swizzle (GF(2)-linear in t: chunk
-// ^= 4 t1 ^ 3 t2) makes both reads below conflict-free under that model: the
-// K rows' b128 reads (lane (g, c): row c, chunks 2g and 2g + 1) and the V
-// tiles' transposed b64 reads (lane (g, c): rows 4g + (c >> 1 & 3), chunk
-// 2 jp + (c >> 3)); the previous swizzle cost 4 and 2 extra cycles per read.
-__device__ __forceinline__ int pf_swz(int t) { return (((t >> 1) & 1) * 4) ^ (((t >> 2) & 1) * 3); }
+// opposite parity the other half.  With chunk ^= 4 t1 ^ t2 ^ 2 t3 both reads
+// below are conflict-free under that model.  K rows (b128, lane (g, r): row
+// r, chunk 2g + const): a pass holds every t1, t2, t3 once per row parity,
+// eight distinct chunks.  V (transposed b64, a half wave: rows 4g + 0..3 and
+// 8 more, chunks 2n and 2n + 1): t1, t3 and the chunk's own bit 0 vary.
+__device__ __forceinline__ int pf_swz(int t) { return (((t >> 1) & 1) * 4) | ((t >> 2) & 1) | (((t >> 3) & 1) * 2); }
 
 // A wave-uniform pointer, moved to SGPRs.
 __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
@@ -97,36 +121,72 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
+template <typename F>
+__device__ __forceinline__ int wave_reduce(int v, F f) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) v = f(v, __shfl_xor(v, off));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
 // Query blocks of sequence i (0 for a sequence with invalid lengths, which
-// is flagged).
-__device__ __forceinline__ int seq_blocks(const PrefillArgs& a, int i, bool flag) {
+// is flagged) and the level of its block 0: block j ends after about
+// QT (level + j) keys.
+template <int QT>
+__device__ __forceinline__ int seq_blocks(const PrefillArgs& a, int i, bool flag, int& level0) {
   const int q0 = a.cu_q[i];
   const int qlen = a.cu_q[i + 1] - q0;
   const int ctx = a.ctx[i];
   if (qlen <= 0 || ctx < qlen || ctx > a.width * a.page) {
     if (flag) flag_sequence(a, i);
+    level0 = 0;
     return 0;
   }
-  return (qlen + kPfQTile - 1) / kPfQTile;
+  level0 = (ctx - qlen) / QT + 1;
+  return (qlen + QT - 1) / QT;
 }
 
-// Workgroup -> (sequence, query block).  Blocks are numbered in reverse so
-// that the last (longest) query blocks start first.  Returns false for a
-// workgroup beyond the real blocks.
-__device__ bool locate(const PrefillArgs& a, int& seq, int& qblock) {
+// Rank (0 first) -> (sequence, query block), the blocks with most keys first:
+// the launch then ends on short blocks.  Blocks above a level u: a sum over
+// the sequences; the rank's level comes from a binary search over u, its
+// sequence from a scan over those with a block at that level.  Returns false
+// for a rank beyond the real blocks.
+template <int QT>
+__device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int& qblock) {
   const int lane = __lane_id();
-  int total = 0;
+  if (a.batch <= 64) {  // one lane per sequence, loaded once
+    int l0 = 0;
+    const int n = lane < a.batch ? seq_blocks<QT>(a, lane, flag, l0) : 0;
+    int lo = 0, hi = wave_reduce(n == 0 ? 0 : l0 + n, [](int x, int y) { return max(x, y); });
+    if (rank >= wave_reduce(n, [](int x, int y) { return x + y; })) return false;
+    auto above = [&](int u) { return min(max(l0 + n - 1 - max(u, l0 - 1), 0), n); };
+    // smallest u in [0, hi] with at most `rank` blocks above level u
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (wave_reduce(above(mid), [](int x, int y) { return x + y; }) <= rank) hi = mid;
+      else lo = mid + 1;
+    }
+    const int at = (n > 0 && lo >= l0 && lo < l0 + n) ? 1 : 0;
+    const int first = wave_reduce(above(lo), [](int x, int y) { return x + y; });
+    const int incl = wave_scan(at) + first;
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(at && incl == rank + 1);
+    const int l = __builtin_ctzll(hit);
+    seq = __builtin_amdgcn_readfirstlane(l);
+    qblock = lo - __builtin_amdgcn_readfirstlane(__shfl(l0, l));
+    return true;
+  }
+  // larger batches: sequence by sequence, in reverse
+  int total = 0, l0;
   for (int base = 0; base < a.batch; base += 64) {
     const int i = base + lane;
-    const int n = i < a.batch ? seq_blocks(a, i, blockIdx.y == 0 && blockIdx.x == 0 && threadIdx.x < 64) : 0;
+    const int n = i < a.batch ? seq_blocks<QT>(a, i, flag, l0) : 0;
     total += __shfl(wave_scan(n), 63);
   }
-  const int target = total - 1 - static_cast<int>(blockIdx.x);
+  const int target = total - 1 - rank;
   if (target < 0) return false;
   int before = 0;
   for (int base = 0; base < a.batch; base += 64) {
     const int i = base + lane;
-    const int n = i < a.batch ? seq_blocks(a, i, false) : 0;
+    const int n = i < a.batch ? seq_blocks<QT>(a, i, false, l0) : 0;
     const int incl = wave_scan(n) + before;
     const uint64_t hit = __builtin_amdgcn_ballot_w64(i < a.batch && target < incl && target >= incl - n);
     if (hit != 0) {
@@ -140,12 +200,12 @@ __device__ bool locate(const PrefillArgs& a, int& seq, int& qblock) {
   return false;
 }
 
-// Query operand (B of S^T = K Q^T); lane (g, c) holds query column c's
-// dims 32g..32g+31, the same dims as the K bytes it meets (row c of the
-// block, LDS chunks 2g and 2g + 1); `mul` turns the column's scores into
-// log2 units.
+// Query operand (B of S^T = K Q^T).  Lane (g, c), g = lane / 32, holds query
+// column c's dims 64 kh + 32 g .. + 31 for the two halves kh, the same dims as
+// the K bytes it meets (row c of the block, LDS chunks 4 kh + 2 g and + 1);
+// `mul` turns the column's scores into log2 units.
 //
-// bf16 queries: the fp8 MFMA (16x16x128) on the K bytes as they are.  The
+// bf16 queries: the fp8 MFMA (32x32x64) on the K bytes as they are.  The
 // column is scaled by 2^e so that its largest |q| lies in [128, 256) and
 // split into two E4M3FN terms (hi, lo).  A bf16 value there is M * 2^k with
 // an 8-bit M; hi rounds it to 4 significant bits, which leaves
@@ -155,395 +215,398 @@ __device__ bool locate(const PrefillArgs& a, int& seq, int& qblock) {
 // largest), as a third term would be.  The score is (K . (hi + lo)) * 2^-e;
 // 2^-e joins the softmax scale in `mul`.
 //
-// f16 queries (11 bits, which two terms do not hold): K converted to f16 per
-// block (exact) and v_mfma_f32_16x16x32_f16.
+// f16 queries (11 bits, which two terms do not hold): K converted to f16
+// (exact) and v_mfma_f32_32x32x16_f16.
 template <int QDT>
 struct PfQOperand {
-  i32x8 t[2];  // hi, lo
-  float mul;   // scale_log2 * 2^-e of this lane's column
+  i32x8 t[2][2];  // [lo, hi][half]
+  float mul;      // scale_log2 * 2^-e of this lane's column
 };
 
 template <>
 struct PfQOperand<PRISM_DTYPE_F16> {
-  f16x8 op[4];
+  f16x8 op[2][4];
   float mul;  // scale_log2
 };
 
 template <int QDT>
 __device__ __forceinline__ void pf_load_q(const uint16_t* src, bool valid, float scale_log2, PfQOperand<QDT>& q) {
+  u32x4 w[2][4];
+#pragma unroll
+  for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc)
+      w[kh][cc] = valid ? *reinterpret_cast<const u32x4*>(src + 64 * kh + 8 * cc) : u32x4{0u, 0u, 0u, 0u};
   if constexpr (QDT == PRISM_DTYPE_F16) {
 #pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      const u32x4 w = valid ? *reinterpret_cast<const u32x4*>(src + 8 * cc) : u32x4{0u, 0u, 0u, 0u};
-      q.op[cc] = __builtin_bit_cast(f16x8, w);
-    }
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) q.op[kh][cc] = __builtin_bit_cast(f16x8, w[kh][cc]);
     q.mul = scale_log2;
   } else {
-    float x[32];
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      const u32x4 w = valid ? *reinterpret_cast<const u32x4*>(src + 8 * cc) : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[8 * cc + 2 * e] = bf16_bits_to_f32(w[e] & 0xFFFFu);
-        x[8 * cc + 2 * e + 1] = bf16_bits_to_f32(w[e] >> 16);
-      }
-    }
     float mx = 0.f;
 #pragma unroll
-    for (int e = 0; e < 32; ++e) mx = fmaxf(mx, fabsf(x[e]));
-    mx = wave_max_across_groups(mx);
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          mx = fmaxf(mx, fmaxf(fabsf(bf16_bits_to_f32(w[kh][cc][e] & 0xFFFFu)), fabsf(bf16_bits_to_f32(w[kh][cc][e] >> 16))));
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     // ilogb(mx) = frexp exponent - 1; clamped so that 2^-e stays a normal
     // fp32 number (columns of zeros, or of non-finite values, keep e = 0)
     const int e = (mx > 0.f && mx <= 3.0e38f) ? min(max(8 - __builtin_amdgcn_frexp_expf(mx), -120), 120) : 0;
     q.mul = ldexpf(scale_log2, -e);
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      const float y[4] = {ldexpf(x[4 * w], e), ldexpf(x[4 * w + 1], e), ldexpf(x[4 * w + 2], e),
-                          ldexpf(x[4 * w + 3], e)};
-      uint32_t parts[2];
-      fp8_split<2>(y, parts);
-      q.t[0][w] = static_cast<int>(parts[0]);
-      q.t[1][w] = static_cast<int>(parts[1]);
-    }
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        const uint32_t w0 = w[kh][d / 2][2 * (d % 2)], w1 = w[kh][d / 2][2 * (d % 2) + 1];
+        const float y[4] = {ldexpf(bf16_bits_to_f32(w0 & 0xFFFFu), e), ldexpf(bf16_bits_to_f32(w0 >> 16), e),
+                            ldexpf(bf16_bits_to_f32(w1 & 0xFFFFu), e), ldexpf(bf16_bits_to_f32(w1 >> 16), e)};
+        uint32_t parts[2];
+        fp8_split<2>(y, parts);
+        q.t[1][kh][d] = static_cast<int>(parts[0]);
+        q.t[0][kh][d] = static_cast<int>(parts[1]);
+      }
   }
 }
 
+// Eight transposed reads of a 32-key half tile: ad[n] are the addresses of
+// dim tile n for the first 16 keys, 16 rows further for the next; one wait.
+template <int OFF>
+__device__ __forceinline__ void pf_read_v(const uint32_t (&ad)[4], uint64_t (&v0)[4], uint64_t (&v1)[4]) {
+  lds_read_tr8_x8<OFF, OFF + 16 * kPfD>(ad, v0, v1);
+}
+
 // Two waves per SIMD: at most 256 VGPRs + AGPRs per lane.
-template <int QDT, int KT, int NW, bool SCALED>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+// G: query heads per kv head; WHOLE: a tile lies in one page (page % 64 == 0),
+// else its 16-key groups are looked up one by one.
+constexpr int pf_waves(int g) { return g <= 4 ? 4 : 8; }
+constexpr int pf_qtile(int g) { return kPfCols * pf_waves(g) / g; }
+
+template <int QDT, int G, bool SCALED, bool WHOLE>
+__global__ void __launch_bounds__(64 * pf_waves(G)) __attribute__((amdgpu_waves_per_eu(2)))
 paged_prefill_kernel(const PrefillArgs a) {
-  constexpr int kRow = kPfD;                  // one key's payload row in LDS (bytes)
-  constexpr int kPayload = KT * kRow;         // K or V payload of a tile
-  constexpr int kStage = 2 * kPayload + 2 * KT * 4;
-  constexpr int kChunks = 2 * KT * (kRow / 16);  // 16-byte payload chunks per tile (K then V)
-  constexpr int NB = KT >= 32 ? 2 : 1;            // 16-key blocks per softmax step
-  constexpr int kStep = 16 * NB;                  // keys per softmax step
-  static_assert(NB == 1 || KT / kStep <= 2, "the V reads below cover two steps per tile");
-  using POp = typename std::conditional<NB == 2, bf16x8, shortx4>::type;  // P * v_scale, bf16 (bits for NB = 1)
+  constexpr int NW = pf_waves(G);
+  constexpr int QT = pf_qtile(G);
+  constexpr int kRow = kPfD;                   // one key's payload row in LDS (bytes)
+  constexpr int kPayload = kPfKT * kRow;       // K or V payload of a tile
+  constexpr int kStage = 2 * kPayload + 2 * kPfKT * 4;
   __shared__ __attribute__((aligned(256))) uint8_t stages[2 * kStage];
 
+  // workgroup -> (block rank, split, kv head): heads fastest, so that the
+  // long blocks of all heads start first and, with 8 kv heads, each XCD reads
+  // one head's K/V
+  const int kv_heads = a.num_heads / G;
+  const int per_block = kv_heads * a.splits;
+  const int rank = static_cast<int>(blockIdx.x) / per_block;
+  const int rest = static_cast<int>(blockIdx.x) - rank * per_block;
+  const int split = rest / kv_heads;
+  const int h = rest - split * kv_heads;
   int seq, qblock;
-  if (!locate(a, seq, qblock)) return;
-  const int h = blockIdx.y;
-  constexpr int nthreads = 64 * NW;
+  if (!locate<QT>(a, rank, blockIdx.x == 0 && threadIdx.x < 64, seq, qblock)) return;
   const int tid = threadIdx.x;
-  const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / 64);  // uniform: SGPR arithmetic below
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);  // uniform: SGPR arithmetic below
   const int lane = tid % 64;
-  const int c = lane % 16;
-  const int g = lane / 16;
-  const int qhead = h * a.groups + wave;
+  const int c = lane % 32;
+  const int g = lane / 32;
+  const int qhead = h * G + wave % G;
 
   // sequence metadata in SGPRs: every branch on it below is uniform
   const int qs = __builtin_amdgcn_readfirstlane(a.cu_q[seq]);
   const int qlen = __builtin_amdgcn_readfirstlane(a.cu_q[seq + 1]) - qs;
   const int ctx = __builtin_amdgcn_readfirstlane(a.ctx[seq]);
   const int prefix = ctx - qlen;
-  const int qb0 = qblock * kPfQTile;                       // first query token of the block
-  const int qcount = min(kPfQTile, qlen - qb0);
-  const int kend = prefix + qb0 + qcount;                  // keys [0, kend) are needed
-  const int ntiles = (kend + KT - 1) / KT;
+  const int kend = prefix + min((qblock + 1) * QT, qlen);  // keys [0, kend) are needed
+  const int qb0 = qblock * QT + wave / G * kPfCols;        // first query token of the wave
+  const int qpos0 = prefix + qb0;                          // its position: query column 0
+  const int qlast = qpos0 + (qb0 < qlen ? kPfCols : 0) - 1;  // no key past it is visible to the wave
+  const int all_tiles = (kend + kPfKT - 1) / kPfKT;
+  // this workgroup's tiles
+  const int t0 = static_cast<int>(static_cast<int64_t>(all_tiles) * split / a.splits);
+  const int t1 = static_cast<int>(static_cast<int64_t>(all_tiles) * (split + 1) / a.splits);
   const int32_t* bt_row = a.bt + static_cast<int64_t>(seq) * a.bt_sb;
 
-  // ---- query operand (B of S^T = K Q^T): column c of block cb is query
-  // token qb0 + 16 cb + c; lane group g holds dims 32g .. 32g + 31.
-  PfQOperand<QDT> qop[kPfColBlocks];
-  bool colv[kPfColBlocks];
-#pragma unroll
-  for (int cb = 0; cb < kPfColBlocks; ++cb) {
-    const int j = qb0 + cb * kPfCols + c;
-    colv[cb] = j < qlen;
-    const uint16_t* src = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(qs + (colv[cb] ? j : 0)) * a.q_st +
-                          static_cast<int64_t>(qhead) * a.q_sh + 32 * g;
-    pf_load_q<QDT>(src, colv[cb], a.scale_log2, qop[cb]);
-  }
+  PfQOperand<QDT> qop;
+  const bool colv = qb0 + c < qlen;
+  pf_load_q<QDT>(static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(qs + (colv ? qb0 + c : 0)) * a.q_st +
+                     static_cast<int64_t>(qhead) * a.q_sh + 32 * g,
+                 colv, a.scale_log2, qop);
 
-  // ---- tile loads, straight into LDS (load-to-LDS, 16 B per lane): K then
-  // V as kChunks 16-byte chunks; chunk i of the stage lands at byte 16 i,
-  // i.e. key row i / 8, LDS chunk i % 8, which holds the row's global chunk
-  // (i % 8) ^ swz(row).  Scales: threads 0..2KT-1 one float each.
+  // ---- tile loads, straight into LDS (load-to-LDS, 16 B per lane): K rows,
+  // V rows, K scales, V scales.  A wave's load covers 8 rows: LDS chunk x of
+  // row t holds the row's global chunk x ^ swz(t).  Every load of a wave is
+  // in one 16-key group and is all K or all V: a uniform 64-bit base (SGPRs)
+  // plus a 32-bit per-lane offset that does not change from tile to tile (the
+  // host checks that a page's rows of one head span less than 2 GiB).
   // Asm so that the compiler's wait-count pass does not drain these loads
   // before each LDS read of the other stage.
-  // (waves past the last chunk or scale issue nothing: the waits below are
-  // vmcnt(0), so waves need not issue equal numbers of loads)
-  static_assert(kChunks % 64 == 0, "whole waves of chunks");
-  constexpr int kPer = (kChunks + nthreads - 1) / nthreads;  // chunks per thread
-  bool tile_ok = true;
-  auto issue_tile = [&](int t, uint8_t* st) {
-    const int tok0 = t * KT;
-    const int page = tok0 / a.page;
-    const int32_t blk = bt_row[static_cast<int64_t>(page) * a.bt_sn];
-    tile_ok = blk >= 0 && blk < a.num_blocks;
-    if (!tile_ok) {
-      if (tid == 0) flag_sequence(a, seq);
-      return;
+  // (the waits below are vmcnt(0), so that waves need not issue equal numbers
+  // of loads)
+  // (the 8-row groups of a wave have the parity of the wave: NW is even)
+  uint32_t k_off, v_off;
+  {
+    const int r = lane / 8;
+    const int part = (lane % 8) ^ pf_swz(8 * (wave & 1) + r);
+    k_off = static_cast<uint32_t>(r * static_cast<int>(a.k_sp) + part * 16);
+    v_off = static_cast<uint32_t>(r * static_cast<int>(a.v_sp) + part * 16);
+  }
+  // Block ids: 64 consecutive entries of the table row in one register,
+  // renewed every 64 pages; (pg, row) walk the pages without divisions.
+  int pg = t0 * kPfKT / a.page;
+  int row = t0 * kPfKT - pg * a.page;
+  int ids_base = pg;
+  auto load_ids = [&](int base) { return bt_row[static_cast<int64_t>(min(base + lane, a.width - 1)) * a.bt_sn]; };
+  int ids = load_ids(ids_base);
+  auto block_at = [&](int page) {
+    if (page >= ids_base + 64) {
+      ids_base = page;
+      ids = load_ids(ids_base);
     }
-    const int row0 = tok0 - page * a.page;
-    const uint32_t st_lds = lds_addr(st);
-    // every chunk of a wave is in one page and is all K or all V: a uniform
-    // 64-bit base (SGPRs) plus a 32-bit per-lane offset (the host checks
-    // that a page's bytes of one head span less than 2^31)
+    return __builtin_amdgcn_readlane(ids, page - ids_base);
+  };
+  auto load_chunks = [&](const uint8_t* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 : : "v"(off), "s"(uniform_ptr(base)), "s"(lds) : "memory", "m0");
+  };
+  auto issue_tile = [&](int t, uint8_t* st) -> bool {
+    constexpr int kGroups = WHOLE ? 1 : kPfKT / 16;  // table lookups per tile
+    constexpr int kGroupRows = kPfKT / kGroups;
+    int blk[kGroups], row0[kGroups];
+    bool ok = true;
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int ch0 = k * nthreads + wave * 64;  // the wave's first chunk (uniform); 64 contiguous chunks
-      const int ch = ch0 + lane;
-      if (ch0 >= kChunks) break;
-      const int isv = ch0 >= kChunks / 2;
-      const int cw = ch - isv * (kChunks / 2);
-      const int tok = cw / (kRow / 16);
-      const int part = (cw % (kRow / 16)) ^ pf_swz(tok);
-      const uint8_t* base = isv ? a.v + blk * a.v_sn + static_cast<int64_t>(row0) * a.v_sp + h * a.v_sh
-                                : a.k + blk * a.k_sn + static_cast<int64_t>(row0) * a.k_sp + h * a.k_sh;
-      const uint32_t off = static_cast<uint32_t>(tok * static_cast<int>(isv ? a.v_sp : a.k_sp) + part * 16);
-      const uint32_t m0 = __builtin_amdgcn_readfirstlane(st_lds + static_cast<uint32_t>(ch0) * 16);
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(uniform_ptr(base)),
-                   "s"(m0) : "memory", "m0");
-    }
-    if constexpr (SCALED) {
-      // threads 0..KT-1 load the K scales, KT..2KT-1 the V scales (exec-masked
-      // halves of one wave share M0: the LDS address is M0 + 4 * lane)
-      const int si = tid;
-      const uint32_t m0 = __builtin_amdgcn_readfirstlane(st_lds + 2 * kPayload + static_cast<uint32_t>(wave * 64) * 4);
-      if (si < KT) {
-        const uint8_t* base = uniform_ptr(reinterpret_cast<const uint8_t*>(
-            a.ks + blk * a.ks_sn + static_cast<int64_t>(row0) * a.ks_sp + h * a.ks_sh));
-        const uint32_t off = static_cast<uint32_t>(si * static_cast<int>(a.ks_sp) * 4);
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(m0)
-                     : "memory", "m0");
-      } else if (si < 2 * KT) {
-        const uint8_t* base = uniform_ptr(reinterpret_cast<const uint8_t*>(
-            a.vs + blk * a.vs_sn + static_cast<int64_t>(row0) * a.vs_sp + h * a.vs_sh));
-        const uint32_t off = static_cast<uint32_t>((si - KT) * static_cast<int>(a.vs_sp) * 4);
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(m0)
-                     : "memory", "m0");
+    for (int x = 0; x < kGroups; ++x) {
+      blk[x] = -1;
+      row0[x] = row;
+      if (WHOLE || t * kPfKT + x * kGroupRows < kend) {  // groups past the keys needed are not looked up
+        blk[x] = block_at(pg);
+        ok = ok && blk[x] >= 0 && blk[x] < a.num_blocks;
+        row += kGroupRows;
+        if (row == a.page) {
+          row = 0;
+          ++pg;
+        }
       }
-    } else {
-      if (tid < 2 * KT) reinterpret_cast<float*>(st + 2 * kPayload)[tid] = 1.f;
     }
+    if (!ok) {
+      if (tid == 0) flag_sequence(a, seq);
+      return false;
+    }
+    const uint32_t st_lds = lds_addr(st);
+    constexpr int kLoads = 2 * kPfKT / 8 / NW;  // 8-row loads per wave, the first half of them K
+#pragma unroll
+    for (int l = 0; l < kLoads; ++l) {
+      const bool isv = l >= kLoads / 2;
+      const int tr = ((isv ? l - kLoads / 2 : l) * NW + wave) * 8;  // first row in the tile
+      const int x = WHOLE ? 0 : tr / 16;
+      int b = blk[0], pr = row0[0] + tr;
+      if constexpr (!WHOLE) {
+#pragma unroll
+        for (int y = 1; y < kGroups; ++y)
+          if (x == y) b = blk[y], pr = row0[y] + tr - 16 * y;
+        if (b < 0) continue;
+      }
+      const uint8_t* base = isv ? a.v + b * a.v_sn + static_cast<int64_t>(pr) * a.v_sp + h * a.v_sh
+                                : a.k + b * a.k_sn + static_cast<int64_t>(pr) * a.k_sp + h * a.k_sh;
+      load_chunks(base, isv ? v_off : k_off,
+                  __builtin_amdgcn_readfirstlane(st_lds + (isv ? kPayload : 0) + static_cast<uint32_t>(tr) * kRow));
+    }
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      if (which != wave) continue;
+      const uint32_t lds = __builtin_amdgcn_readfirstlane(st_lds + 2 * kPayload + static_cast<uint32_t>(which) * kPfKT * 4);
+      if constexpr (SCALED) {
+        const float* s = which ? a.vs : a.ks;
+        const int64_t sn = which ? a.vs_sn : a.ks_sn, sp = which ? a.vs_sp : a.ks_sp, sh = which ? a.vs_sh : a.ks_sh;
+        if constexpr (WHOLE) {
+          const uint8_t* base = uniform_ptr(reinterpret_cast<const uint8_t*>(s + blk[0] * sn + row0[0] * sp + h * sh));
+          const uint32_t off = static_cast<uint32_t>(lane * static_cast<int>(sp) * 4);
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds)
+                       : "memory", "m0");
+        } else {
+          int b = blk[0], pr = row0[0];
+#pragma unroll
+          for (int y = 1; y < kGroups; ++y)
+            if (lane / 16 == y) b = blk[y], pr = row0[y];
+          const float* src = s + b * sn + static_cast<int64_t>(pr + lane % 16) * sp + h * sh;
+          if (b >= 0)
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds)
+                         : "memory", "m0");
+        }
+      } else {
+        reinterpret_cast<float*>(st + 2 * kPayload)[which * kPfKT + lane] = 1.f;
+      }
+    }
+    return true;
   };
 
-  floatx4 acc[kPfColBlocks][8];
-  float m_run[kPfColBlocks], l_run[kPfColBlocks];
+  floatx16 acc[4];  // O^T: dims 32 n + 8 (r / 4) + 4 g + r % 4 of query column c
 #pragma unroll
-  for (int cb = 0; cb < kPfColBlocks; ++cb) {
+  for (int n = 0; n < 4; ++n)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[cb][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    m_run[cb] = -INFINITY;
-    l_run[cb] = 0.f;
-  }
+    for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
 
-  // per-lane LDS offsets inside a stage for sub-block 0 (add 16 rows per sub-block)
-  const uint32_t k_off0 = c * kRow + (((2 * g) ^ pf_swz(c)) << 4);
-  const uint32_t k_off1 = c * kRow + (((2 * g + 1) ^ pf_swz(c)) << 4);
-  uint32_t v_off[4];
-  {
-    const int r = c >> 1;
-    const int t = 4 * g + (r & 3);
-    const int half = c & 1;
+  // per-lane LDS offsets inside a stage, for keys 0..31 (32 rows further for the rest)
+  uint32_t k_rd[4];
 #pragma unroll
-    for (int jp = 0; jp < 4; ++jp) {
-      const int chunk = 2 * jp + (r >> 2);
-      v_off[jp] = kPayload + t * kRow + ((chunk ^ pf_swz(t)) << 4) + half * 8;
-    }
+  for (int x = 0; x < 4; ++x) k_rd[x] = c * kRow + (((4 * (x / 2) + 2 * g + x % 2) ^ pf_swz(c)) << 4);
+  uint32_t v_rd[4];
+  {
+    const int r = (lane % 16) >> 1;
+    const int t = 8 * (r >> 2) + 4 * g + (r & 3);  // key of the 16-key group
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      v_rd[n] = kPayload + t * kRow + (((2 * n + (lane / 16) % 2) ^ pf_swz(t)) << 4) + (lane & 1) * 8;
   }
   const uint32_t stage_base = lds_addr(stages);
-  const int qpos0 = prefix + qb0;  // position of query column 0 of block 0
 
-  issue_tile(0, stages);
-  bool cur_ok = tile_ok;
+  bool cur_ok = t0 < t1 ? issue_tile(t0, stages) : false;
   __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const bool more = t + 1 < ntiles;
+  for (int t = t0; t < t1; ++t) {
+    const uint32_t soff = static_cast<uint32_t>((t - t0) & 1) * kStage;
     // the next tile streams into the other stage, last read by tile t - 1,
     // which every wave finished before the barrier that ended that iteration
-    bool next_ok = true;
-    if (more) {
-      issue_tile(t + 1, stages + ((t + 1) & 1) * kStage);
-      next_ok = tile_ok;
-    }
-    const uint32_t soff = static_cast<uint32_t>(t & 1) * kStage;
+    const bool next_ok = t + 1 < t1 ? issue_tile(t + 1, stages + (kStage - soff)) : true;
     const uint8_t* st = stages + soff;
-    if (cur_ok) {
+    const int key0 = t * kPfKT;
+    if (cur_ok && key0 <= qlast) {
+      const float* scl = reinterpret_cast<const float*>(st + 2 * kPayload) + 4 * g;
+      // S^T = K Q^T, two chains of 32 keys; the second is skipped above the
+      // diagonal (uniform branch)
+      const bool both = key0 + 32 <= qlast;
+      floatx16 sc[2];
 #pragma unroll
-      for (int sp = 0; sp < KT / kStep; ++sp) {
-        const int key0 = t * KT + sp * kStep;                // first key of the step
-        if (key0 > qpos0 + kPfQTile - 1) break;              // above the diagonal for every column
-        // per 16-key block b: K rows, scales and the transposed V reads
-        u32x4 kw[NB][2];
-        floatx4 ksv[NB];
-        uint64_t vt[NB][4];
+      for (int b = 0; b < 2; ++b) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const int sb = sp * NB + b;
-          const uint8_t* sbp = st + sb * 16 * kRow;
-          kw[b][0] = *reinterpret_cast<const u32x4*>(sbp + k_off0);
-          kw[b][1] = *reinterpret_cast<const u32x4*>(sbp + k_off1);
-          const float* scl = reinterpret_cast<const float*>(st + 2 * kPayload) + sb * 16 + 4 * g;
-          ksv[b] = *reinterpret_cast<const floatx4*>(scl);
+        for (int r = 0; r < 16; ++r) sc[b][r] = 0.f;
+        u32x4 kw[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) kw[x] = *reinterpret_cast<const u32x4*>(st + b * 32 * kRow + k_rd[x]);
+        if constexpr (QDT == PRISM_DTYPE_F16) {
+#pragma unroll
+          for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc) {
+              const u32x4& w = kw[2 * kh + cc / 2];
+              sc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fp8x8_to_f16x8(w[2 * (cc % 2)], w[2 * (cc % 2) + 1]),
+                                                             qop.op[kh][cc], sc[b], 0, 0, 0);
+            }
+        } else {
+          // the K bytes are the fp8 MFMA's A operand as they are; smaller term first
+          i32x8 ka[2];
+#pragma unroll
+          for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+            for (int x = 0; x < 8; ++x) ka[kh][x] = static_cast<int>(kw[2 * kh + x / 4][x % 4]);
+#pragma unroll
+          for (int term = 0; term < 2; ++term)
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh)
+              sc[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ka[kh], qop.t[term][kh], sc[b], 0, 0, 0, 0, 0, 0);
         }
+      }
+      // score rows: key key0 + 32 b + 8 (r / 4) + 4 g + r % 4
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const floatx4 ksv = *reinterpret_cast<const floatx4*>(scl + 32 * b + 8 * i);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sc[b][4 * i + j] *= ksv[j];  // score / softmax scale
+        }
+      // causal mask: key k is visible to column c iff it is at or before the
+      // query's position.  Tiles wholly below the diagonal need no mask
+      // (uniform branch); columns without a query hold q = 0 there, so their
+      // scores stay finite and their rows are never written.
+      const bool masked = key0 + kPfKT - 1 > qpos0;
+      if (masked) {
+        const int last = colv ? qpos0 + c - key0 - 4 * g : -1;  // last visible key, as a row offset
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            sc[b][r] = 32 * b + 8 * (r / 4) + r % 4 <= last ? sc[b][r] : -INFINITY;
+      }
+      float tmax = fmaxf(sc[0][0], sc[1][0]);
+#pragma unroll
+      for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, fmaxf(sc[0][r], sc[1][r]));
+      {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+        tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * qop.mul;  // log2 units (mul is positive)
+      }
+      const bool raise = tmax > m_run + kPfRescaleThreshold;
+      if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+        const float m_new = raise ? tmax : m_run;
+        const float alpha = raise ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[n][r] *= alpha;
+      }
+      const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+      // per 32 keys: P (B of O^T += V^T P^T, k-slots 8 g + 0..3 of 16-key group
+      // m are keys 16 m + 4 g + 0..3 and 8 g + 4..7 the keys 8 further, the
+      // order the score rows come out in), then the products
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        if (b == 1 && !both) break;
+        uint64_t vt[2][4];
         {
           uint32_t ad[4];
 #pragma unroll
-          for (int jp = 0; jp < 4; ++jp) ad[jp] = stage_base + soff + v_off[jp];
-          if constexpr (NB == 2) {
-            if (sp == 0) lds_read_tr8_x8<0, 16 * kRow>(ad, vt[0], vt[NB - 1]);
-            else lds_read_tr8_x8<2 * 16 * kRow, 3 * 16 * kRow>(ad, vt[0], vt[NB - 1]);
-          } else {
+          for (int n = 0; n < 4; ++n) ad[n] = stage_base + soff + v_rd[n];
+          if (b == 0) pf_read_v<0>(ad, vt[0], vt[1]);
+          else pf_read_v<32 * kRow>(ad, vt[0], vt[1]);
+        }
+        floatx4 vsv[4];
 #pragma unroll
-            for (int jp = 0; jp < 4; ++jp) ad[jp] += sp * 16 * kRow;
-            lds_read_tr8_x4(ad, vt[0]);
+        for (int i = 0; i < 4; ++i) vsv[i] = *reinterpret_cast<const floatx4*>(scl + kPfKT + 32 * b + 8 * i);
+        // keys past the block's last may hold any bytes and scales (past the
+        // context, or not loaded): zero them (only the block's last tile can
+        // hold such keys; uniform branch)
+        if (key0 + 32 * b + 32 > kend) {
+          const int left = kend - key0 - 32 * b - 4 * g;
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            uint64_t keep = 0;
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj)
+              keep |= (16 * m + 8 * (jj / 4) + jj % 4 < left) ? (uint64_t{0xFF} << (8 * jj)) : 0u;
+#pragma unroll
+            for (int n = 0; n < 4; ++n) vt[m][n] &= keep;
           }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) vsv[i][j] = 8 * i + j < left ? vsv[i][j] : 0.f;
         }
-        // keys past the context end may hold any bytes: zero them in V (only
-        // the context's last step can hold such keys; uniform branch)
-        if (key0 + kStep > ctx) {
+        bf16x8 pa[2];
+        float ps = 0.f;
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            uint32_t keep = 0;
+        for (int i = 0; i < 4; ++i) {
+          float p[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) keep |= (key0 + 16 * b + 4 * g + i < ctx) ? (0xFFu << (8 * i)) : 0u;
-            const uint64_t keep2 = static_cast<uint64_t>(keep) | (static_cast<uint64_t>(keep) << 32);
-#pragma unroll
-            for (int jp = 0; jp < 4; ++jp) vt[b][jp] &= keep2;
+          for (int j = 0; j < 4; ++j) {
+            // v_exp_f32: arguments are at most 2^3 above the running max;
+            // results below 2^-126 (flushed to 0) weigh nothing next to it
+            p[j] = __builtin_amdgcn_exp2f(fmaf(sc[b][4 * i + j], qop.mul, -m_use));  // 0 where masked
+            pa[i / 2][4 * (i % 2) + j] = static_cast<__bf16>(p[j] * vsv[i][j]);
           }
+          ps += (p[0] + p[1]) + (p[2] + p[3]);
         }
-        // S^T = K Q^T for both column blocks, NB x 2 independent chains
-        floatx4 sc[kPfColBlocks][NB];
+        l_run += ps;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          if constexpr (QDT == PRISM_DTYPE_F16) {
-            // K converted once per block for both column blocks
-            f16x8 kop[4];
+        for (int m = 0; m < 2; ++m)
 #pragma unroll
-            for (int cc = 0; cc < 4; ++cc) {
-              const u32x4& w = kw[b][cc >> 1];
-              kop[cc] = fp8x8_to_f16x8(w[(cc & 1) * 2], w[(cc & 1) * 2 + 1]);
-            }
-#pragma unroll
-            for (int cb = 0; cb < kPfColBlocks; ++cb) {
-              floatx4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-              for (int cc = 0; cc < 4; ++cc) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[cc], qop[cb].op[cc], d, 0, 0, 0);
-              sc[cb][b] = d;
-            }
-          } else {
-            // the K bytes are the fp8 MFMA's A operand as they are (row =
-            // key c of the block, k = dims 32g..32g+31); smaller term first
-            const i32x8 ka = {static_cast<int>(kw[b][0][0]), static_cast<int>(kw[b][0][1]),
-                              static_cast<int>(kw[b][0][2]), static_cast<int>(kw[b][0][3]),
-                              static_cast<int>(kw[b][1][0]), static_cast<int>(kw[b][1][1]),
-                              static_cast<int>(kw[b][1][2]), static_cast<int>(kw[b][1][3])};
-#pragma unroll
-            for (int cb = 0; cb < kPfColBlocks; ++cb) {
-              floatx4 d = {0.f, 0.f, 0.f, 0.f};
-              d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ka, qop[cb].t[1], d, 0, 0, 0, 0, 0, 0);
-              d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ka, qop[cb].t[0], d, 0, 0, 0, 0, 0, 0);
-              sc[cb][b] = d;
-            }
-          }
-        }
-        // online softmax per column block -> P (A of O = P V).  One block:
-        // k-slots 4g..4g+3 are keys 4g..4g+3 (16x16x16).  Two blocks: k-slots
-        // 8g..8g+3 are keys 4g..4g+3 of block 0 and 8g+4..8g+7 the same keys
-        // of block 1 (16x16x32), the order the score rows come out in.
-        // Both column blocks go through each phase together (one branch per
-        // phase), so their dependency chains interleave.
-        POp pa[kPfColBlocks];
-        float x[kPfColBlocks][NB][4];
-#pragma unroll
-        for (int cb = 0; cb < kPfColBlocks; ++cb)
-#pragma unroll
-          for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[cb][b][i] = sc[cb][b][i] * ksv[b][i];  // score / softmax scale
-        // causal mask: key k is visible to column c iff it is at or before
-        // the query's position.  Steps wholly below the diagonal of both
-        // column blocks need no mask (uniform branch); columns without a
-        // query hold q = 0 there, so their scores stay finite and their rows
-        // are never written.
-        if (key0 + kStep - 1 > qpos0) {
-#pragma unroll
-          for (int cb = 0; cb < kPfColBlocks; ++cb) {
-            const int qpos = qpos0 + cb * kPfCols + c;
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                x[cb][b][i] = (colv[cb] && key0 + 16 * b + 4 * g + i <= qpos) ? x[cb][b][i] : -INFINITY;
-          }
-        }
-        float tmax[kPfColBlocks];
-        bool raise[kPfColBlocks];
-#pragma unroll
-        for (int cb = 0; cb < kPfColBlocks; ++cb) {
-          float t = fmaxf(fmaxf(x[cb][0][0], x[cb][0][1]), fmaxf(x[cb][0][2], x[cb][0][3]));
-          if constexpr (NB == 2) t = fmaxf(t, fmaxf(fmaxf(x[cb][1][0], x[cb][1][1]), fmaxf(x[cb][1][2], x[cb][1][3])));
-          tmax[cb] = wave_max_across_groups(t) * qop[cb].mul;  // log2 units (the multiplier is positive)
-          raise[cb] = tmax[cb] > m_run[cb] + kPfRescaleThreshold;
-        }
-        if (__builtin_amdgcn_ballot_w64(raise[0] || raise[1]) != 0) {
-#pragma unroll
-          for (int cb = 0; cb < kPfColBlocks; ++cb) {
-            const float m_new = raise[cb] ? tmax[cb] : m_run[cb];
-            const float alpha = raise[cb] ? __builtin_amdgcn_exp2f(m_run[cb] - m_new) : 1.f;
-            m_run[cb] = m_new;
-            l_run[cb] *= alpha;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float ai = __shfl(alpha, 4 * g + i);
-#pragma unroll
-              for (int j = 0; j < 8; ++j) acc[cb][j][i] *= ai;
-            }
-          }
-        }
-        // v scales are read here, where P is formed, not with the K scales:
-        // held across the QK MFMAs they push the kernel past 256 VGPRs
-        floatx4 vsv[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-          vsv[b] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(st + 2 * kPayload) + KT +
-                                                     (sp * NB + b) * 16 + 4 * g);
-#pragma unroll
-        for (int cb = 0; cb < kPfColBlocks; ++cb) {
-          const float m_use = (m_run[cb] == -INFINITY) ? 0.f : m_run[cb];
-          float p[NB][4];
-#pragma unroll
-          for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              // v_exp_f32: arguments are at most 2^3 above the running max;
-              // results below 2^-126 (flushed to 0) weigh nothing next to it
-              p[b][i] = __builtin_amdgcn_exp2f(fmaf(x[cb][b][i], qop[cb].mul, -m_use));  // 0 where masked
-              if constexpr (NB == 2) pa[cb][4 * b + i] = static_cast<__bf16>(p[b][i] * vsv[b][i]);
-              else pa[cb][4 * b + i] = __builtin_bit_cast(short, static_cast<__bf16>(p[b][i] * vsv[b][i]));
-            }
-          }
-          float ps = (p[0][0] + p[0][1]) + (p[0][2] + p[0][3]);
-          if constexpr (NB == 2) ps += (p[1][0] + p[1][1]) + (p[1][2] + p[1][3]);
-          l_run[cb] += ps;
-        }
-        // O += P V: V operand (B) for dims 16 j + c, one N-tile at a time,
-        // shared by the column blocks; k-slots as P's
-#pragma unroll
-        for (int jp = 0; jp < 4; ++jp) {
-#pragma unroll
-          for (int hi = 0; hi < 2; ++hi) {
-            const int j = 2 * jp + hi;
-            const uint32_t w0 = static_cast<uint32_t>(vt[0][jp] >> (32 * hi));
-            if constexpr (NB == 2) {
-              const bf16x8 vb = fp8x8_to_bf16x8(w0, static_cast<uint32_t>(vt[NB - 1][jp] >> (32 * hi)));
-#pragma unroll
-              for (int cb = 0; cb < kPfColBlocks; ++cb)
-                acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[cb], vb, acc[cb][j], 0, 0, 0);
-            } else {
-              const shortx4 v0 = fp8x4_to_bf16x4_bits(w0);
-#pragma unroll
-              for (int cb = 0; cb < kPfColBlocks; ++cb)
-                acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa[cb], v0, acc[cb][j], 0, 0, 0);
-            }
-          }
-        }
+          for (int n = 0; n < 4; ++n)
+            acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                fp8x8_to_bf16x8(static_cast<uint32_t>(vt[m][n]), static_cast<uint32_t>(vt[m][n] >> 32)), pa[m], acc[n], 0, 0, 0);
       }
     }
     cur_ok = next_ok;
@@ -551,61 +614,131 @@ paged_prefill_kernel(const PrefillArgs a) {
     __syncthreads();
   }
 
-  // ---- epilogue: acc[cb][j][i] is query column 4g + i of block cb, dim 16j + c
+  // ---- epilogue
+  const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
+  const float l_tot = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
+  if (!colv) return;
+  const int64_t tok = qs + qb0 + c;
+  if (a.splits > 1) {
+    const int64_t cell = (static_cast<int64_t>(split) * a.total_q + tok) * a.num_heads + qhead;
+    float* dst = a.part + cell * kPfD + 4 * g;
 #pragma unroll
-  for (int cb = 0; cb < kPfColBlocks; ++cb) {
-    float l_tot = l_run[cb] + __shfl_xor(l_run[cb], 16);
-    l_tot += __shfl_xor(l_tot, 32);
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<floatx4*>(dst + 32 * n + 8 * i) =
+            floatx4{acc[n][4 * i], acc[n][4 * i + 1], acc[n][4 * i + 2], acc[n][4 * i + 3]};
+    float* ml = a.part + static_cast<int64_t>(a.splits) * a.total_q * a.num_heads * kPfD + 2 * cell;
+    if (g == 0) *reinterpret_cast<floatx2*>(ml) = floatx2{m_run, l_tot};
+    return;
+  }
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  uint16_t* dst = static_cast<uint16_t*>(a.out) + tok * a.o_st + static_cast<int64_t>(qhead) * a.o_sh + 4 * g;
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int qr = 4 * g + i;
-      const float li = __shfl(l_tot, qr);
-      const int j = qb0 + cb * kPfCols + qr;
-      if (j < qlen) {
-        const float inv = li > 0.f ? 1.f / li : 0.f;
-        uint16_t* dst = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(qs + j) * a.o_st +
-                        static_cast<int64_t>(qhead) * a.o_sh + c;
+      uint32_t o[4];
 #pragma unroll
-        for (int jd = 0; jd < 8; ++jd) {
-          const float o = acc[cb][jd][i] * inv;
-          dst[16 * jd] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o) : f32_to_bf16_bits(o);
-        }
+      for (int j = 0; j < 4; ++j) {
+        const float x = acc[n][4 * i + j] * inv;
+        o[j] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(x) : f32_to_bf16_bits(x);
+      }
+      uint16_t* d = dst + 32 * n + 8 * i;
+      if (a.out_vec) {
+        *reinterpret_cast<u32x2*>(d) = u32x2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[j] = static_cast<uint16_t>(o[j]);
       }
     }
+}
+
+// Merges the splits' partials: one wave per (token, query head), two dims per
+// lane.  Rows outside every sequence hold no partials and are skipped, as is
+// a row of an invalid sequence (the status word names it).
+template <int QDT>
+__global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillArgs a) {
+  const int64_t cell = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / 64;
+  const int64_t cells = static_cast<int64_t>(a.total_q) * a.num_heads;
+  if (cell >= cells) return;
+  const int lane = threadIdx.x % 64;
+  const int tok = static_cast<int>(cell / a.num_heads);
+  if (tok < a.cu_q[0] || tok >= a.cu_q[a.batch]) return;
+  const floatx2* ml = reinterpret_cast<const floatx2*>(a.part + a.splits * cells * kPfD) + cell;
+  const floatx2* row = reinterpret_cast<const floatx2*>(a.part) + cell * (kPfD / 2) + lane;
+  float m = -INFINITY;
+  for (int s = 0; s < a.splits; ++s) {
+    const floatx2 x = ml[s * cells];
+    if (x[1] > 0.f) m = fmaxf(m, x[0]);
   }
+  float l = 0.f, o0 = 0.f, o1 = 0.f;
+  for (int s = 0; s < a.splits; ++s) {
+    const floatx2 x = ml[s * cells];
+    const floatx2 v = row[s * cells * (kPfD / 2)];
+    const float w = x[1] > 0.f ? __builtin_amdgcn_exp2f(x[0] - m) : 0.f;
+    l = fmaf(w, x[1], l);
+    o0 = w > 0.f ? fmaf(w, v[0], o0) : o0;
+    o1 = w > 0.f ? fmaf(w, v[1], o1) : o1;
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* dst = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(tok) * a.o_st +
+                  (cell - static_cast<int64_t>(tok) * a.num_heads) * a.o_sh + 2 * lane;
+  dst[0] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o0 * inv) : f32_to_bf16_bits(o0 * inv);
+  dst[1] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o1 * inv) : f32_to_bf16_bits(o1 * inv);
 }
 
-template <int QDT, int KT, int NW>
-int launch_prefill(const PrefillArgs& a, bool scaled, int total_q, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(ceil_div(total_q, kPfQTile) + a.batch),
-                  static_cast<unsigned>(a.num_heads / a.groups));
-  const dim3 block(64 * NW);
-  if (scaled) hipLaunchKernelGGL((paged_prefill_kernel<QDT, KT, NW, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((paged_prefill_kernel<QDT, KT, NW, false>), grid, block, 0, stream, a);
-  return check_launch("paged_prefill_kernel launch");
+// Query blocks that the launch provides for: every sequence may end in a
+// partial block.
+int64_t block_bound(int total_q, int batch, int groups) { return ceil_div(total_q, pf_qtile(groups)) + batch; }
+
+// Workgroups per (block, kv head).  The kernel fits eight waves on a CU; where the blocks give fewer than that, the keys are split so
+// that the launch fills the chip once, in parts of at least 4 tiles of the
+// longest context the tables can hold.
+int split_count(int total_q, int batch, int num_heads, int num_kv_heads, int64_t capacity) {
+  const int groups = num_heads / num_kv_heads;
+  const int64_t wgs = block_bound(total_q, batch, groups) * num_kv_heads;
+  const int64_t slots = static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(groups);
+  const int64_t s = std::min(slots / wgs, capacity / (4 * kPfKT));
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(s, 64)));
 }
 
-// Key tiles of 64, 32 or 16 keys (the largest dividing the page; at most 32
-// for one or two waves); one wave per query head of the GQA group.
-template <int QDT, int KT>
-int dispatch_waves(const PrefillArgs& a, bool scaled, int total_q, hipStream_t stream) {
+int64_t split_workspace(int splits, int total_q, int num_heads) {
+  return splits > 1 ? static_cast<int64_t>(splits) * total_q * num_heads * (kPfD + 2) * 4 : 0;
+}
+
+template <int QDT, int G>
+int launch_prefill(const PrefillArgs& a, bool scaled, hipStream_t stream) {
+  const int64_t blocks = block_bound(a.total_q, a.batch, G) * (a.num_heads / G) * a.splits;
+  if (blocks > INT32_MAX) {
+    set_error("prism_paged_prefill: too many query blocks for one launch");
+    return PRISM_ERR_INVALID;
+  }
+  const dim3 grid(static_cast<unsigned>(blocks)), block(64 * pf_waves(G));
+  const bool whole = a.page % kPfKT == 0;
+  if (scaled && whole) hipLaunchKernelGGL((paged_prefill_kernel<QDT, G, true, true>), grid, block, 0, stream, a);
+  else if (scaled) hipLaunchKernelGGL((paged_prefill_kernel<QDT, G, true, false>), grid, block, 0, stream, a);
+  else if (whole) hipLaunchKernelGGL((paged_prefill_kernel<QDT, G, false, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((paged_prefill_kernel<QDT, G, false, false>), grid, block, 0, stream, a);
+  if (int rc = check_launch("paged_prefill_kernel launch")) return rc;
+  if (a.splits == 1) return PRISM_OK;
+  const int64_t cells = static_cast<int64_t>(a.total_q) * a.num_heads;
+  hipLaunchKernelGGL((paged_prefill_merge_kernel<QDT>), dim3(static_cast<unsigned>(ceil_div(cells, 4))), dim3(256), 0,
+                     stream, a);
+  return check_launch("paged_prefill_merge_kernel launch");
+}
+
+template <int QDT>
+int dispatch_groups(const PrefillArgs& a, bool scaled, hipStream_t stream) {
   switch (a.groups) {
-    case 1: return launch_prefill<QDT, (KT > 32 ? 32 : KT), 1>(a, scaled, total_q, stream);
-    case 2: return launch_prefill<QDT, (KT > 32 ? 32 : KT), 2>(a, scaled, total_q, stream);
-    case 4: return launch_prefill<QDT, KT, 4>(a, scaled, total_q, stream);
-    case 8: return launch_prefill<QDT, KT, 8>(a, scaled, total_q, stream);
+    case 1: return launch_prefill<QDT, 1>(a, scaled, stream);
+    case 2: return launch_prefill<QDT, 2>(a, scaled, stream);
+    case 4: return launch_prefill<QDT, 4>(a, scaled, stream);
+    case 8: return launch_prefill<QDT, 8>(a, scaled, stream);
     default:
       set_error("prism_paged_prefill: GQA group size %d is not 1, 2, 4 or 8", a.groups);
       return PRISM_ERR_LAYOUT;
   }
-}
-
-template <int QDT>
-int dispatch_tile(const PrefillArgs& a, bool scaled, int total_q, hipStream_t stream) {
-  // a tile lies in one page
-  if (a.page % 64 == 0) return dispatch_waves<QDT, 64>(a, scaled, total_q, stream);
-  if (a.page % 32 == 0) return dispatch_waves<QDT, 32>(a, scaled, total_q, stream);
-  return dispatch_waves<QDT, 16>(a, scaled, total_q, stream);
 }
 
 }  // namespace
@@ -613,20 +746,30 @@ int dispatch_tile(const PrefillArgs& a, bool scaled, int total_q, hipStream_t st
 // Loads this file's code object now rather than at its first kernel launch.
 int preload_paged_prefill() {
   hipFuncAttributes attr;
-  return check_hip(hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&paged_prefill_kernel<PRISM_DTYPE_BF16, 64, 4, true>)), "preload_paged_prefill");
+  return check_hip(hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&paged_prefill_kernel<PRISM_DTYPE_BF16, 4, true, true>)), "preload_paged_prefill");
 }
 
 }  // namespace prism
 
-extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,
-                                   const void* v_cache, int cache_dtype, const int64_t k_strides[4],
-                                   const int64_t v_strides[4], const float* k_scale, const float* v_scale,
-                                   const int64_t k_scale_strides[3], const int64_t v_scale_strides[3],
-                                   const int32_t* block_tables, const int64_t bt_strides[2],
-                                   const int32_t* context_lens, const int32_t* cu_seqlens_q, void* out,
-                                   const int64_t out_strides[3], int batch, int total_q, int num_heads,
-                                   int num_kv_heads, int head_dim, int page_size, int num_blocks, int width,
-                                   float scale, int32_t* status, void* stream_ptr) {
+extern "C" int64_t prism_paged_prefill_workspace_bytes(int batch, int total_q, int num_heads, int num_kv_heads,
+                                                       int page_size, int width) {
+  using namespace prism;
+  if (batch <= 0 || total_q <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      num_heads / num_kv_heads > kPfMaxWaves || page_size <= 0 || width < 0)
+    return 0;
+  const int64_t capacity = static_cast<int64_t>(width) * page_size;
+  return split_workspace(split_count(total_q, batch, num_heads, num_kv_heads, capacity), total_q, num_heads);
+}
+
+extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,
+                                      const void* v_cache, int cache_dtype, const int64_t k_strides[4],
+                                      const int64_t v_strides[4], const float* k_scale, const float* v_scale,
+                                      const int64_t k_scale_strides[3], const int64_t v_scale_strides[3],
+                                      const int32_t* block_tables, const int64_t bt_strides[2],
+                                      const int32_t* context_lens, const int32_t* cu_seqlens_q, void* out,
+                                      const int64_t out_strides[3], int batch, int total_q, int num_heads,
+                                      int num_kv_heads, int head_dim, int page_size, int num_blocks, int width,
+                                      float scale, int32_t* status, void* workspace, int64_t workspace_bytes, void* stream_ptr){
   using namespace prism;
   clear_error();
   if (batch < 0 || total_q < 0 || num_heads <= 0 || num_kv_heads <= 0 || page_size <= 0 || num_blocks < 0 ||
@@ -709,8 +852,31 @@ extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_s
   a.width = width;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.status = status;
+  a.out_vec = aligned(out, 8) && out_strides[0] % 4 == 0 && out_strides[1] % 4 == 0;
+  a.total_q = total_q;
+  a.splits = split_count(total_q, batch, num_heads, num_kv_heads, static_cast<int64_t>(width) * page_size);
+  // without scratch for the partials the keys are not split
+  if (a.splits > 1 &&
+      (workspace == nullptr || !aligned(workspace, 16) || workspace_bytes < split_workspace(a.splits, total_q, num_heads)))
+    a.splits = 1;
+  a.part = static_cast<float*>(workspace);
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   const bool scaled = k_scale != nullptr;
-  if (q_dtype == PRISM_DTYPE_F16) return dispatch_tile<PRISM_DTYPE_F16>(a, scaled, total_q, stream);
-  return dispatch_tile<PRISM_DTYPE_BF16>(a, scaled, total_q, stream);
+  if (q_dtype == PRISM_DTYPE_F16) return dispatch_groups<PRISM_DTYPE_F16>(a, scaled, stream);
+  return dispatch_groups<PRISM_DTYPE_BF16>(a, scaled, stream);
+}
+
+extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,
+                                   const void* v_cache, int cache_dtype, const int64_t k_strides[4],
+                                   const int64_t v_strides[4], const float* k_scale, const float* v_scale,
+                                   const int64_t k_scale_strides[3], const int64_t v_scale_strides[3],
+                                   const int32_t* block_tables, const int64_t bt_strides[2],
+                                   const int32_t* context_lens, const int32_t* cu_seqlens_q, void* out,
+                                   const int64_t out_strides[3], int batch, int total_q, int num_heads,
+                                   int num_kv_heads, int head_dim, int page_size, int num_blocks, int width,
+                                   float scale, int32_t* status, void* stream_ptr) {
+  return prism_paged_prefill_ws(q, q_dtype, q_strides, k_cache, v_cache, cache_dtype, k_strides, v_strides, k_scale,
+                                v_scale, k_scale_strides, v_scale_strides, block_tables, bt_strides, context_lens,
+                                cu_seqlens_q, out, out_strides, batch, total_q, num_heads, num_kv_heads, head_dim,
+                                page_size, num_blocks, width, scale, status, nullptr, 0, stream_ptr);
 }

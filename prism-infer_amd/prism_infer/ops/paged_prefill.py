@@ -153,9 +153,13 @@ def _launch_paged_prefill(q, k_cache, v_cache, context, *, num_heads, num_kv_hea
         q = q.contiguous()
     out = torch.empty(q.shape, dtype=q.dtype, device=device)
     status = torch.full((1,), _STATUS_OK, dtype=torch.int32, device=device)
+    # scratch for split keys (static shapes only; 0 bytes where blocks are not split)
+    ws_bytes = lib.prism_paged_prefill_workspace_bytes(batch, q.shape[0], num_heads, num_kv_heads, k_cache.shape[1],
+                                                       block_tables.shape[1])
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes > 0 else None
     zero3 = _native.int64s(0, 0, 0)
     with torch.cuda.device(device):
-        rc = lib.prism_paged_prefill(
+        rc = lib.prism_paged_prefill_ws(
             q.data_ptr(), _native.dtype_code(q.dtype), _native.strides(q),
             k_cache.data_ptr(), v_cache.data_ptr(), _native.dtype_code(k_cache.dtype),
             _native.strides(k_cache), _native.strides(v_cache),
@@ -166,7 +170,8 @@ def _launch_paged_prefill(q, k_cache, v_cache, context, *, num_heads, num_kv_hea
             context_lens.data_ptr(), cu_seqlens_q.data_ptr(),
             out.data_ptr(), _native.strides(out),
             batch, q.shape[0], num_heads, num_kv_heads, q.shape[2], k_cache.shape[1], k_cache.shape[0],
-            block_tables.shape[1], float(scale), status.data_ptr(), _native.stream_handle(device),
+            block_tables.shape[1], float(scale), status.data_ptr(),
+            workspace.data_ptr() if workspace is not None else None, ws_bytes, _native.stream_handle(device),
         )
     _native.check(rc, "paged_prefill_attention")
     return out, status, (context_lens, cu_seqlens_q, block_tables), batch
