@@ -12,8 +12,8 @@
 // one sequence; a wave owns 32 of the tokens and one of the G query heads of
 // the kv head, so each K/V tile is read once into LDS for all of them (4 waves:
 // 32 tokens for G = 4, 64 and 128 for G = 2 and 1; 8 waves for G = 8).  Tiles of 64 keys
-// are double buffered through LDS: the next tile's loads are in flight while
-// the current one is computed.  Per tile a wave computes S^T = K Q^T with
+// go through four LDS stages: two tiles' loads are in flight beside the tile
+// whose scores and the one whose softmax are computed.  Per tile a wave computes S^T = K Q^T with
 // 32x32 MFMAs (bf16 queries: the fp8 MFMA 32x32x64 on the K bytes as they
 // are, the query split into two fp8 terms that hold it exactly, products
 // exact in fp32; f16 queries: v_mfma_f32_32x32x16_f16 on K converted to f16,
@@ -57,9 +57,11 @@ constexpr int kPfD = 128;                    // head dim
 constexpr int kPfCols = 32;                  // query tokens per wave: the columns of a 32x32 MFMA
 constexpr int kPfKT = 64;                    // keys per tile
 constexpr int kPfMaxWaves = 8;               // GQA group size limit
-constexpr float kPfRescaleThreshold = 8.0f;  // log2 units
+constexpr float kPfSumLimit = 256.0f;        // largest sum of a lane's 32 weights that keeps the running max
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
 
 struct PrefillArgs {
   const void* q;
@@ -106,26 +108,37 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
   return reinterpret_cast<const uint8_t*>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// A uniform value in an SGPR.  Integer divisions come out of the VALU, and what
+// depends on them (the tile loop's counters, addresses and branches) would
+// stay there.
+__device__ __forceinline__ int uniform_int(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 __device__ __forceinline__ void flag_sequence(const PrefillArgs& a, int seq) {
   atomicMin(a.status, seq);
 }
 
-// Inclusive wave scan of v (64 lanes).
-__device__ __forceinline__ int wave_scan(int v) {
-  const int lane = __lane_id();
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int u = __shfl_up(v, off);
-    if (lane >= off) v += u;
-  }
-  return v;
+// Inclusive wave scan with f over lanes of non-negative values (0 is f's
+// neutral element): row shifts, then the row ends broadcast onwards.
+template <typename F>
+__device__ __forceinline__ int wave_scan(int v, F f) {
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false));  // row_shr:1
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false));  // row_shr:2
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false));  // row_shr:4
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false));  // row_shr:8
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
+  return f(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
 }
+
+struct AddInt {
+  __device__ int operator()(int x, int y) const { return x + y; }
+};
+struct MaxInt {
+  __device__ int operator()(int x, int y) const { return max(x, y); }
+};
 
 template <typename F>
 __device__ __forceinline__ int wave_reduce(int v, F f) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) v = f(v, __shfl_xor(v, off));
-  return __builtin_amdgcn_readfirstlane(v);
+  return __builtin_amdgcn_readlane(wave_scan(v, f), 63);
 }
 
 // Query blocks of sequence i (0 for a sequence with invalid lengths, which
@@ -156,18 +169,18 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
   if (a.batch <= 64) {  // one lane per sequence, loaded once
     int l0 = 0;
     const int n = lane < a.batch ? seq_blocks<QT>(a, lane, flag, l0) : 0;
-    int lo = 0, hi = wave_reduce(n == 0 ? 0 : l0 + n, [](int x, int y) { return max(x, y); });
-    if (rank >= wave_reduce(n, [](int x, int y) { return x + y; })) return false;
+    int lo = 0, hi = wave_reduce(n == 0 ? 0 : l0 + n, MaxInt());
+    if (rank >= wave_reduce(n, AddInt())) return false;
     auto above = [&](int u) { return min(max(l0 + n - 1 - max(u, l0 - 1), 0), n); };
     // smallest u in [0, hi] with at most `rank` blocks above level u
     while (lo < hi) {
       const int mid = (lo + hi) / 2;
-      if (wave_reduce(above(mid), [](int x, int y) { return x + y; }) <= rank) hi = mid;
+      if (wave_reduce(above(mid), AddInt()) <= rank) hi = mid;
       else lo = mid + 1;
     }
     const int at = (n > 0 && lo >= l0 && lo < l0 + n) ? 1 : 0;
-    const int first = wave_reduce(above(lo), [](int x, int y) { return x + y; });
-    const int incl = wave_scan(at) + first;
+    const int first = wave_reduce(above(lo), AddInt());
+    const int incl = wave_scan(at, AddInt()) + first;
     const uint64_t hit = __builtin_amdgcn_ballot_w64(at && incl == rank + 1);
     const int l = __builtin_ctzll(hit);
     seq = __builtin_amdgcn_readfirstlane(l);
@@ -179,7 +192,7 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
   for (int base = 0; base < a.batch; base += 64) {
     const int i = base + lane;
     const int n = i < a.batch ? seq_blocks<QT>(a, i, flag, l0) : 0;
-    total += __shfl(wave_scan(n), 63);
+    total += wave_reduce(n, AddInt());
   }
   const int target = total - 1 - rank;
   if (target < 0) return false;
@@ -187,7 +200,7 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
   for (int base = 0; base < a.batch; base += 64) {
     const int i = base + lane;
     const int n = i < a.batch ? seq_blocks<QT>(a, i, false, l0) : 0;
-    const int incl = wave_scan(n) + before;
+    const int incl = wave_scan(n, AddInt()) + before;
     const uint64_t hit = __builtin_amdgcn_ballot_w64(i < a.batch && target < incl && target >= incl - n);
     if (hit != 0) {
       const int l = __builtin_ctzll(hit);
@@ -202,8 +215,7 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
 
 // Query operand (B of S^T = K Q^T).  Lane (g, c), g = lane / 32, holds query
 // column c's dims 64 kh + 32 g .. + 31 for the two halves kh, the same dims as
-// the K bytes it meets (row c of the block, LDS chunks 4 kh + 2 g and + 1);
-// `mul` turns the column's scores into log2 units.
+// the K bytes it meets (row c of the block, LDS chunks 4 kh + 2 g and + 1).
 //
 // bf16 queries: the fp8 MFMA (32x32x64) on the K bytes as they are.  The
 // column is scaled by 2^e so that its largest |q| lies in [128, 256) and
@@ -212,37 +224,31 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
 // (M - 16 H) * 2^k with |M - 16 H| <= 8: at most 4 significant bits, held
 // exactly by lo whenever 2^k is on E4M3FN's grid (elements of 2^-2 and up,
 // 2^-10 of the column's largest), and within 2^-10 below (2^-18 of the
-// largest), as a third term would be.  The score is (K . (hi + lo)) * 2^-e;
-// 2^-e joins the softmax scale in `mul`.
+// largest), as a third term would be.  The MFMA's block scale of the operand
+// takes 2^e back out, so that the scores of every column are in one unit and
+// what turns them into log2 units (softmax scale and key scale) depends on
+// the key alone.
 //
 // f16 queries (11 bits, which two terms do not hold): K converted to f16
 // (exact) and v_mfma_f32_32x32x16_f16.
 template <int QDT>
 struct PfQOperand {
   i32x8 t[2][2];  // [lo, hi][half]
-  float mul;      // scale_log2 * 2^-e of this lane's column
+  int scale;      // 2^-e as the MFMA's E8M0 block scale, in every byte
 };
 
 template <>
 struct PfQOperand<PRISM_DTYPE_F16> {
   f16x8 op[2][4];
-  float mul;  // scale_log2
 };
 
 template <int QDT>
-__device__ __forceinline__ void pf_load_q(const uint16_t* src, bool valid, float scale_log2, PfQOperand<QDT>& q) {
-  u32x4 w[2][4];
-#pragma unroll
-  for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc)
-      w[kh][cc] = valid ? *reinterpret_cast<const u32x4*>(src + 64 * kh + 8 * cc) : u32x4{0u, 0u, 0u, 0u};
+__device__ __forceinline__ void pf_make_q(const u32x4 (&w)[2][4], PfQOperand<QDT>& q) {
   if constexpr (QDT == PRISM_DTYPE_F16) {
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
       for (int cc = 0; cc < 4; ++cc) q.op[kh][cc] = __builtin_bit_cast(f16x8, w[kh][cc]);
-    q.mul = scale_log2;
   } else {
     float mx = 0.f;
 #pragma unroll
@@ -254,10 +260,10 @@ __device__ __forceinline__ void pf_load_q(const uint16_t* src, bool valid, float
           mx = fmaxf(mx, fmaxf(fabsf(bf16_bits_to_f32(w[kh][cc][e] & 0xFFFFu)), fabsf(bf16_bits_to_f32(w[kh][cc][e] >> 16))));
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
     mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    // ilogb(mx) = frexp exponent - 1; clamped so that 2^-e stays a normal
-    // fp32 number (columns of zeros, or of non-finite values, keep e = 0)
+    // ilogb(mx) = frexp exponent - 1; clamped to E8M0's range (columns of
+    // zeros, or of non-finite values, keep e = 0)
     const int e = (mx > 0.f && mx <= 3.0e38f) ? min(max(8 - __builtin_amdgcn_frexp_expf(mx), -120), 120) : 0;
-    q.mul = ldexpf(scale_log2, -e);
+    q.scale = (127 - e) * 0x01010101;
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
@@ -271,13 +277,6 @@ __device__ __forceinline__ void pf_load_q(const uint16_t* src, bool valid, float
         q.t[0][kh][d] = static_cast<int>(parts[1]);
       }
   }
-}
-
-// Eight transposed reads of a 32-key half tile: ad[n] are the addresses of
-// dim tile n for the first 16 keys, 16 rows further for the next; one wait.
-template <int OFF>
-__device__ __forceinline__ void pf_read_v(const uint32_t (&ad)[4], uint64_t (&v0)[4], uint64_t (&v1)[4]) {
-  lds_read_tr8_x8<OFF, OFF + 16 * kPfD>(ad, v0, v1);
 }
 
 // Two waves per SIMD: at most 256 VGPRs + AGPRs per lane.
@@ -294,16 +293,16 @@ paged_prefill_kernel(const PrefillArgs a) {
   constexpr int kRow = kPfD;                   // one key's payload row in LDS (bytes)
   constexpr int kPayload = kPfKT * kRow;       // K or V payload of a tile
   constexpr int kStage = 2 * kPayload + 2 * kPfKT * 4;
-  __shared__ __attribute__((aligned(256))) uint8_t stages[2 * kStage];
+  __shared__ __attribute__((aligned(256))) uint8_t stages[4 * kStage];
 
   // workgroup -> (block rank, split, kv head): heads fastest, so that the
   // long blocks of all heads start first and, with 8 kv heads, each XCD reads
   // one head's K/V
   const int kv_heads = a.num_heads / G;
   const int per_block = kv_heads * a.splits;
-  const int rank = static_cast<int>(blockIdx.x) / per_block;
+  const int rank = uniform_int(static_cast<int>(blockIdx.x) / per_block);
   const int rest = static_cast<int>(blockIdx.x) - rank * per_block;
-  const int split = rest / kv_heads;
+  const int split = uniform_int(rest / kv_heads);
   const int h = rest - split * kv_heads;
   int seq, qblock;
   if (!locate<QT>(a, rank, blockIdx.x == 0 && threadIdx.x < 64, seq, qblock)) return;
@@ -325,15 +324,22 @@ paged_prefill_kernel(const PrefillArgs a) {
   const int qlast = qpos0 + (qb0 < qlen ? kPfCols : 0) - 1;  // no key past it is visible to the wave
   const int all_tiles = (kend + kPfKT - 1) / kPfKT;
   // this workgroup's tiles
-  const int t0 = static_cast<int>(static_cast<int64_t>(all_tiles) * split / a.splits);
-  const int t1 = static_cast<int>(static_cast<int64_t>(all_tiles) * (split + 1) / a.splits);
+  const int t0 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * split / a.splits));
+  const int t1 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * (split + 1) / a.splits));
   const int32_t* bt_row = a.bt + static_cast<int64_t>(seq) * a.bt_sb;
 
-  PfQOperand<QDT> qop;
+  // the query's loads, then the first tiles', then the query's conversion
   const bool colv = qb0 + c < qlen;
-  pf_load_q<QDT>(static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(qs + (colv ? qb0 + c : 0)) * a.q_st +
-                     static_cast<int64_t>(qhead) * a.q_sh + 32 * g,
-                 colv, a.scale_log2, qop);
+  u32x4 qraw[2][4];
+  {
+    const uint16_t* src = static_cast<const uint16_t*>(a.q) + static_cast<int64_t>(qs + (colv ? qb0 + c : 0)) * a.q_st +
+                          static_cast<int64_t>(qhead) * a.q_sh + 32 * g;
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc)
+        qraw[kh][cc] = colv ? *reinterpret_cast<const u32x4*>(src + 64 * kh + 8 * cc) : u32x4{0u, 0u, 0u, 0u};
+  }
 
   // ---- tile loads, straight into LDS (load-to-LDS, 16 B per lane): K rows,
   // V rows, K scales, V scales.  A wave's load covers 8 rows: LDS chunk x of
@@ -347,15 +353,22 @@ paged_prefill_kernel(const PrefillArgs a) {
   // of loads)
   // (the 8-row groups of a wave have the parity of the wave: NW is even)
   uint32_t k_off, v_off;
+  const int k_sp = static_cast<int>(a.k_sp), v_sp = static_cast<int>(a.v_sp);
   {
-    const int r = lane / 8;
-    const int part = (lane % 8) ^ pf_swz(8 * (wave & 1) + r);
-    k_off = static_cast<uint32_t>(r * static_cast<int>(a.k_sp) + part * 16);
-    v_off = static_cast<uint32_t>(r * static_cast<int>(a.v_sp) + part * 16);
+    const int r = 8 * wave + lane / 8;
+    const int part = (lane % 8) ^ pf_swz(r);
+    k_off = static_cast<uint32_t>(r * k_sp + part * 16);
+    v_off = static_cast<uint32_t>(r * v_sp + part * 16);
   }
+  const uint8_t* k_head = a.k + h * a.k_sh;
+  const uint8_t* v_head = a.v + h * a.v_sh;
+  // waves 0 and 1 load the tile's K and V scales
+  const float* s_head = wave ? a.vs + h * a.vs_sh : a.ks + h * a.ks_sh;
+  const int64_t s_sn = wave ? a.vs_sn : a.ks_sn;
+  const int s_sp = static_cast<int>(wave ? a.vs_sp : a.ks_sp);
   // Block ids: 64 consecutive entries of the table row in one register,
   // renewed every 64 pages; (pg, row) walk the pages without divisions.
-  int pg = t0 * kPfKT / a.page;
+  int pg = uniform_int(t0 * kPfKT / a.page);
   int row = t0 * kPfKT - pg * a.page;
   int ids_base = pg;
   auto load_ids = [&](int base) { return bt_row[static_cast<int64_t>(min(base + lane, a.width - 1)) * a.bt_sn]; };
@@ -371,6 +384,8 @@ paged_prefill_kernel(const PrefillArgs a) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  : : "v"(off), "s"(uniform_ptr(base)), "s"(lds) : "memory", "m0");
   };
+  // Starts tile t's loads into stage st; returns whether all of a full tile's
+  // loads were issued.
   auto issue_tile = [&](int t, uint8_t* st) -> bool {
     constexpr int kGroups = WHOLE ? 1 : kPfKT / 16;  // table lookups per tile
     constexpr int kGroupRows = kPfKT / kGroups;
@@ -394,52 +409,54 @@ paged_prefill_kernel(const PrefillArgs a) {
       if (tid == 0) flag_sequence(a, seq);
       return false;
     }
-    const uint32_t st_lds = lds_addr(st);
+    const uint32_t st_lds = lds_addr(st) + static_cast<uint32_t>(wave) * 8 * kRow;
     constexpr int kLoads = 2 * kPfKT / 8 / NW;  // 8-row loads per wave, the first half of them K
 #pragma unroll
     for (int l = 0; l < kLoads; ++l) {
       const bool isv = l >= kLoads / 2;
-      const int tr = ((isv ? l - kLoads / 2 : l) * NW + wave) * 8;  // first row in the tile
-      const int x = WHOLE ? 0 : tr / 16;
+      const int tr = (isv ? l - kLoads / 2 : l) * NW * 8;  // the waves' first row in the tile
       int b = blk[0], pr = row0[0] + tr;
       if constexpr (!WHOLE) {
+        const int x = (tr + wave * 8) / 16;
 #pragma unroll
         for (int y = 1; y < kGroups; ++y)
           if (x == y) b = blk[y], pr = row0[y] + tr - 16 * y;
         if (b < 0) continue;
       }
-      const uint8_t* base = isv ? a.v + b * a.v_sn + static_cast<int64_t>(pr) * a.v_sp + h * a.v_sh
-                                : a.k + b * a.k_sn + static_cast<int64_t>(pr) * a.k_sp + h * a.k_sh;
+      const uint8_t* base = isv ? v_head + b * a.v_sn + pr * v_sp : k_head + b * a.k_sn + pr * k_sp;
       load_chunks(base, isv ? v_off : k_off,
                   __builtin_amdgcn_readfirstlane(st_lds + (isv ? kPayload : 0) + static_cast<uint32_t>(tr) * kRow));
     }
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-      if (which != wave) continue;
-      const uint32_t lds = __builtin_amdgcn_readfirstlane(st_lds + 2 * kPayload + static_cast<uint32_t>(which) * kPfKT * 4);
+    if (wave < 2) {
       if constexpr (SCALED) {
-        const float* s = which ? a.vs : a.ks;
-        const int64_t sn = which ? a.vs_sn : a.ks_sn, sp = which ? a.vs_sp : a.ks_sp, sh = which ? a.vs_sh : a.ks_sh;
-        if constexpr (WHOLE) {
-          const uint8_t* base = uniform_ptr(reinterpret_cast<const uint8_t*>(s + blk[0] * sn + row0[0] * sp + h * sh));
-          const uint32_t off = static_cast<uint32_t>(lane * static_cast<int>(sp) * 4);
-          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds)
-                       : "memory", "m0");
-        } else {
-          int b = blk[0], pr = row0[0];
+        int b = blk[0], pr = row0[0];
+        if constexpr (!WHOLE) {
 #pragma unroll
           for (int y = 1; y < kGroups; ++y)
-            if (lane / 16 == y) b = blk[y], pr = row0[y];
-          const float* src = s + b * sn + static_cast<int64_t>(pr + lane % 16) * sp + h * sh;
-          if (b >= 0)
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds)
-                         : "memory", "m0");
+            if (lane / 16 == y) b = blk[y], pr = row0[y] - 16 * y;
         }
+        const float* src = s_head + b * s_sn + pr * s_sp + lane * s_sp;
+        const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_addr(st) + 2 * kPayload + wave * kPfKT * 4);
+        if (WHOLE || b >= 0)
+          asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds)
+                       : "memory", "m0");
       } else {
-        reinterpret_cast<float*>(st + 2 * kPayload)[which * kPfKT + lane] = 1.f;
+        reinterpret_cast<float*>(st + 2 * kPayload)[wave * kPfKT + lane] = 1.f;
       }
     }
-    return true;
+    return WHOLE || (t + 1) * kPfKT <= kend;
+  };
+  // A tile's K scales are multiplied by the softmax scale in log2 units, in
+  // place, while the tile before it is computed: a score times its entry is
+  // the exponent.
+  auto scale_slot = [&](uint32_t st) { return reinterpret_cast<float*>(stages + st + 2 * kPayload) + lane; };
+  // Waits for this wave's loads but those of the last tile issued (`full`: it
+  // issued all of them; else for all).
+  auto wait_tiles = [&](bool full) {
+    constexpr int kLoads = 2 * kPfKT / 8 / NW;
+    if (!full) __builtin_amdgcn_s_waitcnt(0xF70);                              // vmcnt(0)
+    else if (SCALED && wave < 2) __builtin_amdgcn_s_waitcnt(0xF70 | (kLoads + 1));
+    else __builtin_amdgcn_s_waitcnt(0xF70 | kLoads);
   };
 
   floatx16 acc[4];  // O^T: dims 32 n + 8 (r / 4) + 4 g + r % 4 of query column c
@@ -449,169 +466,224 @@ paged_prefill_kernel(const PrefillArgs a) {
     for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
 
-  // per-lane LDS offsets inside a stage, for keys 0..31 (32 rows further for the rest)
-  uint32_t k_rd[4];
-#pragma unroll
-  for (int x = 0; x < 4; ++x) k_rd[x] = c * kRow + (((4 * (x / 2) + 2 * g + x % 2) ^ pf_swz(c)) << 4);
-  uint32_t v_rd[4];
+  // per-lane LDS offsets inside a stage, for keys 0..31 (32 rows further for
+  // the rest); the lane's other chunks differ by an exclusive or
+  const uint32_t k_rd = c * kRow + (((2 * g) ^ pf_swz(c)) << 4);
+  uint32_t v_rd;
   {
     const int r = (lane % 16) >> 1;
     const int t = 8 * (r >> 2) + 4 * g + (r & 3);  // key of the 16-key group
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      v_rd[n] = kPayload + t * kRow + (((2 * n + (lane / 16) % 2) ^ pf_swz(t)) << 4) + (lane & 1) * 8;
+    v_rd = kPayload + t * kRow + ((((lane / 16) % 2) ^ pf_swz(t)) << 4) + (lane & 1) * 8;
   }
   const uint32_t stage_base = lds_addr(stages);
 
-  bool cur_ok = t0 < t1 ? issue_tile(t0, stages) : false;
-  __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
+  // A tile that could not be loaded (invalid block id) leaves its stage as it
+  // was: the sequence is flagged and its rows are unspecified.
+  uint32_t cur = 0, nxt = kStage, ahead = 2 * kStage, ld = 3 * kStage;  // stages of tiles t .. t + 3
+  if (t0 < t1) issue_tile(t0, stages);
+  if (t0 + 1 < t1) issue_tile(t0 + 1, stages + nxt);
+  const bool full2 = t0 + 2 < t1 && issue_tile(t0 + 2, stages + ahead);
+  PfQOperand<QDT> qop;
+  pf_make_q<QDT>(qraw, qop);
+  wait_tiles(full2);
+  if (wave == 0) *scale_slot(cur) *= a.scale_log2;
   __syncthreads();
-  for (int t = t0; t < t1; ++t) {
-    const uint32_t soff = static_cast<uint32_t>((t - t0) & 1) * kStage;
-    // the next tile streams into the other stage, last read by tile t - 1,
-    // which every wave finished before the barrier that ended that iteration
-    const bool next_ok = t + 1 < t1 ? issue_tile(t + 1, stages + (kStage - soff)) : true;
-    const uint8_t* st = stages + soff;
+  // S^T = K Q^T of the tile at byte `st` of the LDS, in two chains of 32 keys
+  // (b), each of four steps: the K bytes are the fp8 MFMA's A operand as they
+  // are, smaller query term first; f16 queries take two 16-dim MFMAs a step.
+  auto read_k = [&](uint32_t st, int b, u32x4 (&kw)[4]) {
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+      kw[x] = *reinterpret_cast<const u32x4*>(stages + b * 32 * kRow + ((st + k_rd) ^ ((x % 2) << 4) ^ ((x / 2) << 6)));
+  };
+  auto qk_step = [&](int step, const u32x4 (&kw)[4], floatx16& sc) {
+    if (step == 0)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+    if constexpr (QDT == PRISM_DTYPE_F16) {
+      const u32x4& w = kw[step];
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fp8x8_to_f16x8(w[2 * y], w[2 * y + 1]),
+                                                    qop.op[step / 2][2 * (step % 2) + y], sc, 0, 0, 0);
+    } else {
+      const int kh = step % 2;
+      i32x8 ka;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) ka[x] = static_cast<int>(kw[2 * kh + x / 4][x % 4]);
+      sc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ka, qop.t[step / 2][kh], sc, 0, 0, 0, 0x7F7F7F7F, 0, qop.scale);
+    }
+  };
+
+  bool first = true;  // no tile's scores seen yet
+  floatx16 sa[2], sb[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    u32x4 kw[4];
+    read_k(cur, b, kw);
+#pragma unroll
+    for (int step = 0; step < 4; ++step) qk_step(step, kw, sa[b]);
+  }
+
+  // One tile: the scores of the next one (MFMAs) are computed beside this
+  // one's softmax (VALU).
+  auto tile = [&](int t, floatx16 (&sc)[2], floatx16 (&sn)[2]) {
+    // tile t + 3 streams into the stage last read by tile t - 1, which every
+    // wave finished before the barrier that ended that iteration
+    const bool full = t + 3 < t1 && issue_tile(t + 3, stages + ld);
+    if (wave == 0 && t + 1 < t1) *scale_slot(nxt) *= a.scale_log2;
+    const uint8_t* st = stages + cur;
     const int key0 = t * kPfKT;
-    if (cur_ok && key0 <= qlast) {
+    if (key0 <= qlast) {
       const float* scl = reinterpret_cast<const float*>(st + 2 * kPayload) + 4 * g;
-      // S^T = K Q^T, two chains of 32 keys; the second is skipped above the
-      // diagonal (uniform branch)
       const bool both = key0 + 32 <= qlast;
-      floatx16 sc[2];
+      // V^T operands of 32 keys: v[m][n] for 16-key group m and dim tile n
+      auto read_v = [&](int b, u32x2 (&v)[2][4]) {
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
+        for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[b][r] = 0.f;
-        u32x4 kw[4];
+          for (int n = 0; n < 4; ++n)
+            v[m][n] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                reinterpret_cast<lds_i32x2*>(stage_base + ((cur + v_rd) ^ (n << 5)) + (32 * b + 16 * m) * kRow)));
+      };
+      // Online softmax -> P (B of O^T += V^T P^T: the k-slots 8 g + 0..3 of
+      // 16-key group m are keys 16 m + 4 g + 0..3, and 8 g + 4..7 the keys 8
+      // further, the order the score rows come out in: row r of chain b is key
+      // key0 + 32 b + 8 (r / 4) + 4 g + r % 4).
+      //
+      // P is first formed against the running max as it stands; the sum, which
+      // is needed anyway, tells whether that was low enough (every p is at
+      // most the lane's sum).  Only where it was not, on the first tile and on
+      // tiles with masked keys, are the scores' maxima taken and the
+      // accumulators rescaled.
+      bf16x8 pa[2][2];
+      float ps;
+      const bool masked = key0 + kPfKT - 1 > qpos0;  // (uniform) the diagonal or the block's end is in the tile
+      //
+      // An MFMA issues once the one before it is through, and holds its wave
+      // until then.  So the eight of the next tile's scores are spread over
+      // the softmax by hand: each slice is one of them (past the last tile on
+      // stale bytes, for nothing), four scores' worth of softmax, and the LDS
+      // reads of the slices after it.
+      u32x4 kw[2][4];
+      u32x2 vt[2][2][4];
+      floatx4 ksv[2], vsv[2];
+      read_k(nxt, 0, kw[0]);
+      ksv[0] = *reinterpret_cast<const floatx4*>(scl);
+      vsv[0] = *reinterpret_cast<const floatx4*>(scl + kPfKT);
+      ps = 0.f;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int x = 0; x < 4; ++x) kw[x] = *reinterpret_cast<const u32x4*>(st + b * 32 * kRow + k_rd[x]);
-        if constexpr (QDT == PRISM_DTYPE_F16) {
-#pragma unroll
-          for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-            for (int cc = 0; cc < 4; ++cc) {
-              const u32x4& w = kw[2 * kh + cc / 2];
-              sc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fp8x8_to_f16x8(w[2 * (cc % 2)], w[2 * (cc % 2) + 1]),
-                                                             qop.op[kh][cc], sc[b], 0, 0, 0);
-            }
-        } else {
-          // the K bytes are the fp8 MFMA's A operand as they are; smaller term first
-          i32x8 ka[2];
-#pragma unroll
-          for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-            for (int x = 0; x < 8; ++x) ka[kh][x] = static_cast<int>(kw[2 * kh + x / 4][x % 4]);
-#pragma unroll
-          for (int term = 0; term < 2; ++term)
-#pragma unroll
-            for (int kh = 0; kh < 2; ++kh)
-              sc[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ka[kh], qop.t[term][kh], sc[b], 0, 0, 0, 0, 0, 0);
+      for (int x = 0; x < 8; ++x) {
+        const int b = x / 4, i = x % 4;
+        qk_step(i, kw[b], sn[b]);
+        if (x < 7) {
+          ksv[(x + 1) % 2] = *reinterpret_cast<const floatx4*>(scl + 32 * ((x + 1) / 4) + 8 * ((x + 1) % 4));
+          vsv[(x + 1) % 2] = *reinterpret_cast<const floatx4*>(scl + kPfKT + 32 * ((x + 1) / 4) + 8 * ((x + 1) % 4));
         }
+        if (x == 2) read_k(nxt, 1, kw[1]);
+        if (x == 6) read_v(0, vt[0]);
+        float p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // v_exp_f32: arguments are at most 2^3 above the running max;
+          // results below 2^-126 (flushed to 0) weigh nothing next to it
+          p[j] = __builtin_amdgcn_exp2f(fmaf(sc[b][4 * i + j], ksv[x % 2][j], -m_run));
+          pa[b][i / 2][4 * (i % 2) + j] = static_cast<__bf16>(p[j] * vsv[x % 2][j]);
+        }
+        ps += (p[0] + p[1]) + (p[2] + p[3]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // score rows: key key0 + 32 b + 8 (r / 4) + 4 g + r % 4
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const floatx4 ksv = *reinterpret_cast<const floatx4*>(scl + 32 * b + 8 * i);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) sc[b][4 * i + j] *= ksv[j];  // score / softmax scale
-        }
-      // causal mask: key k is visible to column c iff it is at or before the
-      // query's position.  Tiles wholly below the diagonal need no mask
-      // (uniform branch); columns without a query hold q = 0 there, so their
-      // scores stay finite and their rows are never written.
-      const bool masked = key0 + kPfKT - 1 > qpos0;
-      if (masked) {
+      // (the pins keep the sums and the MFMAs in front of the branch)
+      asm volatile("" : "+v"(ps), "+v"(pa[0][0]), "+v"(pa[0][1]), "+v"(pa[1][0]), "+v"(pa[1][1])
+                   : "v"(sn[0]), "v"(sn[1]));
+      if (first || masked || __builtin_amdgcn_ballot_w64(ps > kPfSumLimit) != 0) {
+        first = false;
+        // causal mask: key k is visible to column c iff it is at or before the
+        // query's position; columns without a query see none, and their rows
+        // are never written.  Keys past the block's last may hold any bytes
+        // and scales (past the context, or not loaded).
         const int last = colv ? qpos0 + c - key0 - 4 * g : -1;  // last visible key, as a row offset
+        float tmax = -INFINITY;
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int r = 0; r < 16; ++r)
-            sc[b][r] = 32 * b + 8 * (r / 4) + r % 4 <= last ? sc[b][r] : -INFINITY;
-      }
-      float tmax = fmaxf(sc[0][0], sc[1][0]);
+          for (int i = 0; i < 4; ++i) {
+            const floatx4 ksv = *reinterpret_cast<const floatx4*>(scl + 32 * b + 8 * i);
 #pragma unroll
-      for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, fmaxf(sc[0][r], sc[1][r]));
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
-        tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * qop.mul;  // log2 units (mul is positive)
-      }
-      const bool raise = tmax > m_run + kPfRescaleThreshold;
-      if (__builtin_amdgcn_ballot_w64(raise) != 0) {
-        const float m_new = raise ? tmax : m_run;
-        const float alpha = raise ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+            for (int j = 0; j < 4; ++j) {
+              const float x = sc[b][4 * i + j] * ksv[j];
+              sc[b][4 * i + j] = 32 * b + 8 * i + j <= last ? x : -INFINITY;
+              tmax = fmaxf(tmax, sc[b][4 * i + j]);
+            }
+          }
+        {
+          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+          tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+        }
+        const float m_new = tmax > m_run ? tmax : m_run;
+        // (no key seen: keep the accumulators, all zero, from (-inf) - (-inf))
+        const float alpha = m_new > m_run ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
         m_run = m_new;
         l_run *= alpha;
 #pragma unroll
         for (int n = 0; n < 4; ++n)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[n][r] *= alpha;
+        const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+        ps = 0.f;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const floatx4 vsv = *reinterpret_cast<const floatx4*>(scl + kPfKT + 32 * b + 8 * i);
+            float p[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              p[j] = __builtin_amdgcn_exp2f(sc[b][4 * i + j] - m_use);  // 0 where masked
+              pa[b][i / 2][4 * (i % 2) + j] = static_cast<__bf16>(p[j] > 0.f ? p[j] * vsv[j] : 0.f);
+            }
+            ps += (p[0] + p[1]) + (p[2] + p[3]);
+          }
       }
-      const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
-      // per 32 keys: P (B of O^T += V^T P^T, k-slots 8 g + 0..3 of 16-key group
-      // m are keys 16 m + 4 g + 0..3 and 8 g + 4..7 the keys 8 further, the
-      // order the score rows come out in), then the products
+      l_run += ps;
+      // O^T += V^T P^T
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         if (b == 1 && !both) break;
-        uint64_t vt[2][4];
-        {
-          uint32_t ad[4];
-#pragma unroll
-          for (int n = 0; n < 4; ++n) ad[n] = stage_base + soff + v_rd[n];
-          if (b == 0) pf_read_v<0>(ad, vt[0], vt[1]);
-          else pf_read_v<32 * kRow>(ad, vt[0], vt[1]);
-        }
-        floatx4 vsv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vsv[i] = *reinterpret_cast<const floatx4*>(scl + kPfKT + 32 * b + 8 * i);
-        // keys past the block's last may hold any bytes and scales (past the
-        // context, or not loaded): zero them (only the block's last tile can
-        // hold such keys; uniform branch)
-        if (key0 + 32 * b + 32 > kend) {
+        if (b == 0 && both) read_v(1, vt[1]);
+        if (key0 + 32 * b + 32 > kend) {  // (uniform) 0 x a stray NaN would not be 0
           const int left = kend - key0 - 32 * b - 4 * g;
 #pragma unroll
-          for (int m = 0; m < 2; ++m) {
-            uint64_t keep = 0;
+          for (int m = 0; m < 2; ++m)
 #pragma unroll
-            for (int jj = 0; jj < 8; ++jj)
-              keep |= (16 * m + 8 * (jj / 4) + jj % 4 < left) ? (uint64_t{0xFF} << (8 * jj)) : 0u;
+            for (int half = 0; half < 2; ++half) {
+              uint32_t keep = 0;
 #pragma unroll
-            for (int n = 0; n < 4; ++n) vt[m][n] &= keep;
-          }
+              for (int jj = 0; jj < 4; ++jj) keep |= (16 * m + 8 * half + jj < left) ? (0xFFu << (8 * jj)) : 0u;
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) vsv[i][j] = 8 * i + j < left ? vsv[i][j] : 0.f;
+              for (int n = 0; n < 4; ++n) vt[b][m][n][half] &= keep;
+            }
         }
-        bf16x8 pa[2];
-        float ps = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float p[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            // v_exp_f32: arguments are at most 2^3 above the running max;
-            // results below 2^-126 (flushed to 0) weigh nothing next to it
-            p[j] = __builtin_amdgcn_exp2f(fmaf(sc[b][4 * i + j], qop.mul, -m_use));  // 0 where masked
-            pa[i / 2][4 * (i % 2) + j] = static_cast<__bf16>(p[j] * vsv[i][j]);
-          }
-          ps += (p[0] + p[1]) + (p[2] + p[3]);
-        }
-        l_run += ps;
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
           for (int n = 0; n < 4; ++n)
-            acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                fp8x8_to_bf16x8(static_cast<uint32_t>(vt[m][n]), static_cast<uint32_t>(vt[m][n] >> 32)), pa[m], acc[n], 0, 0, 0);
+            acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fp8x8_to_bf16x8(vt[b][m][n][0], vt[b][m][n][1]), pa[b][m], acc[n],
+                                                             0, 0, 0);
       }
     }
-    cur_ok = next_ok;
-    __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0): this wave's part of tile t + 1 has landed
+    wait_tiles(full);  // this wave's part of tile t + 2 has landed
     __syncthreads();
+    const uint32_t done = cur;
+    cur = nxt;
+    nxt = ahead;
+    ahead = ld;
+    ld = done;
+  };
+  for (int t = t0; t < t1; t += 2) {
+    tile(t, sa, sb);
+    if (t + 1 < t1) tile(t + 1, sb, sa);
   }
 
   // ---- epilogue
@@ -644,14 +716,25 @@ paged_prefill_kernel(const PrefillArgs a) {
         const float x = acc[n][4 * i + j] * inv;
         o[j] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(x) : f32_to_bf16_bits(x);
       }
-      uint16_t* d = dst + 32 * n + 8 * i;
-      if (a.out_vec) {
-        *reinterpret_cast<u32x2*>(d) = u32x2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d[j] = static_cast<uint16_t>(o[j]);
-      }
+      acc[n][4 * i] = __uint_as_float(o[0] | (o[1] << 16));
+      acc[n][4 * i + 1] = __uint_as_float(o[2] | (o[3] << 16));
     }
+  if (a.out_vec) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<u32x2*>(dst + 32 * n + 8 * i) =
+            u32x2{__float_as_uint(acc[n][4 * i]), __float_as_uint(acc[n][4 * i + 1])};
+    return;
+  }
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        dst[32 * n + 8 * i + j] = static_cast<uint16_t>(__float_as_uint(acc[n][4 * i + j / 2]) >> (16 * (j & 1)));
 }
 
 // Merges the splits' partials: one wave per (token, query head), two dims per
@@ -665,19 +748,20 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   const int lane = threadIdx.x % 64;
   const int tok = static_cast<int>(cell / a.num_heads);
   if (tok < a.cu_q[0] || tok >= a.cu_q[a.batch]) return;
+  // lane s holds split s's weight (at most 64 splits)
   const floatx2* ml = reinterpret_cast<const floatx2*>(a.part + a.splits * cells * kPfD) + cell;
+  const floatx2 mine = lane < a.splits ? ml[lane * cells] : floatx2{-INFINITY, 0.f};
+  float m = mine[1] > 0.f ? mine[0] : -INFINITY;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+  const float weight = mine[1] > 0.f ? __builtin_amdgcn_exp2f(mine[0] - m) : 0.f;
   const floatx2* row = reinterpret_cast<const floatx2*>(a.part) + cell * (kPfD / 2) + lane;
-  float m = -INFINITY;
-  for (int s = 0; s < a.splits; ++s) {
-    const floatx2 x = ml[s * cells];
-    if (x[1] > 0.f) m = fmaxf(m, x[0]);
-  }
   float l = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll 4
   for (int s = 0; s < a.splits; ++s) {
-    const floatx2 x = ml[s * cells];
+    const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s));
     const floatx2 v = row[s * cells * (kPfD / 2)];
-    const float w = x[1] > 0.f ? __builtin_amdgcn_exp2f(x[0] - m) : 0.f;
-    l = fmaf(w, x[1], l);
+    l = fmaf(w, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine[1]), s)), l);
     o0 = w > 0.f ? fmaf(w, v[0], o0) : o0;
     o1 = w > 0.f ? fmaf(w, v[1], o1) : o1;
   }
@@ -695,9 +779,10 @@ int64_t block_bound(int total_q, int batch, int groups) { return ceil_div(total_
 // Workgroups per (block, kv head).  The kernel fits eight waves on a CU; where the blocks give fewer than that, the keys are split so
 // that the launch fills the chip once, in parts of at least 4 tiles of the
 // longest context the tables can hold.
+// (a sequence's last block is partial, so it adds half a block on average.)
 int split_count(int total_q, int batch, int num_heads, int num_kv_heads, int64_t capacity) {
   const int groups = num_heads / num_kv_heads;
-  const int64_t wgs = block_bound(total_q, batch, groups) * num_kv_heads;
+  const int64_t wgs = (ceil_div(total_q, pf_qtile(groups)) + batch / 2) * num_kv_heads;
   const int64_t slots = static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(groups);
   const int64_t s = std::min(slots / wgs, capacity / (4 * kPfKT));
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(s, 64)));
