@@ -332,6 +332,14 @@ int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t q_strides[3
                            float scale, int32_t* status, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * Writes {status[0], cu_seqlens_q[0], cu_seqlens_q[batch]} to `out` (int32[3];
+ * device memory or pinned host memory), for a host that reads the outcome of
+ * prism_paged_prefill back with one wait for the stream and no copy.
+ */
+int prism_paged_prefill_report(const int32_t* status, const int32_t* cu_seqlens_q, int batch, int32_t* out,
+                               void* stream);
+
+/*
  * Test hook with no counterpart in the reference: converts n fp32 values to
  * E4M3FN bytes with the exact device routine the scaled store uses (native
  * gfx950 conversion plus the NaN rule), so the rounding can be checked

@@ -16,12 +16,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_ROOT = Path(__file__).resolve().parent
 REPO_ROOT = PKG_ROOT.parent
 CSRC = PKG_ROOT / "csrc"
+HOST_SRC = PKG_ROOT / "csrc_host" / "host_ops.cpp"
 INCLUDE = REPO_ROOT / "include"
 BUILD_DIR = PKG_ROOT / "_build"
 OUT_DIR = PKG_ROOT / "prism_infer" / "_native"
@@ -109,9 +111,29 @@ def build(verbose: bool = True, *, out_dir: Path = OUT_DIR, measure: bool = Fals
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, out)
+    _build_host_ops(out_dir, build_dir, torch_lib)
     if verbose:
         print(f"built {out}")
     return out
+
+
+def _build_host_ops(out_dir: Path, build_dir: Path, torch_lib: Path) -> None:
+    """The CPython extension beside the library (host code only, torch's C++ API)."""
+
+    torch_include = torch_lib.parent / "include"
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    tmp = build_dir / "_host_ops.so"
+    cmd = [
+        "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-I{torch_include}", f"-I{torch_include / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{rocm / 'include'}",
+        f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", str(HOST_SRC), "-o", str(tmp),
+        f"-L{out_dir}", f"-l:{LIB_NAME}", f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+        "-l:libamdhip64.so", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}",
+    ]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {HOST_SRC.name}:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, out_dir / "_host_ops.so")
 
 
 if __name__ == "__main__":

@@ -772,6 +772,16 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   dst[1] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o1 * inv) : f32_to_bf16_bits(o1 * inv);
 }
 
+// What a caller reads back: the status word and the packed rows' extent, in
+// (pinned) memory that the host sees once the stream is done.
+__global__ void paged_prefill_report_kernel(const int32_t* status, const int32_t* cu_q, int batch, int32_t* out) {
+  if (threadIdx.x == 0) {
+    out[0] = status[0];
+    out[1] = cu_q[0];
+    out[2] = cu_q[batch];
+  }
+}
+
 // Query blocks that the launch provides for: every sequence may end in a
 // partial block.
 int64_t block_bound(int total_q, int batch, int groups) { return ceil_div(total_q, pf_qtile(groups)) + batch; }
@@ -949,6 +959,19 @@ extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t 
   const bool scaled = k_scale != nullptr;
   if (q_dtype == PRISM_DTYPE_F16) return dispatch_groups<PRISM_DTYPE_F16>(a, scaled, stream);
   return dispatch_groups<PRISM_DTYPE_BF16>(a, scaled, stream);
+}
+
+extern "C" int prism_paged_prefill_report(const int32_t* status, const int32_t* cu_seqlens_q, int batch, int32_t* out,
+                                          void* stream_ptr) {
+  using namespace prism;
+  clear_error();
+  if (!status || !cu_seqlens_q || !out || batch < 0) {
+    set_error("prism_paged_prefill_report: invalid argument");
+    return PRISM_ERR_INVALID;
+  }
+  hipLaunchKernelGGL(paged_prefill_report_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream_ptr), status,
+                     cu_seqlens_q, batch, out);
+  return check_launch("paged_prefill_report_kernel launch");
 }
 
 extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,

@@ -9,6 +9,8 @@ against torch/lib/libamdhip64.so).  A missing or unloadable library raises
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from pathlib import Path
 
 import torch
@@ -81,6 +83,7 @@ SIGNATURES: dict[str, tuple] = {
         [_VP, _I, _I64P, _VP, _VP, _I, _I64P, _I64P, _VP, _VP, _I64P, _I64P, _VP, _I64P, _VP, _VP, _VP,
          _I64P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _VP, _VP, _I64, _VP],
     ),
+    "prism_paged_prefill_report": (_I, [_VP, _VP, _I, _VP, _VP]),
     "prism_debug_fp8_encode": (_I, [_VP, _VP, _I64, _VP]),
 }
 
@@ -123,6 +126,32 @@ def lib() -> ctypes.CDLL:
     return handle
 
 
+HOST_OPS_PATH = LIB_PATH.with_name("_host_ops.so")
+_HOST_OPS = None
+_HOST_OPS_TRIED = False
+
+
+def host_ops():
+    """The extension that checks and launches the per-layer ops in C++, or None where it is not built.
+
+    Each of its functions returns None for a call it does not take; the ops'
+    Python code then handles it.
+    """
+
+    global _HOST_OPS, _HOST_OPS_TRIED
+    if not _HOST_OPS_TRIED:
+        _HOST_OPS_TRIED = True
+        if HOST_OPS_PATH.exists() and available():
+            loader = importlib.machinery.ExtensionFileLoader("_host_ops", str(HOST_OPS_PATH))
+            try:
+                module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_ops", loader))
+                loader.exec_module(module)
+            except ImportError as exc:
+                raise RuntimeError(f"cannot load {HOST_OPS_PATH}: {exc}") from exc
+            _HOST_OPS = module
+    return _HOST_OPS
+
+
 _PRELOADED: set[int] = set()
 
 
@@ -144,6 +173,8 @@ def device_lib(device: torch.device | None = None) -> ctypes.CDLL:
     if status != 0:
         raise RuntimeError(f"prism_preload failed ({status}): {handle.prism_last_error().decode(errors='replace')}")
     _PRELOADED.add(index)
+    if host_ops() is not None:
+        _HOST_OPS.mark_ready(index)
     return handle
 
 
@@ -201,6 +232,7 @@ __all__ = [
     "check",
     "device_lib",
     "dtype_code",
+    "host_ops",
     "int64s",
     "is_built",
     "lib",

@@ -18,7 +18,7 @@ from __future__ import annotations
 
 import torch
 
-from prism_infer import _native
+from prism_infer import _native, observability
 from prism_infer.engine.kv_quantization import (
     FP8_E4M3FN_MAX,
     FP8_E4M3FN_MIN,
@@ -32,6 +32,7 @@ from prism_infer.observability import profile_region
 # purpose and its callers/tests import that name, so both are provided.
 HAS_HIP_KERNELS = _native.available()
 HAS_TRITON = HAS_HIP_KERNELS
+_HOST = _native.host_ops()
 
 KV_TOKEN_HEAD_TENSOR_RANK = 3
 SUPPORTED_KV_CACHE_RANKS = (3, 4)
@@ -209,6 +210,11 @@ def store_kvcache(
 ) -> None:
     """Write current K/V values into canonical paged KV-cache slots (in place)."""
 
+    # GPU calls that the native checks accept; the rest, and every call while a
+    # profiling provider is installed, goes on below
+    if _HOST is not None and observability._region_provider is None and _HOST.store(
+            key, value, k_cache, v_cache, slot_mapping, k_scale_cache, v_scale_cache):
+        return
     scaled = _validate_store_inputs(key, value, k_cache, v_cache, slot_mapping, k_scale_cache, v_scale_cache)
     tensors = (key, value, k_cache, v_cache, slot_mapping, k_scale_cache, v_scale_cache)
     if not any(t is not None and t.is_cuda for t in tensors):

@@ -29,6 +29,7 @@ from prism_infer import _native
 
 HAS_HIP_KERNELS = _native.available()
 HAS_TRITON = HAS_HIP_KERNELS  # the reference's "kernel available" flag name
+_HOST = _native.host_ops()
 
 QUERY_TENSOR_RANK = 3
 PAGED_KV_CACHE_RANK = 4
@@ -273,6 +274,13 @@ def paged_decode_attention(
 
     if max_context_len is None:
         max_context_len = _no_context_bound(context_lens)
+    # GPU calls that the native checks accept, once their stream has its
+    # workspace; the rest goes on below
+    if _HOST is not None:
+        out = _HOST.decode(q, k_cache, v_cache, block_tables, context_lens, scale, k_scale_cache, v_scale_cache,
+                           max_context_len, block_n, _WORKSPACES)
+        if out is not None:
+            return out
     scaled_kv = _validate_paged_decode_inputs(
         q, k_cache, v_cache, block_tables, context_lens, max_context_len,
         k_scale_cache=k_scale_cache, v_scale_cache=v_scale_cache, block_n=block_n,

@@ -32,15 +32,41 @@ queries; other cases raise ``RuntimeError`` (no CPU fallback).
 
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from prism_infer import _native
 
 HAS_HIP_KERNELS = _native.available()
+_HOST = _native.host_ops()
 
 MINIMUM_PAGED_CACHE_RANK = 3
 PREFILL_HEAD_DIM = 128
 _STATUS_OK = 2**31 - 1
+
+# Per thread and (device, stream): the status word, which holds _STATUS_OK
+# between calls, and the pinned words a call's outcome is read from.  A call
+# waits for its stream before it returns, so a thread's next call finds them
+# free; other threads have their own.
+_OUTCOME = threading.local()
+_MAX_OUTCOME_STREAMS = 16
+
+
+def _outcome_buffers() -> dict:
+    buffers = getattr(_OUTCOME, "buffers", None)
+    if buffers is None:
+        buffers = _OUTCOME.buffers = {}
+    return buffers
+
+
+def _add_outcome_buffers(buffers: dict, device: torch.device) -> None:
+    if len(buffers) >= _MAX_OUTCOME_STREAMS:
+        buffers.clear()
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    status = torch.full((1,), _STATUS_OK, dtype=torch.int32, device=device)
+    buffers[(index, torch.cuda.current_stream(device).cuda_stream)] = (
+        status, torch.empty(3, dtype=torch.int32, pin_memory=True))
 
 
 def _validate_caches(k_cache, v_cache, k_scale_cache, v_scale_cache) -> bool:
@@ -195,6 +221,20 @@ def paged_prefill_attention(
     ``cu_seqlens_q`` tensors (the reference's ``Context``).
     """
 
+    # GPU calls that the native checks accept, once their stream has its
+    # buffers; the rest goes on below
+    buffers = None
+    if _HOST is not None:
+        buffers = _outcome_buffers()
+        done = _HOST.prefill(q, k_cache, v_cache, context.block_tables, context.context_lens, context.cu_seqlens_q,
+                             num_heads, num_kv_heads, scale, k_scale_cache, v_scale_cache, buffers)
+        if done is not None:
+            out, first_bad, row0, row1 = done
+            if first_bad != _STATUS_OK:
+                buffers.clear()  # the status words are made anew
+                _raise_sequence_error(first_bad, context.cu_seqlens_q.cpu(), context.context_lens.cpu(),
+                                      context.block_tables.cpu(), k_cache.shape[0], k_cache.shape[1])
+            return out[row0:row1]
     out, status, (context_lens, cu_seqlens_q, block_tables), batch = _launch_paged_prefill(
         q, k_cache, v_cache, context, num_heads=num_heads, num_kv_heads=num_kv_heads, scale=scale,
         k_scale_cache=k_scale_cache, v_scale_cache=v_scale_cache)
@@ -207,6 +247,8 @@ def paged_prefill_attention(
     if first_bad != _STATUS_OK:
         _raise_sequence_error(first_bad, cu_seqlens_q.cpu(), context_lens.cpu(), block_tables.cpu(),
                               k_cache.shape[0], k_cache.shape[1])
+    if buffers is not None:
+        _add_outcome_buffers(buffers, q.device)
     return out[row0:row1]
 
 
