@@ -126,6 +126,26 @@ int prism_paged_decode(const void* q, int q_dtype, const int64_t q_strides[3], c
                        float scale, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * A layer's decode step: prism_kv_store of the step's rows, then
+ * prism_paged_decode, with the results of the two calls in that order.  Small
+ * batches on the per-split kernel take one launch for both.
+ *
+ * key/value : [batch, num_kv_heads, head_dim] of q_dtype, strides as in
+ *             prism_kv_store; slot_mapping: int32 [batch].
+ * k/v_cache, k/v_scale : contiguous, as the store needs them; the strides are
+ *             those of prism_paged_decode.
+ */
+int prism_paged_decode_step(const void* key, const void* value, const int64_t key_strides[3],
+                            const int64_t value_strides[3], const int32_t* slot_mapping, const void* q, int q_dtype,
+                            const int64_t q_strides[3], void* k_cache, void* v_cache, int cache_dtype,
+                            const int64_t k_strides[4], const int64_t v_strides[4], float* k_scale, float* v_scale,
+                            const int64_t ks_strides[3], const int64_t vs_strides[3], const int32_t* block_tables,
+                            const int64_t bt_strides[2], const int32_t* context_lens, const int32_t* max_context_len,
+                            void* out, const int64_t out_strides[3], int batch, int num_heads, int num_kv_heads,
+                            int head_dim, int page_size, int64_t num_blocks, int max_blocks_per_seq, float scale,
+                            void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Allocation-free paged decode.  NO COUNTERPART IN THE REFERENCE: for callers
  * that cannot allocate device memory or pass a workspace (code under HIP
  * graph capture, tight serving loops, harnesses that forbid allocation).

@@ -33,6 +33,7 @@
 
 #include "common.h"
 #include "fp8_mfma.h"
+#include "kv_quant.h"
 
 namespace prism {
 namespace {
@@ -95,6 +96,13 @@ struct DecodeArgs {
   int s_tpr, s_ttok;
   int plan_spin;  // streaming path: polls a workgroup waits for a plan build before it gives up
   int vcols;      // streaming path: query columns of a virtual sequence (16, or 32 = two MFMA column blocks)
+  // split-K path with the step's store: the new K and V rows ([batch][kv heads][128]
+  // 16-bit elements) and the slots they go to
+  const uint16_t* new_k;
+  const uint16_t* new_v;
+  int64_t new_k_st, new_v_st;  // token strides, elements
+  const int32_t* slots;
+  int64_t num_slots;
 };
 
 // Read-only int32 metadata (block tables, context lengths) through the
@@ -160,6 +168,7 @@ struct TileRegs {
   float ksc[8];    // k scale of the same 8 tokens
   float vsc[8];    // v scale
   uint32_t kvalid; // bit e: token of slot e is attended
+  int base;        // first cache slot of the tile (a tile in one page; INT_MIN: absent block)
 };
 
 // Token order of the 8 per-lane "slots": e < 4 -> 4g + e; e >= 4 -> 16 + 4g + (e - 4).
@@ -179,6 +188,7 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
     const int32_t blk_raw = use_pre ? blk_pre : bt_row[page * a.bt_sn];
     const bool blk_ok = blk_raw >= 0 && blk_raw < a.num_blocks;
     const int64_t blk = blk_ok ? blk_raw : 0;
+    r.base = blk_ok ? blk_raw * a.page_size + off0 : INT_MIN;
     const uint8_t* kbase = a.k + blk * a.k_sblk + static_cast<int64_t>(off0) * a.k_stok + h * a.k_sh;
     const uint8_t* vbase = a.v + blk * a.v_sblk + static_cast<int64_t>(off0) * a.v_stok + h * a.v_sh;
 #pragma unroll
@@ -250,6 +260,7 @@ struct TileRegs16 {
   u32x4 k[2][4];   // [half][dims 8q .. 8q + 7 of the lane's 32]
   u32x4 v[8];      // V rows of tokens {4g+i, 16+4g+i}, dims 8c..8c+7
   uint32_t kvalid; // bit e: token of slot e is attended
+  int base;        // first cache slot of the tile, as in TileRegs
 };
 
 template <bool PAGE_ALIGNED>
@@ -264,6 +275,7 @@ __device__ __forceinline__ void load_tile16(const DecodeArgs& a, int b, int h, i
     const int32_t blk_raw = use_pre ? blk_pre : bt_row[page * a.bt_sn];
     const bool blk_ok = blk_raw >= 0 && blk_raw < a.num_blocks;
     const int64_t blk = blk_ok ? blk_raw : 0;
+    r.base = blk_ok ? blk_raw * a.page_size + off0 : INT_MIN;
     const uint8_t* kbase = a.k + blk * a.k_sblk + static_cast<int64_t>(off0) * a.k_stok + h * a.k_sh;
     const uint8_t* vbase = a.v + blk * a.v_sblk + static_cast<int64_t>(off0) * a.v_stok + h * a.v_sh;
 #pragma unroll
@@ -399,9 +411,19 @@ __device__ __forceinline__ bool split_arrive(unsigned long long* cnt, unsigned i
 // merged through LDS; a sequence with one live chunk writes its output there
 // and then, otherwise the chunk writes a partial and the last chunk of
 // (sequence, kv head) to arrive merges all of them: no second launch.
-template <int QDT, bool SCALED, bool PAGE_ALIGNED, bool QVEC, int CB>
+//
+// STORE: the step's store runs in the same launch (a separate store of a few
+// rows costs a decode step 4.5 us in a graph, almost all of it launch and
+// latency).  Chunk 0 of (sequence, kv head) writes the sequence's new row to
+// its slot.  Nobody waits for it: a tile that covers a slot of this call,
+// whichever sequence's, takes that row from the call's own K and V (quantised
+// as it is stored) instead of from memory, which may hold the old bytes or
+// the new ones.  4 sequences of 700-4090 tokens, 8 layers from a graph:
+// STEPUS.
+template <int QDT, bool SCALED, bool PAGE_ALIGNED, bool QVEC, int CB, bool STORE>
 __global__ void __launch_bounds__(512)
 paged_decode_split_kernel(const DecodeArgs a) {
+  static_assert(!STORE || (PAGE_ALIGNED && QDT != PRISM_DTYPE_F32 && (SCALED || CB == 2)), "forms with a store");
   // CB: bytes per cache element, 1 (FP8, scaled or unit) or 2 (a bf16 / f16
   // cache of the query's dtype, unscaled)
   static_assert(CB == 1 || (CB == 2 && !SCALED && QDT != PRISM_DTYPE_F32), "16-bit caches: unscaled, 16-bit q");
@@ -427,9 +449,40 @@ paged_decode_split_kernel(const DecodeArgs a) {
   if constexpr (PAGE_ALIGNED) {
     if (t0 < a.width * a.page_size) blk0 = ld_meta(a.bt + static_cast<int64_t>(b) * a.bt_sb + (t0 / a.page_size) * a.bt_sn);
   }
+  // The sequence's new rows (every wave: the tile that holds their slot may be
+  // any wave's) and lane i's slot of sequence i.
+  u32x4 own_k = {0, 0, 0, 0}, own_v = {0, 0, 0, 0};
+  int slot_l = -1;
+  auto new_row = [&](const uint16_t* rows, int64_t stride, int i) {
+    return *reinterpret_cast<const u32x4*>(rows + i * stride + h * kHeadDim + 8 * c);
+  };
+  if constexpr (STORE) {
+    own_k = new_row(a.new_k, a.new_k_st, b);
+    own_v = new_row(a.new_v, a.new_v_st, b);
+    if (lane < a.batch) slot_l = a.slots[lane];
+  }
+  // Chunk 0's last wave writes them: lane group 0 K, group 1 V.
+  auto store_new = [&]() {
+    const int slot = __builtin_amdgcn_readlane(slot_l, b);
+    if (slot < 0 || slot >= a.num_slots || g > 1) return;
+    const int64_t row = static_cast<int64_t>(slot) * nkv + h;
+    const u32x4 raw = g == 0 ? own_k : own_v;
+    uint8_t* cache = const_cast<uint8_t*>(g == 0 ? a.k : a.v);
+    if constexpr (CB == 2) {
+      reinterpret_cast<u32x4*>(cache)[row * (kHeadDim / 8) + c] = raw;
+    } else {
+      float x[8], s;
+      InVec8<QDT == PRISM_DTYPE_F32 ? PRISM_DTYPE_BF16 : QDT>::load(&raw, x);
+      reinterpret_cast<u32x2*>(cache)[row * (kHeadDim / 8) + c] = quantize_row<16>(x, s);
+      if (c == 0) const_cast<float*>(g == 0 ? a.ks : a.vs)[row] = s;
+    }
+  };
   const int n_eff = effective_len(a, b);
   if (c_begin >= n_eff) {
     if (z == 0) {
+      if constexpr (STORE) {
+        if (wv == kSplitWaves - 1) store_new();
+      }
       // No attended token: zeros (the reference kernel's l == 0 branch).
       for (int idx = threadIdx.x; idx < G * kHeadDim; idx += blockDim.x) {
         const int qh = h * G + idx / kHeadDim;
@@ -512,8 +565,60 @@ paged_decode_split_kernel(const DecodeArgs a) {
     }
 
 
+    // Puts the call's new rows into a tile that covers their slots (bit i of
+    // `hit`: sequence i's), in sequence order.
+    auto patch = [&](Tile& cur, uint64_t hit) {
+      while (hit != 0) {
+        const int i = __builtin_ctzll(hit);
+        hit &= hit - 1;
+        const int t = __builtin_amdgcn_readlane(slot_l, i) - cur.base;  // token of the tile
+        const u32x4 kr = i == b ? own_k : new_row(a.new_k, a.new_k_st, i);
+        const u32x4 vr = i == b ? own_v : new_row(a.new_v, a.new_v_st, i);
+        const bool k_lane = c == (t & 15);       // holds K row t in half t / 16
+        const bool v_group = g == (t & 15) / 4;  // holds V row t in slot 4 (t / 16) + t % 4
+        const int ve = (t >> 4) * 4 + (t & 3);
+        if constexpr (CB == 2) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+              const uint32_t w = __shfl(kr[d], 16 * g + 4 * g + q);
+              if (k_lane && t < 16) cur.k[0][q][d] = w;
+              if (k_lane && t >= 16) cur.k[1][q][d] = w;
+            }
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (v_group && e == ve) cur.v[e] = vr;
+        } else {
+          constexpr int kIn = QDT == PRISM_DTYPE_F32 ? PRISM_DTYPE_BF16 : QDT;
+          float x[8], ks, vs;
+          InVec8<kIn>::load(&kr, x);
+          const u32x2 kq = quantize_row<16>(x, ks);
+          InVec8<kIn>::load(&vr, x);
+          const u32x2 vq = quantize_row<16>(x, vs);
+#pragma unroll
+          for (int w = 0; w < 8; ++w) {  // dims 32 g + 4 w .. + 3
+            const uint32_t word = __shfl(kq[w & 1], 16 * g + 4 * g + w / 2);
+            if (k_lane && t < 16) cur.k[0][w >> 2][w & 3] = word;
+            if (k_lane && t >= 16) cur.k[1][w >> 2][w & 3] = word;
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (v_group && e == ve) {
+              cur.v[e] = vq;
+              cur.ksc[e] = ks;
+              cur.vsc[e] = vs;
+            }
+        }
+      }
+    };
+
     // One 32-token tile of kv head h: QK, online softmax, PV.
     auto compute = [&](Tile& cur) {
+      if constexpr (STORE) {
+        const uint64_t hit = __builtin_amdgcn_ballot_w64(slot_l >= cur.base && slot_l < cur.base + kTile);
+        if (hit != 0) patch(cur, hit);
+      }
       // ---- QK
       floatx4 sc[2];
 #pragma unroll
@@ -679,6 +784,10 @@ paged_decode_split_kernel(const DecodeArgs a) {
       t0 += kStep;
       if (t0 >= c_end) break;
     }
+  }
+
+  if constexpr (STORE) {
+    if (z == 0 && wv == kSplitWaves - 1) store_new();
   }
 
   // ---- merge the eight waves through LDS.  Wave w's row r (q head h*G + r)
@@ -3420,12 +3529,19 @@ int launch_all(int stage, const DecodeArgs& args, const Geometry& geo, bool page
   {
     const dim3 grid(args.batch, args.num_kv_heads, geo.max_splits);
     const dim3 block(64 * kSplitWaves);
-#define PRISM_LAUNCH_SPLIT(S, A, CB)                                                                   \
-  do {                                                                                                 \
-    if (args.q_vec)                                                                                    \
-      hipLaunchKernelGGL((paged_decode_split_kernel<QDT, S, A, true, CB>), grid, block, 0, stream, args);  \
-    else                                                                                               \
-      hipLaunchKernelGGL((paged_decode_split_kernel<QDT, S, A, false, CB>), grid, block, 0, stream, args); \
+    if (args.slots != nullptr) {  // the step's store in the same launch (prism_paged_decode_step chose the form)
+      if constexpr (QDT != PRISM_DTYPE_F32) {
+        if (scaled) hipLaunchKernelGGL((paged_decode_split_kernel<QDT, true, true, true, 1, true>), grid, block, 0, stream, args);
+        else hipLaunchKernelGGL((paged_decode_split_kernel<QDT, false, true, true, 2, true>), grid, block, 0, stream, args);
+      }
+      return check_launch("paged_decode_split_kernel launch");
+    }
+#define PRISM_LAUNCH_SPLIT(S, A, CB)                                                                          \
+  do {                                                                                                        \
+    if (args.q_vec)                                                                                           \
+      hipLaunchKernelGGL((paged_decode_split_kernel<QDT, S, A, true, CB, false>), grid, block, 0, stream, args);  \
+    else                                                                                                      \
+      hipLaunchKernelGGL((paged_decode_split_kernel<QDT, S, A, false, CB, false>), grid, block, 0, stream, args); \
   } while (0)
     if (args.cache_dtype != PRISM_DTYPE_FP8_E4M3FN) {  // 16-bit cache of the query's dtype, unscaled
       if constexpr (QDT != PRISM_DTYPE_F32) {
@@ -3510,8 +3626,20 @@ extern "C" int prism_paged_decode_kernel_family(int batch, int num_heads, int nu
   return geo.stream_shape ? 2 : 1;
 }
 
-extern "C" int prism_paged_decode_stage(
-    int stage, const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache, const void* v_cache,
+namespace prism {
+namespace {
+
+// A decode step's store, for the launch that can take it along.
+struct StepStore {
+  const void* key;
+  const void* value;
+  int64_t k_st, v_st;  // token strides, elements
+  const int32_t* slots;
+  bool taken;  // set by decode_call: the decode's launch stores the rows
+};
+
+int decode_call(
+    StepStore* step, int stage, const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache, const void* v_cache,
     int cache_dtype, const int64_t k_strides[4], const int64_t v_strides[4], const float* k_scale,
     const float* v_scale, const int64_t ks_strides[3], const int64_t vs_strides[3], const int32_t* block_tables,
     const int64_t bt_strides[2], const int32_t* context_lens, const int32_t* max_context_len, void* out,
@@ -3674,12 +3802,85 @@ extern "C" int prism_paged_decode_stage(
     args.vcols = geo.stream_vcols;
     args.plan_spin = env_overrides().plan_spin.load();
   }
+  if (step != nullptr) {
+    // The store joins the split-K kernel in its main forms: scaled FP8 or a
+    // 16-bit cache of the query's dtype, tiles within a page, aligned dense
+    // rows, at most one slot per lane, and the contiguous cache that the store
+    // addresses by slot.  Everything else takes two launches.
+    const int64_t tok = static_cast<int64_t>(num_kv_heads) * kHeadDim;
+    auto canonical = [&](const int64_t* st) { return st[0] == tok * page_size && st[1] == tok && st[2] == kHeadDim; };
+    auto canonical_scales = [&](const int64_t* st) {
+      return st[0] == static_cast<int64_t>(num_kv_heads) * page_size && st[1] == num_kv_heads && st[2] == 1;
+    };
+    step->taken = geo.fast && !use_stream && page_aligned && args.q_vec && batch <= 64 &&
+                  (q_dtype == PRISM_DTYPE_BF16 || q_dtype == PRISM_DTYPE_F16) &&
+                  (k_scale ? canonical_scales(ks_strides) && canonical_scales(vs_strides) : cache_dtype == q_dtype) &&
+                  canonical(k_strides) && canonical(v_strides) && num_blocks * page_size <= INT32_MAX &&
+                  aligned(step->key, 16) && aligned(step->value, 16) && step->k_st % 8 == 0 && step->v_st % 8 == 0;
+    if (!step->taken) return PRISM_OK;
+    args.new_k = static_cast<const uint16_t*>(step->key);
+    args.new_v = static_cast<const uint16_t*>(step->value);
+    args.new_k_st = step->k_st;
+    args.new_v_st = step->v_st;
+    args.slots = step->slots;
+    args.num_slots = num_blocks * page_size;
+  }
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   switch (q_dtype) {
     case PRISM_DTYPE_BF16: return launch_all<PRISM_DTYPE_BF16>(stage, args, geo, page_aligned, use_stream, stream);
     case PRISM_DTYPE_F16: return launch_all<PRISM_DTYPE_F16>(stage, args, geo, page_aligned, use_stream, stream);
     default: return launch_all<PRISM_DTYPE_F32>(stage, args, geo, page_aligned, use_stream, stream);
   }
+}
+
+}  // namespace
+}  // namespace prism
+
+extern "C" int prism_paged_decode_stage(
+    int stage, const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache, const void* v_cache,
+    int cache_dtype, const int64_t k_strides[4], const int64_t v_strides[4], const float* k_scale,
+    const float* v_scale, const int64_t ks_strides[3], const int64_t vs_strides[3], const int32_t* block_tables,
+    const int64_t bt_strides[2], const int32_t* context_lens, const int32_t* max_context_len, void* out,
+    const int64_t out_strides[3], int batch, int num_heads, int num_kv_heads, int head_dim, int page_size,
+    int64_t num_blocks, int max_blocks_per_seq, float scale, void* workspace, int64_t workspace_bytes,
+    void* stream_ptr) {
+  return prism::decode_call(nullptr, stage, q, q_dtype, q_strides, k_cache, v_cache, cache_dtype, k_strides, v_strides,
+                            k_scale, v_scale, ks_strides, vs_strides, block_tables, bt_strides, context_lens,
+                            max_context_len, out, out_strides, batch, num_heads, num_kv_heads, head_dim, page_size,
+                            num_blocks, max_blocks_per_seq, scale, workspace, workspace_bytes, stream_ptr);
+}
+
+extern "C" int prism_paged_decode_step(
+    const void* key, const void* value, const int64_t key_strides[3], const int64_t value_strides[3],
+    const int32_t* slot_mapping, const void* q, int q_dtype, const int64_t q_strides[3], void* k_cache, void* v_cache,
+    int cache_dtype, const int64_t k_strides[4], const int64_t v_strides[4], float* k_scale, float* v_scale,
+    const int64_t ks_strides[3], const int64_t vs_strides[3], const int32_t* block_tables, const int64_t bt_strides[2],
+    const int32_t* context_lens, const int32_t* max_context_len, void* out, const int64_t out_strides[3], int batch,
+    int num_heads, int num_kv_heads, int head_dim, int page_size, int64_t num_blocks, int max_blocks_per_seq,
+    float scale, void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace prism;
+  if (batch > 0 && (!key || !value || !key_strides || !value_strides || !slot_mapping)) {
+    clear_error();
+    set_error("prism_paged_decode_step: null pointer argument");
+    return PRISM_ERR_INVALID;
+  }
+  auto decode = [&](StepStore* step) {
+    return decode_call(step, 0, q, q_dtype, q_strides, k_cache, v_cache, cache_dtype, k_strides, v_strides, k_scale,
+                       v_scale, ks_strides, vs_strides, block_tables, bt_strides, context_lens, max_context_len, out,
+                       out_strides, batch, num_heads, num_kv_heads, head_dim, page_size, num_blocks,
+                       max_blocks_per_seq, scale, workspace, workspace_bytes, stream);
+  };
+  if (batch > 0 && key_strides[2] == 1 && value_strides[2] == 1 && key_strides[1] == head_dim &&
+      value_strides[1] == head_dim) {
+    StepStore step{key, value, key_strides[0], value_strides[0], slot_mapping, false};
+    if (const int rc = decode(&step); rc != PRISM_OK || step.taken) return rc;
+  }
+  if (const int rc = prism_kv_store(key, value, q_dtype, key_strides, value_strides, k_cache, v_cache, cache_dtype,
+                                    k_scale, v_scale, slot_mapping, batch, num_kv_heads, head_dim,
+                                    num_blocks * page_size, stream);
+      rc != PRISM_OK)
+    return rc;
+  return decode(nullptr);
 }
 
 extern "C" int prism_paged_decode(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,

@@ -9,9 +9,9 @@
 // the GPU needs 14; a 3001-token store 13.0 and 4.9 us; a prefill reads its
 // outcome from pinned memory instead of through a concatenation and a copy,
 // 18 us less).  They only take calls that they can prove good: anything else
-// (another device than the current one, graph capture, a tensor subclass, no
-// workspace yet, a contract violation, an error status) returns None, and the
-// caller's Python path handles it, with its messages.
+// (another device than the current one, a tensor subclass, no workspace yet, a
+// contract violation, an error status) returns None, and the caller's Python
+// path handles it, with its messages.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -142,52 +142,108 @@ struct Strides {
   }
 };
 
+// A paged decode's arguments, checked: decode's of eleven (from args[0]).
+struct DecodeCall {
+  const at::Tensor *q, *kc, *vc, *bt, *ctx, *max_ctx, *ks, *vs;
+  double scale;
+  int device, qd, cd;
+  int64_t batch, heads, dim, blocks, page, kv_heads, width;
+  void* stream;
+  int64_t need;       // workspace bytes
+  at::Tensor ws_own;  // a captured call's workspace, from the graph's pool
+  void* ws;
+};
+
+bool check_decode(PyObject* const* args, DecodeCall& d) {
+  d.q = tensor(args[0]), d.kc = tensor(args[1]), d.vc = tensor(args[2]), d.bt = tensor(args[3]);
+  d.ctx = tensor(args[4]), d.max_ctx = tensor(args[8]);
+  if (!d.q || !d.kc || !d.vc || !d.bt || !d.ctx || !d.max_ctx || !optional_pair(args[6], args[7], d.ks, d.vs)) return false;
+  if (!PyFloat_CheckExact(args[5]) || !PyLong_CheckExact(args[9])) return false;
+  d.scale = PyFloat_AS_DOUBLE(args[5]);
+  int overflow = 0;
+  const long block_n = PyLong_AsLongAndOverflow(args[9], &overflow);
+  if (overflow || block_n <= 0 || (block_n & (block_n - 1))) return false;
+  const at::Tensor &q = *d.q, &kc = *d.kc;
+  if (!on_current_device(d.device, d.q, d.kc, d.vc, d.bt, d.ctx, d.max_ctx, d.ks, d.vs)) return false;
+  if (q.dim() != 3 || kc.dim() != 4 || kc.sizes() != d.vc->sizes() || kc.scalar_type() != d.vc->scalar_type() ||
+      d.bt->dim() != 2 || d.ctx->dim() != 1 || d.bt->scalar_type() != at::kInt || d.ctx->scalar_type() != at::kInt ||
+      !d.ctx->is_contiguous() || d.max_ctx->numel() != 1 || d.max_ctx->scalar_type() != at::kInt ||
+      !scale_pair(kc, d.ks, d.vs))
+    return false;
+  d.batch = q.size(0), d.heads = q.size(1), d.dim = q.size(2);
+  d.blocks = kc.size(0), d.page = kc.size(1), d.kv_heads = kc.size(2), d.width = d.bt->size(1);
+  d.qd = dtype_code(q.scalar_type()), d.cd = dtype_code(kc.scalar_type());
+  if (d.qd < 0 || d.qd == PRISM_DTYPE_FP8_E4M3FN || d.cd < 0 || d.batch <= 0 || d.heads <= 0 || d.dim <= 0 ||
+      d.dim > 256 || kc.size(3) != d.dim || d.page <= 0 || d.kv_heads <= 0 || d.heads % d.kv_heads != 0 ||
+      d.bt->size(0) < d.batch || d.ctx->size(0) < d.batch || kc.stride(3) != 1 || d.batch > INT32_MAX ||
+      d.heads > INT32_MAX || d.page > INT32_MAX || d.width > INT32_MAX)
+    return false;
+  d.stream = current_stream(d.device);
+  d.need = prism_paged_decode_workspace_bytes(static_cast<int>(d.batch), static_cast<int>(d.heads),
+                                              static_cast<int>(d.kv_heads), static_cast<int>(d.dim),
+                                              static_cast<int>(d.page), static_cast<int>(d.width), d.cd);
+  d.ws = nullptr;
+  if (d.need > 0) {
+    if (capturing()) {
+      d.ws_own = at::empty({d.need}, q.options().dtype(at::kByte));
+      d.ws = d.ws_own.data_ptr();
+    } else {
+      PyObject* found = by_stream(args[10], d.device, d.stream);
+      const at::Tensor* ws = found ? tensor(found) : nullptr;
+      if (ws == nullptr || ws->numel() < d.need) return false;
+      d.ws = ws->data_ptr();
+    }
+  }
+  return true;
+}
+
+const float* scales(const at::Tensor* t) { return t ? static_cast<const float*>(t->data_ptr()) : nullptr; }
+
 // decode(q, k_cache, v_cache, block_tables, context_lens, scale, k_scale, v_scale, max_context_len, block_n,
 //        workspaces) -> output or None
 PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 11) Py_RETURN_NONE;
-  const at::Tensor *q = tensor(args[0]), *kc = tensor(args[1]), *vc = tensor(args[2]), *bt = tensor(args[3]),
-                   *ctx = tensor(args[4]), *max_ctx = tensor(args[8]), *ks, *vs;
-  if (!q || !kc || !vc || !bt || !ctx || !max_ctx || !optional_pair(args[6], args[7], ks, vs)) Py_RETURN_NONE;
-  if (!PyFloat_CheckExact(args[5]) || !PyLong_CheckExact(args[9])) Py_RETURN_NONE;
-  const double scale = PyFloat_AS_DOUBLE(args[5]);
-  int overflow = 0;
-  const long block_n = PyLong_AsLongAndOverflow(args[9], &overflow);
-  if (overflow || block_n <= 0 || (block_n & (block_n - 1))) Py_RETURN_NONE;
-  int device;
-  if (!on_current_device(device, q, kc, vc, bt, ctx, max_ctx, ks, vs) || capturing()) Py_RETURN_NONE;
-  if (q->dim() != 3 || kc->dim() != 4 || kc->sizes() != vc->sizes() || kc->scalar_type() != vc->scalar_type() ||
-      bt->dim() != 2 || ctx->dim() != 1 || bt->scalar_type() != at::kInt || ctx->scalar_type() != at::kInt ||
-      !ctx->is_contiguous() || max_ctx->numel() != 1 || max_ctx->scalar_type() != at::kInt || !scale_pair(*kc, ks, vs))
-    Py_RETURN_NONE;
-  const int64_t batch = q->size(0), heads = q->size(1), dim = q->size(2);
-  const int64_t blocks = kc->size(0), page = kc->size(1), kv_heads = kc->size(2), width = bt->size(1);
-  const int qd = dtype_code(q->scalar_type()), cd = dtype_code(kc->scalar_type());
-  if (qd < 0 || qd == PRISM_DTYPE_FP8_E4M3FN || cd < 0 || batch <= 0 || heads <= 0 || dim <= 0 || dim > 256 ||
-      kc->size(3) != dim || page <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || bt->size(0) < batch ||
-      ctx->size(0) < batch || kc->stride(3) != 1 || batch > INT32_MAX || heads > INT32_MAX || page > INT32_MAX ||
-      width > INT32_MAX)
-    Py_RETURN_NONE;
-  void* stream = current_stream(device);
-  const int64_t need = prism_paged_decode_workspace_bytes(static_cast<int>(batch), static_cast<int>(heads),
-                                                          static_cast<int>(kv_heads), static_cast<int>(dim),
-                                                          static_cast<int>(page), static_cast<int>(width), cd);
-  const at::Tensor* ws = nullptr;
-  if (need > 0) {
-    PyObject* found = by_stream(args[10], device, stream);
-    ws = found ? tensor(found) : nullptr;
-    if (ws == nullptr || ws->numel() < need) Py_RETURN_NONE;
-  }
-  at::Tensor out = at::empty_like(*q);
-  const Strides sq(q), sk(kc), sv(vc), sks(ks), svs(vs), sbt(bt), so(&out);
+  DecodeCall d;
+  if (n != 11 || !check_decode(args, d)) Py_RETURN_NONE;
+  at::Tensor out = at::empty_like(*d.q);
+  const Strides sq(d.q), sk(d.kc), sv(d.vc), sks(d.ks), svs(d.vs), sbt(d.bt), so(&out);
   const int rc = prism_paged_decode(
-      q->data_ptr(), qd, sq.v, kc->data_ptr(), vc->data_ptr(), cd, sk.v, sv.v,
-      ks ? static_cast<const float*>(ks->data_ptr()) : nullptr, vs ? static_cast<const float*>(vs->data_ptr()) : nullptr,
-      sks.v, svs.v, static_cast<const int32_t*>(bt->data_ptr()), sbt.v, static_cast<const int32_t*>(ctx->data_ptr()),
-      static_cast<const int32_t*>(max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(batch),
-      static_cast<int>(heads), static_cast<int>(kv_heads), static_cast<int>(dim), static_cast<int>(page), blocks,
-      static_cast<int>(width), static_cast<float>(scale), ws ? ws->data_ptr() : nullptr, need, stream);
+      d.q->data_ptr(), d.qd, sq.v, d.kc->data_ptr(), d.vc->data_ptr(), d.cd, sk.v, sv.v, scales(d.ks), scales(d.vs),
+      sks.v, svs.v, static_cast<const int32_t*>(d.bt->data_ptr()), sbt.v, static_cast<const int32_t*>(d.ctx->data_ptr()),
+      static_cast<const int32_t*>(d.max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(d.batch),
+      static_cast<int>(d.heads), static_cast<int>(d.kv_heads), static_cast<int>(d.dim), static_cast<int>(d.page),
+      d.blocks, static_cast<int>(d.width), static_cast<float>(d.scale), d.ws, d.need, d.stream);
+  if (rc != PRISM_OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// step(decode's eleven, key, value, slot_mapping) -> output or None: the store
+// of the step's rows, then the decode
+PyObject* step(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  DecodeCall d;
+  if (n != 14 || !check_decode(args, d)) Py_RETURN_NONE;
+  const at::Tensor *key = tensor(args[11]), *value = tensor(args[12]), *slots = tensor(args[13]);
+  int device;
+  if (!key || !value || !slots || !on_current_device(device, key, value, slots) || device != d.device) Py_RETURN_NONE;
+  if (key->dim() != 3 || key->sizes() != value->sizes() || key->size(0) != d.batch || key->size(1) != d.kv_heads ||
+      key->size(2) != d.dim || slots->dim() != 1 || slots->numel() != d.batch || slots->scalar_type() != at::kInt ||
+      !slots->is_contiguous() || key->scalar_type() != d.q->scalar_type() ||
+      value->scalar_type() != d.q->scalar_type() || key->stride(2) != 1 || value->stride(2) != 1 ||
+      key->stride(1) != d.dim || value->stride(1) != d.dim || !d.kc->is_contiguous() || !d.vc->is_contiguous() ||
+      (d.ks && (!d.ks->is_contiguous() || !d.vs->is_contiguous())))
+    Py_RETURN_NONE;
+  at::Tensor out = at::empty_like(*d.q);
+  const Strides skey(key), sval(value), sq(d.q), sk(d.kc), sv(d.vc), sks(d.ks), svs(d.vs), sbt(d.bt), so(&out);
+  const int rc = prism_paged_decode_step(
+      key->data_ptr(), value->data_ptr(), skey.v, sval.v, static_cast<const int32_t*>(slots->data_ptr()),
+      d.q->data_ptr(), d.qd, sq.v, d.kc->data_ptr(), d.vc->data_ptr(), d.cd, sk.v, sv.v,
+      const_cast<float*>(scales(d.ks)), const_cast<float*>(scales(d.vs)), sks.v, svs.v,
+      static_cast<const int32_t*>(d.bt->data_ptr()), sbt.v, static_cast<const int32_t*>(d.ctx->data_ptr()),
+      static_cast<const int32_t*>(d.max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(d.batch),
+      static_cast<int>(d.heads), static_cast<int>(d.kv_heads), static_cast<int>(d.dim), static_cast<int>(d.page),
+      d.blocks, static_cast<int>(d.width), static_cast<float>(d.scale), d.ws, d.need, d.stream);
   if (rc != PRISM_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -266,6 +322,7 @@ PyMethodDef methods[] = {
     {"mark_ready", mark_ready, METH_O, nullptr},
     {"store", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(store)), METH_FASTCALL, nullptr},
     {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(decode)), METH_FASTCALL, nullptr},
+    {"step", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(step)), METH_FASTCALL, nullptr},
     {"prefill", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(prefill)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

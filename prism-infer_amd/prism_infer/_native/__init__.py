@@ -68,6 +68,11 @@ SIGNATURES: dict[str, tuple] = {
         [_I, _VP, _I, _I64P, _VP, _VP, _I, _I64P, _I64P, _VP, _VP, _I64P, _I64P, _VP, _I64P, _VP, _VP, _VP,
          _I64P, _I, _I, _I, _I, _I, _I64, _I, _F, _VP, _I64, _VP],
     ),
+    "prism_paged_decode_step": (
+        _I,
+        [_VP, _VP, _I64P, _I64P, _VP, _VP, _I, _I64P, _VP, _VP, _I, _I64P, _I64P, _VP, _VP, _I64P, _I64P, _VP, _I64P,
+         _VP, _VP, _VP, _I64P, _I, _I, _I, _I, _I, _I64, _I, _F, _VP, _I64, _VP],
+    ),
     "prism_compact_slots_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64]),
     "prism_compact_slots": (_I, [_VP, _I64, _I64, _I64, _VP, _VP, _I64, _VP, _I64, _VP]),
     "prism_copy_blocks": (_I, [_VP, _VP, _I64, _I64, _I64, _I64, _I64, _I64, _I64P, _I64P, _I64, _VP]),

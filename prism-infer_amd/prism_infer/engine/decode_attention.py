@@ -22,8 +22,11 @@ from dataclasses import dataclass
 
 import torch
 
+from prism_infer import _native, observability
 from prism_infer.ops.kv_cache_store import store_kvcache
-from prism_infer.ops.paged_decode import paged_decode_attention
+from prism_infer.ops.paged_decode import _WORKSPACES, DEFAULT_PAGED_DECODE_BLOCK_N, paged_decode_attention
+
+_HOST = _native.host_ops()
 
 
 @dataclass
@@ -127,6 +130,15 @@ class PagedKVDecodeAttention:
         self._validate_cache_bindings()
         if metadata.slot_mapping is None:
             raise RuntimeError("bound KV cache requires slot_mapping")
+        # both ops in one native call, and for small batches in one launch; what
+        # it does not take, and every call while a profiling provider is
+        # installed, goes through the two ops
+        if _HOST is not None and observability._region_provider is None:
+            out = _HOST.step(q, self.k_cache, self.v_cache, metadata.block_tables, metadata.context_lens, self.scale,
+                             self.k_scale_cache, self.v_scale_cache, metadata.max_context_len,
+                             DEFAULT_PAGED_DECODE_BLOCK_N, _WORKSPACES, k, v, metadata.slot_mapping)
+            if out is not None:
+                return out
         store_kvcache(k, v, self.k_cache, self.v_cache, metadata.slot_mapping, self.k_scale_cache,
                       self.v_scale_cache)
         return paged_decode_attention(
