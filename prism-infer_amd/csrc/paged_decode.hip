@@ -165,8 +165,7 @@ __device__ __forceinline__ void store_out8(const Args& a, int64_t idx, const flo
 struct TileRegs {
   u32x4 k[2][2];   // [half][part]: 32 bytes of K row (c + 16 * half), dims 32g..32g+31
   u32x2 v[8];      // V rows of tokens {4g+i, 16+4g+i}, dims 8c..8c+7
-  float ksc[8];    // k scale of the same 8 tokens
-  float vsc[8];    // v scale
+  float scale;     // lanes 0..31: k scale of token t0 + lane, lanes 32..63: v scales
   uint32_t kvalid; // bit e: token of slot e is attended
   int base;        // first cache slot of the tile (a tile in one page; INT_MIN: absent block)
 };
@@ -197,22 +196,35 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
       r.k[hh][0] = p[0];
       r.k[hh][1] = p[1];
     }
-    const float* ksb = a.ks + blk * a.ks_sblk + static_cast<int64_t>(off0) * a.ks_stok + h * a.ks_sh;
-    const float* vsb = a.vs + blk * a.vs_sblk + static_cast<int64_t>(off0) * a.vs_stok + h * a.vs_sh;
+    // the tile's 64 scales in one load: lane l < 32 token l's k scale, lane
+    // 32 + l its v scale (one load per token a lane weighs was 16 of the 28
+    // loads of a tile)
+    r.scale = 1.f;
+    if (SCALED) {
+      const int64_t tok = off0 + (c + 16 * (g & 1));
+      r.scale = g < 2 ? a.ks[blk * a.ks_sblk + tok * a.ks_stok + h * a.ks_sh]
+                      : a.vs[blk * a.vs_sblk + tok * a.vs_stok + h * a.vs_sh];
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int tk = slot_token(g, e);
       r.v[e] = *reinterpret_cast<const u32x2*>(vbase + tk * a.v_stok + 8 * c);
-      if (SCALED) {
-        r.ksc[e] = ksb[tk * a.ks_stok];
-        r.vsc[e] = vsb[tk * a.vs_stok];
-      } else {
-        r.ksc[e] = r.vsc[e] = 1.f;
-      }
       r.kvalid |= (blk_ok && t0 + tk < t_end) ? (1u << e) : 0u;
     }
   } else {
     // Tiles may straddle pages: resolve every row separately.
+    r.scale = SCALED ? 0.f : 1.f;
+    if (SCALED) {
+      const int tok = t0 + c + 16 * (g & 1);
+      if (tok < t_end) {
+        const int page = tok / a.page_size;
+        const int64_t off = tok - page * a.page_size;
+        const int32_t blk = bt_row[page * a.bt_sn];
+        if (blk >= 0 && blk < a.num_blocks)
+          r.scale = g < 2 ? a.ks[blk * a.ks_sblk + off * a.ks_stok + h * a.ks_sh]
+                          : a.vs[blk * a.vs_sblk + off * a.vs_stok + h * a.vs_sh];
+      }
+    }
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       const int tok = t0 + c + 16 * hh;
@@ -232,7 +244,6 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
     for (int e = 0; e < 8; ++e) {
       const int tok = t0 + slot_token(g, e);
       r.v[e] = u32x2{0, 0};
-      r.ksc[e] = r.vsc[e] = 0.f;
       if (tok < t_end) {
         const int page = tok / a.page_size;
         const int off = tok - page * a.page_size;
@@ -240,12 +251,6 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
         if (blk >= 0 && blk < a.num_blocks) {
           r.v[e] = *reinterpret_cast<const u32x2*>(a.v + blk * a.v_sblk + static_cast<int64_t>(off) * a.v_stok +
                                                    h * a.v_sh + 8 * c);
-          if (SCALED) {
-            r.ksc[e] = a.ks[blk * a.ks_sblk + static_cast<int64_t>(off) * a.ks_stok + h * a.ks_sh];
-            r.vsc[e] = a.vs[blk * a.vs_sblk + static_cast<int64_t>(off) * a.vs_stok + h * a.vs_sh];
-          } else {
-            r.ksc[e] = r.vsc[e] = 1.f;
-          }
           r.kvalid |= 1u << e;
         }
       }
@@ -418,8 +423,8 @@ __device__ __forceinline__ bool split_arrive(unsigned long long* cnt, unsigned i
 // its slot.  Nobody waits for it: a tile that covers a slot of this call,
 // whichever sequence's, takes that row from the call's own K and V (quantised
 // as it is stored) instead of from memory, which may hold the old bytes or
-// the new ones.  4 sequences of 700-4090 tokens, 8 layers from a graph:
-// STEPUS.
+// the new ones.  4 sequences of 700-4090 tokens, 8 layers from a graph: 171 us
+// with the store's launch, 153 without, 142 with the tile's scales in one load.
 template <int QDT, bool SCALED, bool PAGE_ALIGNED, bool QVEC, int CB, bool STORE>
 __global__ void __launch_bounds__(512)
 paged_decode_split_kernel(const DecodeArgs a) {
@@ -495,6 +500,7 @@ paged_decode_split_kernel(const DecodeArgs a) {
   const int c_end = min(c_begin + a.split, n_eff);
   const int n_live = (n_eff + a.split - 1) / a.split;  // chunks with attended tokens (>= 1)
 
+  __shared__ __attribute__((aligned(16))) float s_scale[kSplitWaves][64];
   floatx4 acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -604,11 +610,9 @@ paged_decode_split_kernel(const DecodeArgs a) {
           }
 #pragma unroll
           for (int e = 0; e < 8; ++e)
-            if (v_group && e == ve) {
-              cur.v[e] = vq;
-              cur.ksc[e] = ks;
-              cur.vsc[e] = vs;
-            }
+            if (v_group && e == ve) cur.v[e] = vq;
+          if (lane == t) cur.scale = ks;
+          if (lane == 32 + t) cur.scale = vs;
         }
       }
     };
@@ -619,6 +623,15 @@ paged_decode_split_kernel(const DecodeArgs a) {
         const uint64_t hit = __builtin_amdgcn_ballot_w64(slot_l >= cur.base && slot_l < cur.base + kTile);
         if (hit != 0) patch(cur, hit);
       }
+      // The scales change hands through the wave's own LDS (no barrier: only
+      // this wave reads them, in order behind its write).
+      float ksc[8], vsc[8];
+      if constexpr (CB == 1 && SCALED) {
+        __builtin_amdgcn_wave_barrier();
+        s_scale[wv][lane] = cur.scale;
+        __builtin_amdgcn_wave_barrier();
+      }
+
       // ---- QK
       floatx4 sc[2];
 #pragma unroll
@@ -650,15 +663,26 @@ paged_decode_split_kernel(const DecodeArgs a) {
         sc[hh] = accs;
       }
 
+      if constexpr (CB == 1 && SCALED) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const floatx4 kq = *reinterpret_cast<const floatx4*>(&s_scale[wv][16 * q + 4 * g]);
+          const floatx4 vq = *reinterpret_cast<const floatx4*>(&s_scale[wv][32 + 16 * q + 4 * g]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ksc[4 * q + i] = kq[i], vsc[4 * q + i] = vq[i];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ksc[e] = vsc[e] = 1.f;
+      }
+
       // ---- online softmax (log2 domain).  Value e of this lane: half e/4, row e%4.
       float x[8];
       float tmax = -INFINITY;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const bool ok = ((cur.kvalid >> e) & 1u) && c < G;
-        float ksc = 1.f;
-        if constexpr (CB == 1) ksc = cur.ksc[e];
-        const float v = sc[e >> 2][e & 3] * (ksc * a.scale_log2);
+        const float v = sc[e >> 2][e & 3] * (ksc[e] * a.scale_log2);
         x[e] = ok ? v : -INFINITY;
         tmax = fmaxf(tmax, x[e]);
       }
@@ -679,9 +703,7 @@ paged_decode_split_kernel(const DecodeArgs a) {
       for (int e = 0; e < 8; ++e) {
         const float p = exp2f(x[e] - m_use);  // 0 for masked slots
         psum += p;
-        float vsc = 1.f;
-        if constexpr (CB == 1) vsc = cur.vsc[e];
-        const float pv = ((cur.kvalid >> e) & 1u) ? p * vsc : 0.f;
+        const float pv = ((cur.kvalid >> e) & 1u) ? p * vsc[e] : 0.f;
         if constexpr (CB == 2 && QDT == PRISM_DTYPE_F16) {
           const _Float16 hi = static_cast<_Float16>(pv);
           pa[e] = hi;
