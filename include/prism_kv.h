@@ -337,6 +337,10 @@ int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], 
  * 0 where none is used.  With it, few query blocks behind long contexts have
  * their keys split over several workgroups, whose fp32 partials a second
  * kernel merges; with less, or NULL, every block is one workgroup's.
+ * `report` (int32[3] in pinned host memory, or NULL) lets a host see the
+ * outcome with one wait for the stream and no copy: report[0], set to 0 by the
+ * caller, becomes 1 where a sequence is recorded in `status`; report[1] and
+ * report[2] get cu_seqlens_q[0] and cu_seqlens_q[batch].
  */
 int64_t prism_paged_prefill_workspace_bytes(int batch, int total_q, int num_heads, int num_kv_heads, int page_size,
                                             int width);
@@ -349,15 +353,8 @@ int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t q_strides[3
                            const int32_t* context_lens, const int32_t* cu_seqlens_q, void* out,
                            const int64_t out_strides[3], int batch, int total_q, int num_heads,
                            int num_kv_heads, int head_dim, int page_size, int num_blocks, int width,
-                           float scale, int32_t* status, void* workspace, int64_t workspace_bytes, void* stream);
-
-/*
- * Writes {status[0], cu_seqlens_q[0], cu_seqlens_q[batch]} to `out` (int32[3];
- * device memory or pinned host memory), for a host that reads the outcome of
- * prism_paged_prefill back with one wait for the stream and no copy.
- */
-int prism_paged_prefill_report(const int32_t* status, const int32_t* cu_seqlens_q, int batch, int32_t* out,
-                               void* stream);
+                           float scale, int32_t* status, void* workspace, int64_t workspace_bytes, int32_t* report,
+                           void* stream);
 
 /*
  * Test hook with no counterpart in the reference: converts n fp32 values to

@@ -81,9 +81,12 @@ struct PrefillArgs {
   int batch, num_heads, groups, page, num_blocks, width;
   float scale_log2;
   int* status;
+  int* report;    // pinned: [0] set to 1 where a sequence is flagged, [1] and [2] the packed rows' extent; or null
   int out_vec;    // output rows can be stored 8 bytes at a time
-  int splits;     // workgroups per (block, kv head)
+  int splits;     // most workgroups per (block, kv head); the kernel takes as many of them as fill the chip
+  int slots;      // workgroups that the chip holds at once
   int total_q;
+  int* used;      // splits that the kernel took (written for the merge)
   float* part;    // [splits][total_q][num_heads][kPfD] unnormalised outputs, then [..][2] (max, sum)
 };
 
@@ -115,6 +118,7 @@ __device__ __forceinline__ int uniform_int(int v) { return __builtin_amdgcn_read
 
 __device__ __forceinline__ void flag_sequence(const PrefillArgs& a, int seq) {
   atomicMin(a.status, seq);
+  if (a.report != nullptr) a.report[0] = 1;  // (every writer stores the same)
 }
 
 // Inclusive wave scan with f over lanes of non-negative values (0 is f's
@@ -158,19 +162,42 @@ __device__ __forceinline__ int seq_blocks(const PrefillArgs& a, int i, bool flag
   return (qlen + QT - 1) / QT;
 }
 
+// A workgroup's work: query block, part of its keys, kv head.
+struct PfWork {
+  int seq, qblock, split, splits, head;
+};
+
+// Workgroup id -> work, from the number of real blocks: heads fastest (so that
+// the long blocks of all heads start first and, with 8 kv heads, each XCD
+// reads one head's K/V), then the parts of the keys, then the block's rank.
+// Returns the rank.  The keys are split as often as the chip has room for the
+// blocks' workgroups.
+__device__ __forceinline__ int pf_parts(const PrefillArgs& a, int kv_heads, int total, PfWork& w) {
+  w.splits = 1;
+  if (a.splits > 1 && total > 0) w.splits = uniform_int(min(max(a.slots / (total * kv_heads), 1), a.splits));
+  const int per_block = kv_heads * w.splits;
+  const int rank = uniform_int(static_cast<int>(blockIdx.x) / per_block);
+  const int rest = static_cast<int>(blockIdx.x) - rank * per_block;
+  w.split = uniform_int(rest / kv_heads);
+  w.head = rest - w.split * kv_heads;
+  return rank;
+}
+
 // Rank (0 first) -> (sequence, query block), the blocks with most keys first:
 // the launch then ends on short blocks.  Blocks above a level u: a sum over
 // the sequences; the rank's level comes from a binary search over u, its
 // sequence from a scan over those with a block at that level.  Returns false
-// for a rank beyond the real blocks.
+// for a workgroup beyond the real blocks.
 template <int QT>
-__device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int& qblock) {
+__device__ bool locate(const PrefillArgs& a, int kv_heads, bool flag, PfWork& w) {
   const int lane = __lane_id();
   if (a.batch <= 64) {  // one lane per sequence, loaded once
     int l0 = 0;
     const int n = lane < a.batch ? seq_blocks<QT>(a, lane, flag, l0) : 0;
     int lo = 0, hi = wave_reduce(n == 0 ? 0 : l0 + n, MaxInt());
-    if (rank >= wave_reduce(n, AddInt())) return false;
+    const int total = wave_reduce(n, AddInt());
+    const int rank = pf_parts(a, kv_heads, total, w);
+    if (rank >= total) return false;
     auto above = [&](int u) { return min(max(l0 + n - 1 - max(u, l0 - 1), 0), n); };
     // smallest u in [0, hi] with at most `rank` blocks above level u
     while (lo < hi) {
@@ -183,8 +210,8 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
     const int incl = wave_scan(at, AddInt()) + first;
     const uint64_t hit = __builtin_amdgcn_ballot_w64(at && incl == rank + 1);
     const int l = __builtin_ctzll(hit);
-    seq = __builtin_amdgcn_readfirstlane(l);
-    qblock = lo - __builtin_amdgcn_readfirstlane(__shfl(l0, l));
+    w.seq = __builtin_amdgcn_readfirstlane(l);
+    w.qblock = lo - __builtin_amdgcn_readfirstlane(__shfl(l0, l));
     return true;
   }
   // larger batches: sequence by sequence, in reverse
@@ -194,7 +221,7 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
     const int n = i < a.batch ? seq_blocks<QT>(a, i, flag, l0) : 0;
     total += wave_reduce(n, AddInt());
   }
-  const int target = total - 1 - rank;
+  const int target = total - 1 - pf_parts(a, kv_heads, total, w);
   if (target < 0) return false;
   int before = 0;
   for (int base = 0; base < a.batch; base += 64) {
@@ -204,8 +231,8 @@ __device__ bool locate(const PrefillArgs& a, int rank, bool flag, int& seq, int&
     const uint64_t hit = __builtin_amdgcn_ballot_w64(i < a.batch && target < incl && target >= incl - n);
     if (hit != 0) {
       const int l = __builtin_ctzll(hit);
-      seq = __builtin_amdgcn_readfirstlane(base + l);
-      qblock = __builtin_amdgcn_readfirstlane(target - (__shfl(incl, l) - __shfl(n, l)));
+      w.seq = __builtin_amdgcn_readfirstlane(base + l);
+      w.qblock = __builtin_amdgcn_readfirstlane(target - (__shfl(incl, l) - __shfl(n, l)));
       return true;
     }
     before = __shfl(incl, 63);
@@ -295,17 +322,18 @@ paged_prefill_kernel(const PrefillArgs a) {
   constexpr int kStage = 2 * kPayload + 2 * kPfKT * 4;
   __shared__ __attribute__((aligned(256))) uint8_t stages[4 * kStage];
 
-  // workgroup -> (block rank, split, kv head): heads fastest, so that the
-  // long blocks of all heads start first and, with 8 kv heads, each XCD reads
-  // one head's K/V
-  const int kv_heads = a.num_heads / G;
-  const int per_block = kv_heads * a.splits;
-  const int rank = uniform_int(static_cast<int>(blockIdx.x) / per_block);
-  const int rest = static_cast<int>(blockIdx.x) - rank * per_block;
-  const int split = uniform_int(rest / kv_heads);
-  const int h = rest - split * kv_heads;
-  int seq, qblock;
-  if (!locate<QT>(a, rank, blockIdx.x == 0 && threadIdx.x < 64, seq, qblock)) return;
+  PfWork work;
+  const bool found = locate<QT>(a, a.num_heads / G, blockIdx.x == 0 && threadIdx.x < 64, work);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (a.splits > 1) *a.used = work.splits;
+    if (a.report != nullptr) {
+      a.report[1] = a.cu_q[0];
+      a.report[2] = a.cu_q[a.batch];
+    }
+  }
+  if (!found) return;
+  const int seq = uniform_int(work.seq), qblock = uniform_int(work.qblock), h = uniform_int(work.head);
+  const int split = uniform_int(work.split), splits = uniform_int(work.splits);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);  // uniform: SGPR arithmetic below
   const int lane = tid % 64;
@@ -324,8 +352,8 @@ paged_prefill_kernel(const PrefillArgs a) {
   const int qlast = qpos0 + (qb0 < qlen ? kPfCols : 0) - 1;  // no key past it is visible to the wave
   const int all_tiles = (kend + kPfKT - 1) / kPfKT;
   // this workgroup's tiles
-  const int t0 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * split / a.splits));
-  const int t1 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * (split + 1) / a.splits));
+  const int t0 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * split / splits));
+  const int t1 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * (split + 1) / splits));
   const int32_t* bt_row = a.bt + static_cast<int64_t>(seq) * a.bt_sb;
 
   // the query's loads, then the first tiles', then the query's conversion
@@ -435,11 +463,17 @@ paged_prefill_kernel(const PrefillArgs a) {
           for (int y = 1; y < kGroups; ++y)
             if (lane / 16 == y) b = blk[y], pr = row0[y] - 16 * y;
         }
-        const float* src = s_head + b * s_sn + pr * s_sp + lane * s_sp;
         const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_addr(st) + 2 * kPayload + wave * kPfKT * 4);
-        if (WHOLE || b >= 0)
-          asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds)
-                       : "memory", "m0");
+        if constexpr (WHOLE) {
+          const uint8_t* base = uniform_ptr(reinterpret_cast<const uint8_t*>(s_head + b * s_sn + pr * s_sp));
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                       : : "v"(static_cast<uint32_t>(lane * s_sp * 4)), "s"(base), "s"(lds) : "memory", "m0");
+        } else {
+          const float* src = s_head + b * s_sn + pr * s_sp + lane * s_sp;
+          if (b >= 0)
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds)
+                         : "memory", "m0");
+        }
       } else {
         reinterpret_cast<float*>(st + 2 * kPayload)[wave * kPfKT + lane] = 1.f;
       }
@@ -581,7 +615,7 @@ paged_prefill_kernel(const PrefillArgs a) {
           ksv[(x + 1) % 2] = *reinterpret_cast<const floatx4*>(scl + 32 * ((x + 1) / 4) + 8 * ((x + 1) % 4));
           vsv[(x + 1) % 2] = *reinterpret_cast<const floatx4*>(scl + kPfKT + 32 * ((x + 1) / 4) + 8 * ((x + 1) % 4));
         }
-        if (x == 2) read_k(nxt, 1, kw[1]);
+        if (x == 3) read_k(nxt, 1, kw[1]);  // (into the registers that chain 0 is done with)
         if (x == 6) read_v(0, vt[0]);
         float p[4];
 #pragma unroll
@@ -691,7 +725,7 @@ paged_prefill_kernel(const PrefillArgs a) {
   const float l_tot = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
   if (!colv) return;
   const int64_t tok = qs + qb0 + c;
-  if (a.splits > 1) {
+  if (splits > 1) {
     const int64_t cell = (static_cast<int64_t>(split) * a.total_q + tok) * a.num_heads + qhead;
     float* dst = a.part + cell * kPfD + 4 * g;
 #pragma unroll
@@ -746,11 +780,13 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   const int64_t cells = static_cast<int64_t>(a.total_q) * a.num_heads;
   if (cell >= cells) return;
   const int lane = threadIdx.x % 64;
+  const int splits = *a.used;
+  if (splits == 1) return;  // the outputs are written
   const int tok = static_cast<int>(cell / a.num_heads);
   if (tok < a.cu_q[0] || tok >= a.cu_q[a.batch]) return;
   // lane s holds split s's weight (at most 64 splits)
   const floatx2* ml = reinterpret_cast<const floatx2*>(a.part + a.splits * cells * kPfD) + cell;
-  const floatx2 mine = lane < a.splits ? ml[lane * cells] : floatx2{-INFINITY, 0.f};
+  const floatx2 mine = lane < splits ? ml[lane * cells] : floatx2{-INFINITY, 0.f};
   float m = mine[1] > 0.f ? mine[0] : -INFINITY;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
@@ -758,7 +794,7 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   const floatx2* row = reinterpret_cast<const floatx2*>(a.part) + cell * (kPfD / 2) + lane;
   float l = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll 4
-  for (int s = 0; s < a.splits; ++s) {
+  for (int s = 0; s < splits; ++s) {
     const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s));
     const floatx2 v = row[s * cells * (kPfD / 2)];
     l = fmaf(w, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine[1]), s)), l);
@@ -772,39 +808,34 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   dst[1] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o1 * inv) : f32_to_bf16_bits(o1 * inv);
 }
 
-// What a caller reads back: the status word and the packed rows' extent, in
-// (pinned) memory that the host sees once the stream is done.
-__global__ void paged_prefill_report_kernel(const int32_t* status, const int32_t* cu_q, int batch, int32_t* out) {
-  if (threadIdx.x == 0) {
-    out[0] = status[0];
-    out[1] = cu_q[0];
-    out[2] = cu_q[batch];
-  }
-}
-
 // Query blocks that the launch provides for: every sequence may end in a
 // partial block.
 int64_t block_bound(int total_q, int batch, int groups) { return ceil_div(total_q, pf_qtile(groups)) + batch; }
 
-// Workgroups per (block, kv head).  The kernel fits eight waves on a CU; where the blocks give fewer than that, the keys are split so
-// that the launch fills the chip once, in parts of at least 4 tiles of the
-// longest context the tables can hold.
-// (a sequence's last block is partial, so it adds half a block on average.)
-int split_count(int total_q, int batch, int num_heads, int num_kv_heads, int64_t capacity) {
+// Workgroups that the chip holds at once: the kernel fits eight waves on a CU.
+int64_t chip_slots(int groups) { return static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(groups); }
+
+// Most workgroups per (block, kv head), for the fewest blocks that total_q rows
+// make: where the blocks leave slots free, the keys are split, in parts of at
+// least 4 tiles of the longest context the tables can hold.  The kernel, which
+// sees the real number of blocks, takes as many as the slots allow.
+int split_count(int total_q, int num_heads, int num_kv_heads, int64_t capacity) {
   const int groups = num_heads / num_kv_heads;
-  const int64_t wgs = (ceil_div(total_q, pf_qtile(groups)) + batch / 2) * num_kv_heads;
-  const int64_t slots = static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(groups);
-  const int64_t s = std::min(slots / wgs, capacity / (4 * kPfKT));
+  const int64_t wgs = ceil_div(total_q, pf_qtile(groups)) * num_kv_heads;
+  const int64_t s = std::min(chip_slots(groups) / wgs, capacity / (4 * kPfKT));
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(s, 64)));
 }
 
+constexpr int64_t kPfPartOffset = 256;  // the partials follow the count of splits
+
 int64_t split_workspace(int splits, int total_q, int num_heads) {
-  return splits > 1 ? static_cast<int64_t>(splits) * total_q * num_heads * (kPfD + 2) * 4 : 0;
+  return splits > 1 ? kPfPartOffset + static_cast<int64_t>(splits) * total_q * num_heads * (kPfD + 2) * 4 : 0;
 }
 
 template <int QDT, int G>
 int launch_prefill(const PrefillArgs& a, bool scaled, hipStream_t stream) {
-  const int64_t blocks = block_bound(a.total_q, a.batch, G) * (a.num_heads / G) * a.splits;
+  int64_t blocks = block_bound(a.total_q, a.batch, G) * (a.num_heads / G);
+  if (a.splits > 1) blocks = std::max<int64_t>(blocks, a.slots);  // split blocks never take more than the slots
   if (blocks > INT32_MAX) {
     set_error("prism_paged_prefill: too many query blocks for one launch");
     return PRISM_ERR_INVALID;
@@ -853,7 +884,7 @@ extern "C" int64_t prism_paged_prefill_workspace_bytes(int batch, int total_q, i
       num_heads / num_kv_heads > kPfMaxWaves || page_size <= 0 || width < 0)
     return 0;
   const int64_t capacity = static_cast<int64_t>(width) * page_size;
-  return split_workspace(split_count(total_q, batch, num_heads, num_kv_heads, capacity), total_q, num_heads);
+  return split_workspace(split_count(total_q, num_heads, num_kv_heads, capacity), total_q, num_heads);
 }
 
 extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,
@@ -864,7 +895,8 @@ extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t 
                                       const int32_t* context_lens, const int32_t* cu_seqlens_q, void* out,
                                       const int64_t out_strides[3], int batch, int total_q, int num_heads,
                                       int num_kv_heads, int head_dim, int page_size, int num_blocks, int width,
-                                      float scale, int32_t* status, void* workspace, int64_t workspace_bytes, void* stream_ptr){
+                                      float scale, int32_t* status, void* workspace, int64_t workspace_bytes, int32_t* report,
+                                      void* stream_ptr) {
   using namespace prism;
   clear_error();
   if (batch < 0 || total_q < 0 || num_heads <= 0 || num_kv_heads <= 0 || page_size <= 0 || num_blocks < 0 ||
@@ -947,31 +979,21 @@ extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t 
   a.width = width;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.status = status;
+  a.report = report;
   a.out_vec = aligned(out, 8) && out_strides[0] % 4 == 0 && out_strides[1] % 4 == 0;
   a.total_q = total_q;
-  a.splits = split_count(total_q, batch, num_heads, num_kv_heads, static_cast<int64_t>(width) * page_size);
+  a.slots = static_cast<int>(chip_slots(num_heads / num_kv_heads));
+  a.splits = split_count(total_q, num_heads, num_kv_heads, static_cast<int64_t>(width) * page_size);
   // without scratch for the partials the keys are not split
   if (a.splits > 1 &&
       (workspace == nullptr || !aligned(workspace, 16) || workspace_bytes < split_workspace(a.splits, total_q, num_heads)))
     a.splits = 1;
-  a.part = static_cast<float*>(workspace);
+  a.used = static_cast<int*>(workspace);
+  a.part = a.splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kPfPartOffset) : nullptr;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   const bool scaled = k_scale != nullptr;
   if (q_dtype == PRISM_DTYPE_F16) return dispatch_groups<PRISM_DTYPE_F16>(a, scaled, stream);
   return dispatch_groups<PRISM_DTYPE_BF16>(a, scaled, stream);
-}
-
-extern "C" int prism_paged_prefill_report(const int32_t* status, const int32_t* cu_seqlens_q, int batch, int32_t* out,
-                                          void* stream_ptr) {
-  using namespace prism;
-  clear_error();
-  if (!status || !cu_seqlens_q || !out || batch < 0) {
-    set_error("prism_paged_prefill_report: invalid argument");
-    return PRISM_ERR_INVALID;
-  }
-  hipLaunchKernelGGL(paged_prefill_report_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream_ptr), status,
-                     cu_seqlens_q, batch, out);
-  return check_launch("paged_prefill_report_kernel launch");
 }
 
 extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,
@@ -986,5 +1008,5 @@ extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_s
   return prism_paged_prefill_ws(q, q_dtype, q_strides, k_cache, v_cache, cache_dtype, k_strides, v_strides, k_scale,
                                 v_scale, k_scale_strides, v_scale_strides, block_tables, bt_strides, context_lens,
                                 cu_seqlens_q, out, out_strides, batch, total_q, num_heads, num_kv_heads, head_dim,
-                                page_size, num_blocks, width, scale, status, nullptr, 0, stream_ptr);
+                                page_size, num_blocks, width, scale, status, nullptr, 0, nullptr, stream_ptr);
 }

@@ -292,26 +292,24 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor ws;
   if (need > 0) ws = at::empty({need}, q->options().dtype(at::kByte));
   const Strides sq(q), sk(kc), sv(vc), sks(ks), svs(vs), sbt(bt), so(&out);
-  int rc = prism_paged_prefill_ws(
-      q->data_ptr(), qd, sq.v, kc->data_ptr(), vc->data_ptr(), PRISM_DTYPE_FP8_E4M3FN, sk.v, sv.v,
-      ks ? static_cast<const float*>(ks->data_ptr()) : nullptr, vs ? static_cast<const float*>(vs->data_ptr()) : nullptr,
+  int32_t* words = static_cast<int32_t*>(report->data_ptr());
+  words[0] = 0;  // (the thread's previous call on this stream has been waited for)
+  const int rc = prism_paged_prefill_ws(
+      q->data_ptr(), qd, sq.v, kc->data_ptr(), vc->data_ptr(), PRISM_DTYPE_FP8_E4M3FN, sk.v, sv.v, scales(ks), scales(vs),
       sks.v, svs.v, static_cast<const int32_t*>(bt->data_ptr()), sbt.v, static_cast<const int32_t*>(ctx->data_ptr()),
       static_cast<const int32_t*>(cu->data_ptr()), out.data_ptr(), so.v, static_cast<int>(batch), static_cast<int>(total),
       static_cast<int>(heads), static_cast<int>(kv_heads), static_cast<int>(dim), page, static_cast<int>(kc->size(0)),
       width, static_cast<float>(scale), static_cast<int32_t*>(status->data_ptr()), need > 0 ? ws.data_ptr() : nullptr,
-      need, stream);
-  if (rc == PRISM_OK)
-    rc = prism_paged_prefill_report(static_cast<const int32_t*>(status->data_ptr()),
-                                    static_cast<const int32_t*>(cu->data_ptr()), static_cast<int>(batch),
-                                    static_cast<int32_t*>(report->data_ptr()), stream);
+      need, words, stream);
   if (rc != PRISM_OK) Py_RETURN_NONE;
   hipError_t err;
   Py_BEGIN_ALLOW_THREADS
   err = hipStreamSynchronize(static_cast<hipStream_t>(stream));
   Py_END_ALLOW_THREADS
   C10_HIP_CHECK(err);
-  const volatile int32_t* r = static_cast<const int32_t*>(report->data_ptr());
-  const int bad = r[0], row0 = r[1], row1 = r[2];
+  const volatile int32_t* r = words;
+  const int row0 = r[1], row1 = r[2];
+  const int bad = r[0] == 0 ? INT32_MAX : status->item<int32_t>();
   PyObject* wrapped = THPVariable_Wrap(std::move(out));
   if (wrapped == nullptr) return nullptr;
   return Py_BuildValue("(Niii)", wrapped, bad, row0, row1);

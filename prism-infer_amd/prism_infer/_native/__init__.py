@@ -86,9 +86,8 @@ SIGNATURES: dict[str, tuple] = {
     "prism_paged_prefill_ws": (
         _I,
         [_VP, _I, _I64P, _VP, _VP, _I, _I64P, _I64P, _VP, _VP, _I64P, _I64P, _VP, _I64P, _VP, _VP, _VP,
-         _I64P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _VP, _VP, _I64, _VP],
+         _I64P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _VP, _VP, _I64, _VP, _VP],
     ),
-    "prism_paged_prefill_report": (_I, [_VP, _VP, _I, _VP, _VP]),
     "prism_debug_fp8_encode": (_I, [_VP, _VP, _I64, _VP]),
 }
 

@@ -46,7 +46,7 @@ PREFILL_HEAD_DIM = 128
 _STATUS_OK = 2**31 - 1
 
 # Per thread and (device, stream): the status word, which holds _STATUS_OK
-# between calls, and the pinned words a call's outcome is read from.  A call
+# between calls, and the pinned words that a call's outcome is read from.  A call
 # waits for its stream before it returns, so a thread's next call finds them
 # free; other threads have their own.
 _OUTCOME = threading.local()
@@ -197,7 +197,7 @@ def _launch_paged_prefill(q, k_cache, v_cache, context, *, num_heads, num_kv_hea
             out.data_ptr(), _native.strides(out),
             batch, q.shape[0], num_heads, num_kv_heads, q.shape[2], k_cache.shape[1], k_cache.shape[0],
             block_tables.shape[1], float(scale), status.data_ptr(),
-            workspace.data_ptr() if workspace is not None else None, ws_bytes, _native.stream_handle(device),
+            workspace.data_ptr() if workspace is not None else None, ws_bytes, None, _native.stream_handle(device),
         )
     _native.check(rc, "paged_prefill_attention")
     return out, status, (context_lens, cu_seqlens_q, block_tables), batch

@@ -41,7 +41,7 @@ def _run(c, split):
             t["k"].shape[0], width, 128 ** -0.5, status.data_ptr()]
     stream = _native.stream_handle(dev)
     if split:
-        rc = lib.prism_paged_prefill_ws(*args, ws.data_ptr(), need, stream)
+        rc = lib.prism_paged_prefill_ws(*args, ws.data_ptr(), need, None, stream)
     else:
         rc = lib.prism_paged_prefill(*args, stream)
     _native.check(rc, "prefill")
