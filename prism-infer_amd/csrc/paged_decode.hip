@@ -343,27 +343,6 @@ struct QOperand<PRISM_DTYPE_F16> {
   f16x8 hi[4];
 };
 
-// Query operand of the streaming kernel for the fp8 MFMA (16x16x128): lane
-// (g, c) holds column c's dims 32g..32g+31 as fp8 bytes, the same bytes of
-// the K rows it multiplies.  Each column is scaled by 2^e so that its
-// largest |q| lies in [128, 256), then split into three E4M3FN terms,
-// hi + mid + lo, each the round-to-nearest of what the previous terms left
-// (four significant bits per term).  A bf16 query (eight bits) is held
-// exactly by hi + mid for elements of 2^-2 and up after scaling (2^-10 of
-// the column's largest) and within 2^-10 below (2^-18 of the largest); its
-// lo term is then zero, so the kernel skips that MFMA for bf16 queries.  An
-// f16 query is held exactly from 2 up and within 2^-10 below, an f32 query
-// to about 2^-12 relative.  The score is then (K . (hi + mid + lo)) * 2^-e,
-// and 2^-e is folded into the per-column score multiplier.
-struct QOperandF8 {
-  i32x8 t[3];      // hi, mid, lo
-  float colscale;  // scale_log2 * 2^-e of this lane's column
-};
-
-template <int QDT, bool QVEC>
-__device__ __forceinline__ void stream_load_q8(const DecodeArgs& a, int qrow, int qhead, bool qvalid, int g,
-                                               QOperandF8& qop);
-
 // Partials cross workgroups (and XCDs, whose L2 caches are not coherent with
 // each other) inside one launch.  They are written with device-scope stores
 // (sc1: written through to the device-coherent level) and read back with
@@ -388,7 +367,6 @@ __device__ __forceinline__ float2 load_coherent2(__amdgpu_buffer_rsrc_t r, uint3
 }
 
 constexpr int kSplitWaves = 8;       // waves per split-K workgroup (tile lanes of one kv head)
-constexpr float kSplitRescaleThreshold = 8.0f;  // log2 units
 constexpr int kSplitMaxChunks = 64;  // chunks per (sequence, kv head) at most
 
 // Chunk counters of the split-K path, one 64-bit word per (sequence, kv
@@ -544,13 +522,8 @@ paged_decode_split_kernel(const DecodeArgs a) {
 
     // ---- query operand (B of QK): column c = q head h*G + c, k slot 8g+e of
     // chunk cc <-> dim 32g + 8cc + e.
-    // FP8 caches under bf16 queries: the fp8 MFMA's operand (two terms, exact
-    // for bf16) against the K bytes as they are, without converting K.
-    constexpr bool kF8 = CB == 1 && QDT == PRISM_DTYPE_BF16;
-    typename std::conditional<kF8, QOperandF8, QOperand<QDT>>::type qop;
-    if constexpr (kF8) {
-      stream_load_q8<QDT, QVEC>(a, b, h * G + (c < G ? c : 0), c < G, g, qop);
-    } else {
+    QOperand<QDT> qop;
+    {
       // Lanes c >= G read q head h*G (a valid row) and zero their copy, so the
       // loads carry no branch.
       const bool qvalid = c < G;
@@ -664,15 +637,6 @@ paged_decode_split_kernel(const DecodeArgs a) {
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         floatx4 accs = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (kF8) {
-          const i32x8 ka = {static_cast<int>(cur.k[hh][0][0]), static_cast<int>(cur.k[hh][0][1]),
-                            static_cast<int>(cur.k[hh][0][2]), static_cast<int>(cur.k[hh][0][3]),
-                            static_cast<int>(cur.k[hh][1][0]), static_cast<int>(cur.k[hh][1][1]),
-                            static_cast<int>(cur.k[hh][1][2]), static_cast<int>(cur.k[hh][1][3])};
-          accs = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ka, qop.t[1], accs, 0, 0, 0, 0, 0, 0);
-          sc[hh] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ka, qop.t[0], accs, 0, 0, 0, 0, 0, 0);
-          continue;
-        } else
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
           if constexpr (CB == 2) {  // the cache rows are already MFMA operands
@@ -713,60 +677,33 @@ paged_decode_split_kernel(const DecodeArgs a) {
       }
 
       // ---- online softmax (log2 domain).  Value e of this lane: half e/4, row e%4.
-      // Only tiles with unattended tokens (the chunk's last, an absent page)
-      // mask them (uniform branch).  Columns without a query hold q = 0: their
-      // scores are finite and their rows are never written.
-      const bool whole = __builtin_amdgcn_ballot_w64(cur.kvalid != 0xFFu) == 0;
-      float mul = a.scale_log2;
-      if constexpr (kF8) mul = qop.colscale;
       float x[8];
+      float tmax = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = sc[e >> 2][e & 3] * (ksc[e] * mul);
-      if (!whole) {
-        // (V bytes of rows past the end may be NaN codes, which the PV MFMA
-        // would not multiply away, and their scales anything.  Done here, at
-        // use, so the prefetch of this tile stays asynchronous.)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bool ok = (cur.kvalid >> e) & 1u;
-          x[e] = ok ? x[e] : -INFINITY;
-          vsc[e] = ok ? vsc[e] : 0.f;
-          if constexpr (CB == 1) cur.v[e] = ok ? cur.v[e] : u32x2{0, 0};
-          else cur.v[e] = ok ? cur.v[e] : u32x4{0, 0, 0, 0};
-        }
+      for (int e = 0; e < 8; ++e) {
+        const bool ok = ((cur.kvalid >> e) & 1u) && c < G;
+        const float v = sc[e >> 2][e & 3] * (ksc[e] * a.scale_log2);
+        x[e] = ok ? v : -INFINITY;
+        tmax = fmaxf(tmax, x[e]);
       }
-      float tmax = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-      tmax = wave_max_across_groups(tmax);
-      // Lazy rescaling: the running max moves only when a score exceeds it by
-      // more than 2^8, so the accumulators (rows: q heads 4g + i) are seldom
-      // multiplied.
-      const bool raise = tmax > m_run + kSplitRescaleThreshold;
-      if (__builtin_amdgcn_ballot_w64(raise) != 0) {
-        const float m_new = raise ? tmax : m_run;
-        const float alpha = raise ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
-        m_run = m_new;
-        l_run *= alpha;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float ai = __shfl(alpha, 4 * g + i);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[j][i] *= ai;
-        }
-      }
-      const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+      const float m_new = fmaxf(m_run, tmax);
+      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+      const float alpha = exp2f(m_run - m_use);
+      m_run = m_new;
       // P * v_scale as a hi/lo pair of the PV MFMA's 16-bit type (about 16
       // significant bits): the PV product then matches fp32 accumulation
       // closely (V itself is exact).  bf16 for FP8 and bf16 caches, f16 for
-      // an f16 cache (P <= 2^8 there: no scale).
+      // an f16 cache (P <= 1 there: no scale).
       using PvT = typename std::conditional<CB == 2 && QDT == PRISM_DTYPE_F16, f16x8, bf16x8>::type;
       float psum = 0.f;
       PvT pa, pa_lo;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        // v_exp_f32: results below 2^-126 (flushed to 0) weigh nothing next to the max
-        const float p = __builtin_amdgcn_exp2f(x[e] - m_use);  // 0 for masked slots
+        const float p = exp2f(x[e] - m_use);  // 0 for masked slots
         psum += p;
-        const float pv = p * vsc[e];
+        const float pv = ((cur.kvalid >> e) & 1u) ? p * vsc[e] : 0.f;
         if constexpr (CB == 2 && QDT == PRISM_DTYPE_F16) {
           const _Float16 hi = static_cast<_Float16>(pv);
           pa[e] = hi;
@@ -777,7 +714,27 @@ paged_decode_split_kernel(const DecodeArgs a) {
           pa_lo[e] = static_cast<__bf16>(pv - static_cast<float>(hi));
         }
       }
-      l_run += psum;
+      l_run = l_run * alpha + psum;
+
+      // Rescale accumulator rows (q heads 4g+i) by their alpha.
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float ai = __shfl(alpha, 4 * g + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j][i] *= ai;
+      }
+
+      // Rows past the end of the chunk may hold anything (NaN codes included);
+      // their V bytes are zeroed because the PV MFMA would turn 0 * NaN into
+      // NaN.  (Done here, at use, so the prefetch of this tile stays
+      // asynchronous.)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (!((cur.kvalid >> e) & 1u)) {
+          if constexpr (CB == 1) cur.v[e] = u32x2{0, 0};
+          else cur.v[e] = u32x4{0, 0, 0, 0};
+        }
+      }
 
       // ---- PV: B operand of N-tile j = element j of the lane's 8 V rows.
 #pragma unroll
@@ -1347,6 +1304,23 @@ __device__ __forceinline__ void stream_load_q(const DecodeArgs& a, int qrow, int
 }
 
 
+
+// Query operand of the streaming kernel for the fp8 MFMA (16x16x128): lane
+// (g, c) holds column c's dims 32g..32g+31 as fp8 bytes, the same bytes of
+// the K rows it multiplies.  Each column is scaled by 2^e so that its
+// largest |q| lies in [128, 256), then split into three E4M3FN terms,
+// hi + mid + lo, each the round-to-nearest of what the previous terms left
+// (four significant bits per term).  A bf16 query (eight bits) is held
+// exactly by hi + mid for elements of 2^-2 and up after scaling (2^-10 of
+// the column's largest) and within 2^-10 below (2^-18 of the largest); its
+// lo term is then zero, so the kernel skips that MFMA for bf16 queries.  An
+// f16 query is held exactly from 2 up and within 2^-10 below, an f32 query
+// to about 2^-12 relative.  The score is then (K . (hi + mid + lo)) * 2^-e,
+// and 2^-e is folded into the per-column score multiplier.
+struct QOperandF8 {
+  i32x8 t[3];      // hi, mid, lo
+  float colscale;  // scale_log2 * 2^-e of this lane's column
+};
 
 // B operand of S^T = K Q^T for 16-bit caches (bf16 / f16 MFMA 16x16x32):
 // lane (g, c) holds query column c's dims 32g + 8kb .. 32g + 8kb + 7 for MFMA
