@@ -489,7 +489,7 @@ paged_decode_split_kernel(const DecodeArgs a) {
         if (wv == kSplitWaves - 1) store_new();
       }
       // No attended token: zeros (the reference kernel's l == 0 branch).
-      for (int idx = threadIdx.x; idx < G * kHeadDim; idx += blockDim.x) {
+      for (int idx = threadIdx.x; idx < G * kHeadDim; idx += 64 * kSplitWaves) {
         const int qh = h * G + idx / kHeadDim;
         const int d = idx % kHeadDim;
         store_out<QDT>(a.out, b * a.o_sb + qh * a.o_sh + d * a.o_sd, 0.f);
@@ -837,7 +837,7 @@ paged_decode_split_kernel(const DecodeArgs a) {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   const int64_t prow0 = ((static_cast<int64_t>(b) * nkv + h) * a.max_splits + z) * G;  // first partial row
-  for (int e = threadIdx.x; e < G * kHeadDim; e += blockDim.x) {
+  for (int e = threadIdx.x; e < G * kHeadDim; e += 64 * kSplitWaves) {
     const int r = e / kHeadDim;
     const int d = e - r * kHeadDim;
     float mx = -INFINITY;
@@ -875,7 +875,7 @@ paged_decode_split_kernel(const DecodeArgs a) {
   // Thread (cg, u): unit u = float4 u of the G x 128 outputs, chunk group cg
   // takes chunks cg, cg + NG, ...; the NG groups then meet in LDS.
   const int units = G * (kHeadDim / 4);
-  const int NG = blockDim.x / units;  // 1 (G = 16) .. 16 (G = 1)
+  const int NG = 64 * kSplitWaves / units;  // 1 (G = 16) .. 16 (G = 1)
   const int cg = threadIdx.x / units;
   const int u = threadIdx.x - cg * units;
   const int r = u / (kHeadDim / 4);
