@@ -61,16 +61,9 @@ def _torch_lib_dir() -> Path:
     return lib
 
 
-# Per-source extra flags.  The prefill kernel's max reductions run without the
-# IEEE mode's NaN quieting (no operand there is a NaN), which halves their cost.
-EXTRA_FLAGS = {
-    "paged_prefill.hip": ["-mno-amdgpu-ieee", "-fno-honor-nans"],
-}
-
-
 def _compile(src: Path, build_dir: Path = BUILD_DIR, defines: tuple = ()) -> Path:
     obj = build_dir / (src.stem + ".o")
-    cmd = [_hipcc(), *HIPCC_FLAGS, *EXTRA_FLAGS.get(src.name, []), *(f"-D{d}" for d in defines), f"-I{INCLUDE}",
+    cmd = [_hipcc(), *HIPCC_FLAGS, *(f"-D{d}" for d in defines), f"-I{INCLUDE}",
            f"-I{CSRC}", "-c", str(src), "-o", str(obj)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -587,9 +587,10 @@ paged_prefill_kernel(const PrefillArgs a) {
       //
       // P is first formed against the running max as it stands; the sum, which
       // is needed anyway, tells whether that was low enough (every p is at
-      // most the lane's sum).  Only where it was not, on the first tile and on
-      // tiles with masked keys, are the scores' maxima taken and the
-      // accumulators rescaled.
+      // most the lane's sum).  Only where it was not (or is no number: a score
+      // of -inf against a running max of -inf weighs 0, not NaN), on the first
+      // tile and on tiles with masked keys, are the scores' maxima taken and
+      // the accumulators rescaled.
       bf16x8 pa[2][2];
       float ps;
       const bool masked = key0 + kPfKT - 1 > qpos0;  // (uniform) the diagonal or the block's end is in the tile
@@ -631,7 +632,7 @@ paged_prefill_kernel(const PrefillArgs a) {
       // (the pins keep the sums and the MFMAs in front of the branch)
       asm volatile("" : "+v"(ps), "+v"(pa[0][0]), "+v"(pa[0][1]), "+v"(pa[1][0]), "+v"(pa[1][1])
                    : "v"(sn[0]), "v"(sn[1]));
-      if (first || masked || __builtin_amdgcn_ballot_w64(ps > kPfSumLimit) != 0) {
+      if (first || masked || __builtin_amdgcn_ballot_w64(!(ps <= kPfSumLimit)) != 0) {
         first = false;
         // causal mask: key k is visible to column c iff it is at or before the
         // query's position; columns without a query see none, and their rows
@@ -665,6 +666,11 @@ paged_prefill_kernel(const PrefillArgs a) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[n][r] *= alpha;
         const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+        // Weights are dropped by the key's visibility and not by p, so that a
+        // NaN stays one (compared anew: 32 lane masks kept from above would
+        // fill the SGPRs).
+        int seen = last;
+        asm("" : "+v"(seen));
         ps = 0.f;
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -675,7 +681,7 @@ paged_prefill_kernel(const PrefillArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               p[j] = __builtin_amdgcn_exp2f(sc[b][4 * i + j] - m_use);  // 0 where masked
-              pa[b][i / 2][4 * (i % 2) + j] = static_cast<__bf16>(p[j] > 0.f ? p[j] * vsv[j] : 0.f);
+              pa[b][i / 2][4 * (i % 2) + j] = static_cast<__bf16>(32 * b + 8 * i + j <= seen ? p[j] * vsv[j] : 0.f);
             }
             ps += (p[0] + p[1]) + (p[2] + p[3]);
           }
@@ -738,7 +744,7 @@ paged_prefill_kernel(const PrefillArgs a) {
     if (g == 0) *reinterpret_cast<floatx2*>(ml) = floatx2{m_run, l_tot};
     return;
   }
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  const float inv = l_tot == 0.f ? 0.f : 1.f / l_tot;  // (a NaN sum makes the row NaN)
   uint16_t* dst = static_cast<uint16_t*>(a.out) + tok * a.o_st + static_cast<int64_t>(qhead) * a.o_sh + 4 * g;
 #pragma unroll
   for (int n = 0; n < 4; ++n)
@@ -787,10 +793,13 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   // lane s holds split s's weight (at most 64 splits)
   const floatx2* ml = reinterpret_cast<const floatx2*>(a.part + a.splits * cells * kPfD) + cell;
   const floatx2 mine = lane < splits ? ml[lane * cells] : floatx2{-INFINITY, 0.f};
-  float m = mine[1] > 0.f ? mine[0] : -INFINITY;
+  // Parts without a visible key hold zeros and weigh nothing; a NaN sum goes
+  // through whatever its part's weight is.
+  const bool live = mine[1] != 0.f;
+  float m = live ? mine[0] : -INFINITY;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
-  const float weight = mine[1] > 0.f ? __builtin_amdgcn_exp2f(mine[0] - m) : 0.f;
+  const float weight = live ? __builtin_amdgcn_exp2f(mine[0] - m) : 0.f;
   const floatx2* row = reinterpret_cast<const floatx2*>(a.part) + cell * (kPfD / 2) + lane;
   float l = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll 4
@@ -798,10 +807,10 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
     const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s));
     const floatx2 v = row[s * cells * (kPfD / 2)];
     l = fmaf(w, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine[1]), s)), l);
-    o0 = w > 0.f ? fmaf(w, v[0], o0) : o0;
-    o1 = w > 0.f ? fmaf(w, v[1], o1) : o1;
+    o0 = fmaf(w, v[0], o0);
+    o1 = fmaf(w, v[1], o1);
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l == 0.f ? 0.f : 1.f / l;
   uint16_t* dst = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(tok) * a.o_st +
                   (cell - static_cast<int64_t>(tok) * a.num_heads) * a.o_sh + 2 * lane;
   dst[0] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o0 * inv) : f32_to_bf16_bits(o0 * inv);
