@@ -373,20 +373,19 @@ paged_prefill_kernel(const PrefillArgs a) {
   // V rows, K scales, V scales.  A wave's load covers 8 rows: LDS chunk x of
   // row t holds the row's global chunk x ^ swz(t).  Every load of a wave is
   // in one 16-key group and is all K or all V: a uniform 64-bit base (SGPRs)
-  // plus a 32-bit per-lane offset that does not change from tile to tile (the
-  // host checks that a page's rows of one head span less than 2 GiB).
+  // plus a 32-bit per-lane offset that does not change from tile to tile.  The
+  // base holds the row in its page and the offset the 8 rows from there, so
+  // that both fit in 32 bits (the host checks that a page's rows of one head
+  // span less than 2 GiB; a tile of several pages' rows may span more).
   // Asm so that the compiler's wait-count pass does not drain these loads
   // before each LDS read of the other stage.
-  // (the waits below are vmcnt(0), so that waves need not issue equal numbers
-  // of loads)
   // (the 8-row groups of a wave have the parity of the wave: NW is even)
   uint32_t k_off, v_off;
   const int k_sp = static_cast<int>(a.k_sp), v_sp = static_cast<int>(a.v_sp);
   {
-    const int r = 8 * wave + lane / 8;
-    const int part = (lane % 8) ^ pf_swz(r);
-    k_off = static_cast<uint32_t>(r * k_sp + part * 16);
-    v_off = static_cast<uint32_t>(r * v_sp + part * 16);
+    const int part = (lane % 8) ^ pf_swz(8 * wave + lane / 8);
+    k_off = static_cast<uint32_t>(lane / 8 * k_sp + part * 16);
+    v_off = static_cast<uint32_t>(lane / 8 * v_sp + part * 16);
   }
   const uint8_t* k_head = a.k + h * a.k_sh;
   const uint8_t* v_head = a.v + h * a.v_sh;
@@ -443,12 +442,13 @@ paged_prefill_kernel(const PrefillArgs a) {
     for (int l = 0; l < kLoads; ++l) {
       const bool isv = l >= kLoads / 2;
       const int tr = (isv ? l - kLoads / 2 : l) * NW * 8;  // the waves' first row in the tile
-      int b = blk[0], pr = row0[0] + tr;
+      const int wr = tr + wave * 8;                        // this wave's first row
+      int b = blk[0], pr = row0[0] + wr;                   // its block and row in the page
       if constexpr (!WHOLE) {
-        const int x = (tr + wave * 8) / 16;
+        const int x = wr / 16;
 #pragma unroll
         for (int y = 1; y < kGroups; ++y)
-          if (x == y) b = blk[y], pr = row0[y] + tr - 16 * y;
+          if (x == y) b = blk[y], pr = row0[y] + wr - 16 * y;
         if (b < 0) continue;
       }
       const uint8_t* base = isv ? v_head + b * a.v_sn + pr * v_sp : k_head + b * a.k_sn + pr * k_sp;
@@ -469,7 +469,7 @@ paged_prefill_kernel(const PrefillArgs a) {
           asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                        : : "v"(static_cast<uint32_t>(lane * s_sp * 4)), "s"(base), "s"(lds) : "memory", "m0");
         } else {
-          const float* src = s_head + b * s_sn + pr * s_sp + lane * s_sp;
+          const float* src = s_head + b * s_sn + (pr + lane) * s_sp;
           if (b >= 0)
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds)
                          : "memory", "m0");
