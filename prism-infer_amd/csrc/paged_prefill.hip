@@ -349,7 +349,7 @@ paged_prefill_kernel(const PrefillArgs a) {
   const int kend = prefix + min((qblock + 1) * QT, qlen);  // keys [0, kend) are needed
   const int qb0 = qblock * QT + wave / G * kPfCols;        // first query token of the wave
   const int qpos0 = prefix + qb0;                          // its position: query column 0
-  const int qlast = qpos0 + (qb0 < qlen ? kPfCols : 0) - 1;  // no key past it is visible to the wave
+  const int qlast = qb0 < qlen ? qpos0 + kPfCols - 1 : -1; // no key past it is visible to the wave (no query: none at all)
   const int all_tiles = (kend + kPfKT - 1) / kPfKT;
   // this workgroup's tiles
   const int t0 = uniform_int(static_cast<int>(static_cast<int64_t>(all_tiles) * split / splits));
@@ -498,7 +498,10 @@ paged_prefill_kernel(const PrefillArgs a) {
   for (int n = 0; n < 4; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  // Columns without a query (all scores 0) start at 0: from -inf, which no key
+  // of theirs would ever raise, every tile of the wave would count as rising
+  // (8 query heads per kv head, 1000 tokens behind 8000: 468 against 271 us).
+  float m_run = colv ? -INFINITY : 0.f, l_run = 0.f;
 
   // per-lane LDS offsets inside a stage, for keys 0..31 (32 rows further for
   // the rest); the lane's other chunks differ by an exclusive or
