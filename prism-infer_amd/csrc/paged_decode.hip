@@ -455,15 +455,21 @@ paged_decode_split_kernel(const DecodeArgs a) {
     if (t0 < a.width * a.page_size) blk0 = ld_meta(a.bt + static_cast<int64_t>(b) * a.bt_sb + (t0 / a.page_size) * a.bt_sn);
   }
   // The sequence's new rows (every wave: the tile that holds their slot may be
-  // any wave's) and lane i's slot of sequence i.
+  // any wave's) and lane i's slot of sequence i.  16-bit tiles leave no
+  // registers to hold the rows over the walk: they are read where they are
+  // used (held, 8 registers spilled: 4 sequences of 4000 tokens, 8 layers 220
+  // us, 204 in two launches, 201 like this).
+  constexpr bool kHoldOwn = CB == 1;
   u32x4 own_k = {0, 0, 0, 0}, own_v = {0, 0, 0, 0};
   int slot_l = -1;
   auto new_row = [&](const uint16_t* rows, int64_t stride, int i) {
     return *reinterpret_cast<const u32x4*>(rows + i * stride + h * kHeadDim + 8 * c);
   };
   if constexpr (STORE) {
-    own_k = new_row(a.new_k, a.new_k_st, b);
-    own_v = new_row(a.new_v, a.new_v_st, b);
+    if constexpr (kHoldOwn) {
+      own_k = new_row(a.new_k, a.new_k_st, b);
+      own_v = new_row(a.new_v, a.new_v_st, b);
+    }
     if (lane < a.batch) slot_l = a.slots[lane];
   }
   // Chunk 0's last wave writes them: lane group 0 K, group 1 V.
@@ -471,7 +477,8 @@ paged_decode_split_kernel(const DecodeArgs a) {
     const int slot = __builtin_amdgcn_readlane(slot_l, b);
     if (slot < 0 || slot >= a.num_slots || g > 1) return;
     const int64_t row = static_cast<int64_t>(slot) * nkv + h;
-    const u32x4 raw = g == 0 ? own_k : own_v;
+    const u32x4 raw = kHoldOwn ? (g == 0 ? own_k : own_v)
+                               : (g == 0 ? new_row(a.new_k, a.new_k_st, b) : new_row(a.new_v, a.new_v_st, b));
     uint8_t* cache = const_cast<uint8_t*>(g == 0 ? a.k : a.v);
     if constexpr (CB == 2) {
       reinterpret_cast<u32x4*>(cache)[row * (kHeadDim / 8) + c] = raw;
@@ -578,24 +585,27 @@ paged_decode_split_kernel(const DecodeArgs a) {
         const int i = __builtin_ctzll(hit);
         hit &= hit - 1;
         const int t = __builtin_amdgcn_readlane(slot_l, i) - cur.base;  // token of the tile
-        const u32x4 kr = i == b ? own_k : new_row(a.new_k, a.new_k_st, i);
-        const u32x4 vr = i == b ? own_v : new_row(a.new_v, a.new_v_st, i);
         const bool k_lane = c == (t & 15);       // holds K row t in half t / 16
         const bool v_group = g == (t & 15) / 4;  // holds V row t in slot 4 (t / 16) + t % 4
         const int ve = (t >> 4) * 4 + (t & 3);
         if constexpr (CB == 2) {
+          // straight from memory into the tile's registers, by the lanes that hold the row
+          const u32x4* kr = reinterpret_cast<const u32x4*>(a.new_k + i * a.new_k_st + h * kHeadDim + 32 * g);
+          if (k_lane && t < 16) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < 4; ++q) cur.k[0][q] = kr[q];
+          }
+          if (k_lane && t >= 16) {
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-              const uint32_t w = __shfl(kr[d], 16 * g + 4 * g + q);
-              if (k_lane && t < 16) cur.k[0][q][d] = w;
-              if (k_lane && t >= 16) cur.k[1][q][d] = w;
-            }
+            for (int q = 0; q < 4; ++q) cur.k[1][q] = kr[q];
+          }
+          const u32x4 vr = new_row(a.new_v, a.new_v_st, i);
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             if (v_group && e == ve) cur.v[e] = vr;
         } else {
+          const u32x4 kr = i == b ? own_k : new_row(a.new_k, a.new_k_st, i);
+          const u32x4 vr = i == b ? own_v : new_row(a.new_v, a.new_v_st, i);
           constexpr int kIn = QDT == PRISM_DTYPE_F32 ? PRISM_DTYPE_BF16 : QDT;
           float x[8], ks, vs;
           InVec8<kIn>::load(&kr, x);
