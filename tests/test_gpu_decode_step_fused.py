@@ -4,10 +4,14 @@ Forms: scaled FP8 and 16-bit caches, bf16 and f16, GQA groups 1 to 16, pages of 
 64 slots a wave holds and above (two launches); contexts that end on a tile's first and last row, one-token and empty
 ones; slots that are skipped (-1, past the cache), that lie in another sequence's pages (which must then see the new
 row, as after a store) and in nobody's.  Old bytes under the new rows are NaN codes, so a row taken from memory too
-early cannot pass unnoticed.
+early cannot pass unnoticed.  The split-K family is forced, the native call must take the step, and a captured step
+must be the number of launches that is meant, so that no case passes without the kernel that it is for.
 """
 
 from __future__ import annotations
+
+import ctypes
+from pathlib import Path
 
 import pytest
 import torch
@@ -19,11 +23,41 @@ pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
 
 
+def _launches(fn) -> int:
+    """Nodes of the graph that `fn` captures."""
+
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        fn()
+    count = ctypes.c_size_t()
+    hip = ctypes.CDLL(str(Path(torch.__file__).parent / "lib" / "libamdhip64.so"))
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+class _MustTake:
+    """The native ops, where every call has to be taken."""
+
+    def __init__(self, host):
+        self._host = host
+
+    def __getattr__(self, name):
+        def call(*args):
+            out = getattr(self._host, name)(*args)
+            assert out is not None, f"{name} was left to Python"
+            return out
+        return call
+
+
 def _check(batch, hkv, groups, page, width, dtype, scaled, lens, odd_slots=False, view=False):
+    from prism_infer import _native
+    from prism_infer.engine import decode_attention
     from prism_infer.engine.decode_attention import PagedKVDecodeAttention, pack_decode_metadata
     from prism_infer.ops import paged_decode
     from prism_infer.ops.kv_cache_store import store_kvcache
 
+    paged_decode.set_decode_overrides(path="split")  # (restored behind every test)
+    assert decode_attention._HOST is not None, "the native host path is not built"
     g = torch.Generator().manual_seed(batch * 131 + hkv * 7 + page + groups)
     pool = batch * width + 3
     tables = torch.randperm(pool, generator=g)[:batch * width].view(batch, width)
@@ -34,6 +68,9 @@ def _check(batch, hkv, groups, page, width, dtype, scaled, lens, odd_slots=False
         slots[1] = int(tables[2, 0]) * page + 1       # a row that sequence 2 attends
         slots[3] = pool * page + 5                    # past the cache
         slots[4] = free[0] * page                     # a page nobody reads
+        if batch > 8:
+            slots[batch - 1] = int(tables[2, 0]) * page + 2   # the last sequence's row is sequence 2's to attend,
+            slots[5] = int(tables[batch - 2, 0]) * page + 1   # and a row of the one before it is sequence 5's
     cache = FP8 if scaled else dtype
     shape = (pool, page, hkv, 128)
     k, v = ((torch.randn(shape, generator=g) * 2).to(cache) for _ in range(2))
@@ -51,12 +88,21 @@ def _check(batch, hkv, groups, page, width, dtype, scaled, lens, odd_slots=False
     meta = pack_decode_metadata(slots, lens, tables, device="cuda")
     q = q.cuda()
     results = []
+    family = _native.lib().prism_paged_decode_kernel_family(batch, hkv * groups, hkv, 128, page, width,
+                                                            _native.dtype_code(cache))
+    assert family == 1
     for fused in (False, True, True):
         caches = [x.cuda() for x in (k, v)] + ([x.cuda() for x in (ks, vs)] if scaled else [None, None])
         if fused:
             layer = PagedKVDecodeAttention(hkv * groups, hkv, 128, 0.09)
             layer.k_cache, layer.v_cache, layer.k_scale_cache, layer.v_scale_cache = caches
-            out = layer(q, new_k, new_v, meta)
+            if results[1:]:  # (the stream's workspace exists)
+                with pytest.MonkeyPatch.context() as m:
+                    m.setattr(decode_attention, "_HOST", _MustTake(decode_attention._HOST))
+                    out = layer(q, new_k, new_v, meta)
+                assert _launches(lambda: layer(q, new_k, new_v, meta)) == (1 if batch <= 64 else 2)
+            else:
+                out = layer(q, new_k, new_v, meta)
         else:
             store_kvcache(new_k, new_v, caches[0], caches[1], meta.slot_mapping, caches[2], caches[3])
             out = paged_decode.paged_decode_attention(

@@ -35,6 +35,31 @@ def python_path(monkeypatch):
     return run
 
 
+class _Recorder:
+    """The native ops, keeping whether each call was taken."""
+
+    def __init__(self, host):
+        assert host is not None, "the native host path is not built"
+        self._host, self.taken = host, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            out = getattr(self._host, name)(*args)
+            self.taken.append(out is not None)
+            return out
+        return call
+
+
+@pytest.fixture
+def native_calls(monkeypatch):
+    """Whether the native path took each call since the list was last cleared."""
+
+    recorder = _Recorder(_native.host_ops())
+    for module in MODULES:
+        monkeypatch.setattr(module, "_HOST", recorder)
+    return recorder.taken
+
+
 def test_cpu_tensors_and_odd_arguments_are_left_to_python():
     host = _native.host_ops()
     if host is None:
@@ -57,8 +82,9 @@ def _bytes(x):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("cache", ["scaled", "unit", "dense"])
-def test_store_both_paths(python_path, dtype, cache):
+def test_store_both_paths(python_path, native_calls, dtype, cache):
     require_gpu()
+    _native.device_lib(torch.device("cuda", 0))  # (the first call of a process loads the kernels from Python)
     g = torch.Generator().manual_seed(5)
     key, value = (torch.randn(33, 6, 128, generator=g).to(dtype).cuda()[:, 1:5].contiguous() for _ in range(2))
     packed = torch.randn(33, 3 * 512, generator=g).to(dtype).cuda()
@@ -73,7 +99,9 @@ def test_store_both_paths(python_path, dtype, cache):
                 vc = kc.clone()
                 scales = [torch.zeros(shape[:-1], device="cuda") for _ in range(2)] if cache == "scaled" else [None] * 2
                 call = lambda: kv_cache_store.store_kvcache(k, v, kc, vc, slots[:k.shape[0]], *scales)  # noqa: E731
+                native_calls.clear()
                 call() if native else python_path(call)
+                assert native_calls == ([k.shape[0] > 0] if native else [])
                 out.append([_bytes(x).flatten() for x in (kc, vc, *scales) if x is not None])
         for other in out[1:]:
             assert all(torch.equal(a, b) for a, b in zip(out[0], other))
@@ -93,7 +121,7 @@ def _decode_case(dtype, cache, batch=3, hkv=4, groups=2, page=32, width=4):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,cache", [(torch.bfloat16, FP8), (torch.float16, FP8), (torch.float32, FP8),
                                          (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
-def test_decode_both_paths(python_path, dtype, cache):
+def test_decode_both_paths(python_path, native_calls, dtype, cache):
     require_gpu()
     q, k, v, tables, lens, ks, vs = _decode_case(dtype, cache)
     bound = torch.tensor(60, dtype=torch.int32, device="cuda")
@@ -104,7 +132,10 @@ def test_decode_both_paths(python_path, dtype, cache):
     for qq, tt in ((q, tables), (wide, tables), (q, tables.t().contiguous().t()), (q[:2], tables)):
         for form in forms:
             call = lambda: paged_decode.paged_decode_attention(qq, k, v, tt, lens, 0.1, **form)  # noqa: E731
-            first, native, python = call(), call(), python_path(call)
+            first = call()
+            native_calls.clear()
+            native, python = call(), python_path(call)
+            assert native_calls == [True]
             assert native.stride() == python.stride() and native.dtype == python.dtype
             assert torch.equal(_bytes(native), _bytes(python)) and torch.equal(_bytes(first), _bytes(python))
     other = torch.cuda.Stream()
@@ -169,7 +200,7 @@ def test_store_keeps_its_profile_region():
 
 
 @pytest.mark.gpu
-def test_prefill_both_paths_errors_and_threads(python_path):
+def test_prefill_both_paths_errors_and_threads(python_path, native_calls):
     require_gpu()
     _, k, v, tables, _, ks, vs = _decode_case(torch.bfloat16, FP8)
     q = torch.randn(40, 8, 128, device="cuda").to(torch.bfloat16)
@@ -177,7 +208,10 @@ def test_prefill_both_paths_errors_and_threads(python_path):
                               cu_seqlens_q=torch.tensor([2, 22, 27, 37], dtype=torch.int32).cuda())
     call = lambda c=context: paged_prefill.paged_prefill_attention(  # noqa: E731
         q, k, v, c, num_heads=8, num_kv_heads=4, scale=0.1, k_scale_cache=ks, v_scale_cache=vs)
-    first, native, python = call(), call(), python_path(call)
+    first = call()
+    native_calls.clear()
+    native, python = call(), python_path(call)
+    assert native_calls == [True]
     assert native.shape == python.shape == (35, 8, 128)
     assert torch.equal(_bytes(native), _bytes(python)) and torch.equal(_bytes(first), _bytes(python))
     # a bad sequence raises its message, and the next good call is unaffected
