@@ -92,6 +92,21 @@ bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c1
 // not needed since the tensors are on the current device.
 void* current_stream(int device) { return c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream(); }
 
+// The GIL is released over allocations and launches, which may wait (for memory,
+// for room in a full queue): other Python threads run meanwhile, as they do
+// under the ctypes calls.  The arguments stay alive, their caller holds them;
+// what is found elsewhere (a stream's workspace) has to be held here.
+class WithoutGil {
+ public:
+  WithoutGil() : state_(PyEval_SaveThread()) {}
+  ~WithoutGil() { PyEval_RestoreThread(state_); }
+  WithoutGil(const WithoutGil&) = delete;
+  WithoutGil& operator=(const WithoutGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
 // mark_ready(device): prism_preload has run there.
 PyObject* mark_ready(PyObject*, PyObject* arg) {
   const long device = PyLong_AsLong(arg);
@@ -124,11 +139,15 @@ PyObject* store(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
   const int64_t kst[3] = {key->stride(0), key->stride(1), key->stride(2)};
   const int64_t vst[3] = {value->stride(0), value->stride(1), value->stride(2)};
-  const int rc = prism_kv_store(key->data_ptr(), value->data_ptr(), in, kst, vst, kc->data_ptr(), vc->data_ptr(), out,
-                                ks ? static_cast<float*>(ks->data_ptr()) : nullptr,
-                                vs ? static_cast<float*>(vs->data_ptr()) : nullptr,
-                                static_cast<const int32_t*>(slots->data_ptr()), tokens, static_cast<int>(heads),
-                                static_cast<int>(dim), kc->numel() / (heads * dim), current_stream(device));
+  int rc;
+  {
+    WithoutGil released;
+    rc = prism_kv_store(key->data_ptr(), value->data_ptr(), in, kst, vst, kc->data_ptr(), vc->data_ptr(), out,
+                        ks ? static_cast<float*>(ks->data_ptr()) : nullptr,
+                        vs ? static_cast<float*>(vs->data_ptr()) : nullptr,
+                        static_cast<const int32_t*>(slots->data_ptr()), tokens, static_cast<int>(heads),
+                        static_cast<int>(dim), kc->numel() / (heads * dim), current_stream(device));
+  }
   if (rc != PRISM_OK) Py_RETURN_NONE;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -150,7 +169,8 @@ struct DecodeCall {
   int64_t batch, heads, dim, blocks, page, kv_heads, width;
   void* stream;
   int64_t need;       // workspace bytes
-  at::Tensor ws_own;  // a captured call's workspace, from the graph's pool
+  at::Tensor ws_own;  // the workspace: the stream's, held over the launch (another thread may put a larger one in
+                      // its place), or a captured call's from the graph's pool
   void* ws;
 };
 
@@ -185,14 +205,15 @@ bool check_decode(PyObject* const* args, DecodeCall& d) {
   d.ws = nullptr;
   if (d.need > 0) {
     if (capturing()) {
+      WithoutGil released;
       d.ws_own = at::empty({d.need}, q.options().dtype(at::kByte));
-      d.ws = d.ws_own.data_ptr();
     } else {
       PyObject* found = by_stream(args[10], d.device, d.stream);
       const at::Tensor* ws = found ? tensor(found) : nullptr;
       if (ws == nullptr || ws->numel() < d.need) return false;
-      d.ws = ws->data_ptr();
+      d.ws_own = *ws;
     }
+    d.ws = d.ws_own.data_ptr();
   }
   return true;
 }
@@ -205,14 +226,19 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   DecodeCall d;
   if (n != 11 || !check_decode(args, d)) Py_RETURN_NONE;
-  at::Tensor out = at::empty_like(*d.q);
-  const Strides sq(d.q), sk(d.kc), sv(d.vc), sks(d.ks), svs(d.vs), sbt(d.bt), so(&out);
-  const int rc = prism_paged_decode(
-      d.q->data_ptr(), d.qd, sq.v, d.kc->data_ptr(), d.vc->data_ptr(), d.cd, sk.v, sv.v, scales(d.ks), scales(d.vs),
-      sks.v, svs.v, static_cast<const int32_t*>(d.bt->data_ptr()), sbt.v, static_cast<const int32_t*>(d.ctx->data_ptr()),
-      static_cast<const int32_t*>(d.max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(d.batch),
-      static_cast<int>(d.heads), static_cast<int>(d.kv_heads), static_cast<int>(d.dim), static_cast<int>(d.page),
-      d.blocks, static_cast<int>(d.width), static_cast<float>(d.scale), d.ws, d.need, d.stream);
+  at::Tensor out;
+  int rc;
+  {
+    WithoutGil released;
+    out = at::empty_like(*d.q);
+    const Strides sq(d.q), sk(d.kc), sv(d.vc), sks(d.ks), svs(d.vs), sbt(d.bt), so(&out);
+    rc = prism_paged_decode(
+        d.q->data_ptr(), d.qd, sq.v, d.kc->data_ptr(), d.vc->data_ptr(), d.cd, sk.v, sv.v, scales(d.ks), scales(d.vs),
+        sks.v, svs.v, static_cast<const int32_t*>(d.bt->data_ptr()), sbt.v, static_cast<const int32_t*>(d.ctx->data_ptr()),
+        static_cast<const int32_t*>(d.max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(d.batch),
+        static_cast<int>(d.heads), static_cast<int>(d.kv_heads), static_cast<int>(d.dim), static_cast<int>(d.page),
+        d.blocks, static_cast<int>(d.width), static_cast<float>(d.scale), d.ws, d.need, d.stream);
+  }
   if (rc != PRISM_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -234,16 +260,21 @@ PyObject* step(PyObject*, PyObject* const* args, Py_ssize_t n) {
       key->stride(1) != d.dim || value->stride(1) != d.dim || !d.kc->is_contiguous() || !d.vc->is_contiguous() ||
       (d.ks && (!d.ks->is_contiguous() || !d.vs->is_contiguous())))
     Py_RETURN_NONE;
-  at::Tensor out = at::empty_like(*d.q);
-  const Strides skey(key), sval(value), sq(d.q), sk(d.kc), sv(d.vc), sks(d.ks), svs(d.vs), sbt(d.bt), so(&out);
-  const int rc = prism_paged_decode_step(
-      key->data_ptr(), value->data_ptr(), skey.v, sval.v, static_cast<const int32_t*>(slots->data_ptr()),
-      d.q->data_ptr(), d.qd, sq.v, d.kc->data_ptr(), d.vc->data_ptr(), d.cd, sk.v, sv.v,
-      const_cast<float*>(scales(d.ks)), const_cast<float*>(scales(d.vs)), sks.v, svs.v,
-      static_cast<const int32_t*>(d.bt->data_ptr()), sbt.v, static_cast<const int32_t*>(d.ctx->data_ptr()),
-      static_cast<const int32_t*>(d.max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(d.batch),
-      static_cast<int>(d.heads), static_cast<int>(d.kv_heads), static_cast<int>(d.dim), static_cast<int>(d.page),
-      d.blocks, static_cast<int>(d.width), static_cast<float>(d.scale), d.ws, d.need, d.stream);
+  at::Tensor out;
+  int rc;
+  {
+    WithoutGil released;
+    out = at::empty_like(*d.q);
+    const Strides skey(key), sval(value), sq(d.q), sk(d.kc), sv(d.vc), sks(d.ks), svs(d.vs), sbt(d.bt), so(&out);
+    rc = prism_paged_decode_step(
+        key->data_ptr(), value->data_ptr(), skey.v, sval.v, static_cast<const int32_t*>(slots->data_ptr()),
+        d.q->data_ptr(), d.qd, sq.v, d.kc->data_ptr(), d.vc->data_ptr(), d.cd, sk.v, sv.v,
+        const_cast<float*>(scales(d.ks)), const_cast<float*>(scales(d.vs)), sks.v, svs.v,
+        static_cast<const int32_t*>(d.bt->data_ptr()), sbt.v, static_cast<const int32_t*>(d.ctx->data_ptr()),
+        static_cast<const int32_t*>(d.max_ctx->data_ptr()), out.data_ptr(), so.v, static_cast<int>(d.batch),
+        static_cast<int>(d.heads), static_cast<int>(d.kv_heads), static_cast<int>(d.dim), static_cast<int>(d.page),
+        d.blocks, static_cast<int>(d.width), static_cast<float>(d.scale), d.ws, d.need, d.stream);
+  }
   if (rc != PRISM_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -288,25 +319,25 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int page = static_cast<int>(kc->size(1)), width = static_cast<int>(bt->size(1));
   const int64_t need = prism_paged_prefill_workspace_bytes(static_cast<int>(batch), static_cast<int>(total),
                                                            static_cast<int>(heads), static_cast<int>(kv_heads), page, width);
-  at::Tensor out = at::empty(q->sizes(), q->options());
-  at::Tensor ws;
-  if (need > 0) ws = at::empty({need}, q->options().dtype(at::kByte));
-  const Strides sq(q), sk(kc), sv(vc), sks(ks), svs(vs), sbt(bt), so(&out);
+  at::Tensor out, ws;
   int32_t* words = static_cast<int32_t*>(report->data_ptr());
   words[0] = 0;  // (the thread's previous call on this stream has been waited for)
-  const int rc = prism_paged_prefill_ws(
-      q->data_ptr(), qd, sq.v, kc->data_ptr(), vc->data_ptr(), PRISM_DTYPE_FP8_E4M3FN, sk.v, sv.v, scales(ks), scales(vs),
-      sks.v, svs.v, static_cast<const int32_t*>(bt->data_ptr()), sbt.v, static_cast<const int32_t*>(ctx->data_ptr()),
-      static_cast<const int32_t*>(cu->data_ptr()), out.data_ptr(), so.v, static_cast<int>(batch), static_cast<int>(total),
-      static_cast<int>(heads), static_cast<int>(kv_heads), static_cast<int>(dim), page, static_cast<int>(kc->size(0)),
-      width, static_cast<float>(scale), static_cast<int32_t*>(status->data_ptr()), need > 0 ? ws.data_ptr() : nullptr,
-      need, words, stream);
+  int rc;
+  {
+    WithoutGil released;
+    out = at::empty(q->sizes(), q->options());
+    if (need > 0) ws = at::empty({need}, q->options().dtype(at::kByte));
+    const Strides sq(q), sk(kc), sv(vc), sks(ks), svs(vs), sbt(bt), so(&out);
+    rc = prism_paged_prefill_ws(
+        q->data_ptr(), qd, sq.v, kc->data_ptr(), vc->data_ptr(), PRISM_DTYPE_FP8_E4M3FN, sk.v, sv.v, scales(ks),
+        scales(vs), sks.v, svs.v, static_cast<const int32_t*>(bt->data_ptr()), sbt.v,
+        static_cast<const int32_t*>(ctx->data_ptr()), static_cast<const int32_t*>(cu->data_ptr()), out.data_ptr(), so.v,
+        static_cast<int>(batch), static_cast<int>(total), static_cast<int>(heads), static_cast<int>(kv_heads),
+        static_cast<int>(dim), page, static_cast<int>(kc->size(0)), width, static_cast<float>(scale),
+        static_cast<int32_t*>(status->data_ptr()), need > 0 ? ws.data_ptr() : nullptr, need, words, stream);
+    if (rc == PRISM_OK) C10_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+  }
   if (rc != PRISM_OK) Py_RETURN_NONE;
-  hipError_t err;
-  Py_BEGIN_ALLOW_THREADS
-  err = hipStreamSynchronize(static_cast<hipStream_t>(stream));
-  Py_END_ALLOW_THREADS
-  C10_HIP_CHECK(err);
   const volatile int32_t* r = words;
   const int row0 = r[1], row1 = r[2];
   const int bad = r[0] == 0 ? INT32_MAX : status->item<int32_t>();

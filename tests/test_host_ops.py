@@ -8,7 +8,9 @@ run as before.  The CPU tests need the built extension only.
 
 from __future__ import annotations
 
+import sys
 import threading
+import time
 from types import SimpleNamespace
 
 import pytest
@@ -233,3 +235,51 @@ def test_prefill_both_paths_errors_and_threads(python_path, native_calls):
     for t in threads:
         t.join()
     assert len(results) == 15 and all(torch.equal(r, _bytes(python)) for r in results)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["store", "decode", "step"])
+def test_other_threads_run_during_launches(native_calls, op):
+    """A launch may wait for room in the queue: the native path gives up the GIL over it, as ctypes does.
+
+    The interpreter's own switching is off meanwhile, so another thread advances only where a call lets it.
+    """
+
+    require_gpu()
+    from prism_infer.engine.decode_attention import PagedKVDecodeAttention, pack_decode_metadata
+
+    q, k, v, tables, lens, ks, vs = _decode_case(torch.bfloat16, FP8)
+    key = q[:, :4].contiguous()
+    layer = PagedKVDecodeAttention(8, 4, 128, 0.1)
+    layer.k_cache, layer.v_cache, layer.k_scale_cache, layer.v_scale_cache = k, v, ks, vs
+    meta = pack_decode_metadata([5, 77, 400], [6, 70, 33], tables.cpu(), device="cuda")
+    bound = torch.tensor(60, dtype=torch.int32, device="cuda")
+    call = {"store": lambda: kv_cache_store.store_kvcache(key, key, k, v, lens, ks, vs),
+            "decode": lambda: paged_decode.paged_decode_attention(q, k, v, tables, lens, 0.1, max_context_len=bound),
+            "step": lambda: layer(q, key, key, meta)}[op]
+    call()
+    call()
+    torch.cuda.synchronize()
+    passes, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            passes[0] += 1
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    thread.start()
+    try:
+        sys.setswitchinterval(1000.0)
+        before = passes[0]
+        for _ in range(20000):
+            call()
+        ran = passes[0] - before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()
+        torch.cuda.synchronize()
+    print(f"{op}: {ran} passes of another thread in 20000 calls", flush=True)
+    assert ran > 1000  # (with the GIL held the calls let 2 to 19 passes through, without it 285000 to 460000)
