@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import importlib.machinery
 import importlib.util
+import warnings
 from pathlib import Path
 
 import torch
@@ -136,10 +137,12 @@ _HOST_OPS_TRIED = False
 
 
 def host_ops():
-    """The extension that checks and launches the per-layer ops in C++, or None where it is not built.
+    """The extension that checks and launches the per-layer ops in C++, or None where it is not built or does not load.
 
     Each of its functions returns None for a call it does not take; the ops'
-    Python code then handles it.
+    Python code then handles it.  An extension that does not load (built
+    against another torch) is reported once: the Python code launches the same
+    kernels.
     """
 
     global _HOST_OPS, _HOST_OPS_TRIED
@@ -151,8 +154,10 @@ def host_ops():
                 module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_ops", loader))
                 loader.exec_module(module)
             except ImportError as exc:
-                raise RuntimeError(f"cannot load {HOST_OPS_PATH}: {exc}") from exc
-            _HOST_OPS = module
+                warnings.warn(f"the ops run their slower Python path: cannot load {HOST_OPS_PATH}: {exc}",
+                              RuntimeWarning, stacklevel=2)
+            else:
+                _HOST_OPS = module
     return _HOST_OPS
 
 

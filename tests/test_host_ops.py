@@ -11,6 +11,7 @@ from __future__ import annotations
 import sys
 import threading
 import time
+import warnings
 from types import SimpleNamespace
 
 import pytest
@@ -75,6 +76,21 @@ def test_cpu_tensors_and_odd_arguments_are_left_to_python():
     assert host.store(t, t) is None
     assert host.decode(t, c, c, s, s, 1.0, None, None, s, 32, {}) is None
     assert host.prefill(t, c, c, s, s, s, 1, 1, 1.0, None, None, {}) is None
+
+
+def test_an_extension_that_does_not_load_leaves_the_python_path(monkeypatch, tmp_path):
+    if not _native.available():
+        pytest.skip("the library is not built")
+    broken = tmp_path / "_host_ops.so"
+    broken.write_bytes(b"not a shared object")
+    monkeypatch.setattr(_native, "HOST_OPS_PATH", broken)
+    monkeypatch.setattr(_native, "_HOST_OPS", None)
+    monkeypatch.setattr(_native, "_HOST_OPS_TRIED", False)
+    with pytest.warns(RuntimeWarning, match="Python path"):
+        assert _native.host_ops() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _native.host_ops() is None
 
 
 def _bytes(x):
