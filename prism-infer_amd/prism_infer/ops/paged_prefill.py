@@ -61,12 +61,14 @@ def _outcome_buffers() -> dict:
 
 
 def _add_outcome_buffers(buffers: dict, device: torch.device) -> None:
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    key = (index, torch.cuda.current_stream(device).cuda_stream)
+    if key in buffers:  # a call of a form that stays here, on a stream that has them
+        return
     if len(buffers) >= _MAX_OUTCOME_STREAMS:
         buffers.clear()
-    index = device.index if device.index is not None else torch.cuda.current_device()
     status = torch.full((1,), _STATUS_OK, dtype=torch.int32, device=device)
-    buffers[(index, torch.cuda.current_stream(device).cuda_stream)] = (
-        status, torch.empty(3, dtype=torch.int32, pin_memory=True))
+    buffers[key] = (status, torch.empty(3, dtype=torch.int32, pin_memory=True))
 
 
 def _validate_caches(k_cache, v_cache, k_scale_cache, v_scale_cache) -> bool:

@@ -93,6 +93,27 @@ def test_an_extension_that_does_not_load_leaves_the_python_path(monkeypatch, tmp
         assert _native.host_ops() is None
 
 
+def test_prefill_outcome_buffers_are_made_once_per_stream(monkeypatch):
+    """Calls that the native path declines each time (int64 metadata, say) make no buffers after the first."""
+
+    stream, made = SimpleNamespace(cuda_stream=7), []
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: stream)
+    monkeypatch.setattr(torch, "full", lambda *a, **k: made.append("status") or object())
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: made.append("pinned") or object())
+    buffers: dict = {}
+    for _ in range(3):
+        paged_prefill._add_outcome_buffers(buffers, torch.device("cuda", 0))
+    assert made == ["status", "pinned"] and list(buffers) == [(0, 7)]
+    kept = buffers[(0, 7)]
+    for other in range(8, 8 + paged_prefill._MAX_OUTCOME_STREAMS - 1):
+        stream.cuda_stream = other
+        paged_prefill._add_outcome_buffers(buffers, torch.device("cuda", 0))
+    assert buffers[(0, 7)] is kept and len(buffers) == paged_prefill._MAX_OUTCOME_STREAMS
+    stream.cuda_stream = 99
+    paged_prefill._add_outcome_buffers(buffers, torch.device("cuda", 0))
+    assert list(buffers) == [(0, 99)]
+
+
 def _bytes(x):
     return x.contiguous().view(torch.uint8).cpu()
 
