@@ -276,9 +276,19 @@ int launch_held(uint8_t* cache, int64_t rows, int64_t num_slots, int64_t vec_byt
 
 // log2 of the held path's strip width in chunks, or -1 where the plan is too
 // large for it.  A strip covers whole 128-byte lines (or the whole of a
-// shorter vector) and grows while a workgroup holds few chunks (long vectors
-// with few entries: whole blocks); where the grid would leave CUs idle it
-// narrows to as little as 32 bytes.
+// shorter vector), also where that leaves CUs idle: narrower strips read and
+// write every line in parts (72 rows of 128 bytes, 2048 entries: 12.0 us in 72
+// workgroups, 14.9 with 64-byte strips, 37 with 32; 8 rows of 1 KB: 16.1, 18.1
+// and 33).  It grows while a workgroup holds few chunks (long vectors with few
+// entries: whole blocks; 72 rows of 4 KB, 512 entries: 67 us at 128 bytes, 61
+// at 256; 256 entries: 36.5 and 32.4) and every CU keeps a strip.
+//
+// The limit in entries is what a workgroup's registers hold.  Against the
+// staged path, 1 to 144 rows of 128 bytes to 4 KB: plans that overlap
+// themselves take 0.4 to 0.8 of its time up to the limit; plans that do not,
+// which it moves in one pass (the host cannot tell them), 0.5 to 1.08 up to
+// 1300 entries and, with one workgroup per CU, up to 1.14 at 1600 and 1.36 at
+// 2048.
 int held_strip_shift(int64_t rows, int64_t num_slots, int64_t vec_bytes, int64_t retained, int bytes) {
   const int64_t cpv = vec_bytes / bytes;
   auto strips = [&](int sh) { return ceil_div(cpv, int64_t{1} << sh) * rows; };
@@ -288,7 +298,6 @@ int held_strip_shift(int64_t rows, int64_t num_slots, int64_t vec_bytes, int64_t
   while ((int64_t{1} << shift) < cpv && (retained << (shift + 1)) <= kHeldWideChunks &&
          strips(shift + 1) >= device_cu_count())
     ++shift;
-  while ((int64_t{bytes} << shift) > 32 && strips(shift) < device_cu_count()) --shift;
   return shift;
 }
 

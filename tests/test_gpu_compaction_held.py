@@ -3,7 +3,7 @@
 Every plan overlaps itself (destinations that are other entries' sources), repeats a source, holds a no-op entry and
 entries out of range on either side (skipped).  Sizes: both sides of the 16384-chunk limit and of its half (entries
 x chunks of a 128-byte strip), vectors that are no power of two, shorter than a strip, of 4- and 1-byte chunks, long
-vectors with few entries (strips that widen) and few rows (strips that narrow).
+vectors with few entries (strips that widen) and few rows (fewer workgroups than CUs).
 """
 
 from __future__ import annotations
