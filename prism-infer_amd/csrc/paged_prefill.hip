@@ -167,14 +167,36 @@ struct PfWork {
   int seq, qblock, split, splits, head;
 };
 
+// Time of a launch, in units of 64 ns, whose longest block walks `tiles` tiles
+// in s parts.  A tile takes a workgroup 1.2 us, 1.7 where a CU holds eight
+// waves; parts cost a second launch and, for each of them, an fp32 row per
+// (token, query head) written and read again (0.34 ns a row).  Measured split
+// and not split, 1 to 8 query heads per kv head, 33 to 800 tokens behind 0 to
+// 4096: parts for every free slot took 1.5 times as long where rows are many
+// and tiles few (64 heads, 400 tokens: 41.7 against 27.8 us; 32 heads, 800
+// tokens: 38.2 and 29.7), 0.3 of the time where it is the other way round (32
+// heads, 33 tokens behind 4096: 27.6 and 91.9).
+__host__ __device__ inline int split_cost(int s, int tiles, int wgs, int waves, int slots, int rows) {
+  const int tile = waves == 8 || 2 * wgs * s > slots ? 27 : 19;
+  return tiles * tile / s + (s > 1 ? 47 + s * (rows / 190) : 0);
+}
+
 // Workgroup id -> work, from the number of real blocks: heads fastest (so that
 // the long blocks of all heads start first and, with 8 kv heads, each XCD
 // reads one head's K/V), then the parts of the keys, then the block's rank.
-// Returns the rank.  The keys are split as often as the chip has room for the
-// blocks' workgroups.
-__device__ __forceinline__ int pf_parts(const PrefillArgs& a, int kv_heads, int total, PfWork& w) {
+// Returns the rank.  The keys are split, if that pays, into the cheapest number
+// of parts that the chip has room for (lane s - 1 weighs s parts).
+template <int NW>
+__device__ __forceinline__ int pf_parts(const PrefillArgs& a, int kv_heads, int total, int tiles, PfWork& w) {
   w.splits = 1;
-  if (a.splits > 1 && total > 0) w.splits = uniform_int(min(max(a.slots / (total * kv_heads), 1), a.splits));
+  if (a.splits > 1 && total > 0) {
+    const int wgs = total * kv_heads;
+    const int s = static_cast<int>(__lane_id()) + 1;
+    constexpr int kMost = (1 << 24) - 1;
+    const int cost = min(split_cost(s, min(tiles, kMost / 27), wgs, NW, a.slots, a.total_q * a.num_heads), kMost);
+    const bool room = s == 1 || (s <= a.splits && s * wgs <= a.slots);
+    w.splits = 64 - (wave_reduce(room ? ((kMost - cost) << 6) | (64 - s) : 0, MaxInt()) & 63);
+  }
   const int per_block = kv_heads * w.splits;
   const int rank = uniform_int(static_cast<int>(blockIdx.x) / per_block);
   const int rest = static_cast<int>(blockIdx.x) - rank * per_block;
@@ -188,7 +210,7 @@ __device__ __forceinline__ int pf_parts(const PrefillArgs& a, int kv_heads, int 
 // the sequences; the rank's level comes from a binary search over u, its
 // sequence from a scan over those with a block at that level.  Returns false
 // for a workgroup beyond the real blocks.
-template <int QT>
+template <int QT, int NW>
 __device__ bool locate(const PrefillArgs& a, int kv_heads, bool flag, PfWork& w) {
   const int lane = __lane_id();
   if (a.batch <= 64) {  // one lane per sequence, loaded once
@@ -196,7 +218,7 @@ __device__ bool locate(const PrefillArgs& a, int kv_heads, bool flag, PfWork& w)
     const int n = lane < a.batch ? seq_blocks<QT>(a, lane, flag, l0) : 0;
     int lo = 0, hi = wave_reduce(n == 0 ? 0 : l0 + n, MaxInt());
     const int total = wave_reduce(n, AddInt());
-    const int rank = pf_parts(a, kv_heads, total, w);
+    const int rank = pf_parts<NW>(a, kv_heads, total, (hi - 1) * QT / kPfKT + 1, w);
     if (rank >= total) return false;
     auto above = [&](int u) { return min(max(l0 + n - 1 - max(u, l0 - 1), 0), n); };
     // smallest u in [0, hi] with at most `rank` blocks above level u
@@ -215,13 +237,14 @@ __device__ bool locate(const PrefillArgs& a, int kv_heads, bool flag, PfWork& w)
     return true;
   }
   // larger batches: sequence by sequence, in reverse
-  int total = 0, l0;
+  int total = 0, levels = 1, l0;
   for (int base = 0; base < a.batch; base += 64) {
     const int i = base + lane;
     const int n = i < a.batch ? seq_blocks<QT>(a, i, flag, l0) : 0;
     total += wave_reduce(n, AddInt());
+    levels = max(levels, wave_reduce(n == 0 ? 0 : l0 + n, MaxInt()));
   }
-  const int target = total - 1 - pf_parts(a, kv_heads, total, w);
+  const int target = total - 1 - pf_parts<NW>(a, kv_heads, total, (levels - 1) * QT / kPfKT + 1, w);
   if (target < 0) return false;
   int before = 0;
   for (int base = 0; base < a.batch; base += 64) {
@@ -323,7 +346,7 @@ paged_prefill_kernel(const PrefillArgs a) {
   __shared__ __attribute__((aligned(256))) uint8_t stages[4 * kStage];
 
   PfWork work;
-  const bool found = locate<QT>(a, a.num_heads / G, blockIdx.x == 0 && threadIdx.x < 64, work);
+  const bool found = locate<QT, NW>(a, a.num_heads / G, blockIdx.x == 0 && threadIdx.x < 64, work);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (a.splits > 1) *a.used = work.splits;
     if (a.report != nullptr) {
@@ -828,14 +851,20 @@ int64_t block_bound(int total_q, int batch, int groups) { return ceil_div(total_
 int64_t chip_slots(int groups) { return static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(groups); }
 
 // Most workgroups per (block, kv head), for the fewest blocks that total_q rows
-// make: where the blocks leave slots free, the keys are split, in parts of at
-// least 4 tiles of the longest context the tables can hold.  The kernel, which
-// sees the real number of blocks, takes as many as the slots allow.
+// make: where these leave slots free, parts of at least 4 tiles of the longest
+// context the tables can hold; 1 where no number of parts pays even for that
+// one (shorter contexts gain less).  The kernel chooses by the real blocks.
 int split_count(int total_q, int num_heads, int num_kv_heads, int64_t capacity) {
   const int groups = num_heads / num_kv_heads;
-  const int64_t wgs = ceil_div(total_q, pf_qtile(groups)) * num_kv_heads;
-  const int64_t s = std::min(chip_slots(groups) / wgs, capacity / (4 * kPfKT));
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(s, 64)));
+  const int64_t slots = chip_slots(groups), wgs = ceil_div(total_q, pf_qtile(groups)) * num_kv_heads;
+  const int most = static_cast<int>(std::min<int64_t>({slots / wgs, capacity / (4 * kPfKT), 64}));
+  const int tiles = static_cast<int>(std::min<int64_t>(ceil_div(capacity, kPfKT), 1 << 24));
+  auto cost = [&](int s) {  // (two parts or more: few workgroups, and so few rows)
+    return split_cost(s, tiles, static_cast<int>(wgs), pf_waves(groups), static_cast<int>(slots), total_q * num_heads);
+  };
+  for (int s = 2; s <= most; ++s)
+    if (cost(s) < cost(1)) return most;
+  return 1;
 }
 
 constexpr int64_t kPfPartOffset = 256;  // the partials follow the count of splits

@@ -19,7 +19,7 @@ from test_gpu_prefill import _case, _want
 pytestmark = pytest.mark.gpu
 
 
-def _run(c, split):
+def _run(c, split, parts=None):
     from prism_infer import _native
 
     lib, dev = _native.device_lib(torch.device("cuda", 0)), torch.device("cuda", 0)
@@ -47,6 +47,8 @@ def _run(c, split):
     _native.check(rc, "prefill")
     torch.cuda.synchronize()
     assert status.item() == 2**31 - 1
+    if parts is not None:
+        parts.append(ws.view(torch.int32)[0].item())  # the parts that the kernel chose
     return out.float().cpu()
 
 
@@ -86,3 +88,19 @@ def test_query_tiles_and_order(heads, kv):
     c = _case(20270300 + heads, seqs, num_heads=heads, num_kv_heads=kv, page=64)
     from test_gpu_prefill import _check
     _check(c, f"heads {heads}/{kv}")
+
+
+def test_parts_follow_the_contexts_and_not_the_tables():
+    """One table width (a 4800-token context's) serves all: the kernel weighs the real contexts."""
+
+    require_gpu()
+    chosen = {}
+    for context in (100, 600, 4700):
+        c, parts = _case(20270400, [(70, context), (30, 60)], num_heads=32, num_kv_heads=8, page=64), []
+        wide = torch.full((2, 75), -1, dtype=torch.int32)
+        wide[:, :c["tables"].shape[1]] = c["tables"]
+        c["tables"] = wide
+        _run(c, True, parts)
+        _both(c, f"context {context}")
+        chosen[context] = parts[0]
+    assert chosen[100] == 1 and 1 < chosen[600] < chosen[4700], chosen
