@@ -11,7 +11,8 @@
 // Work layout.  A workgroup owns one kv head and one block of query tokens of
 // one sequence; a wave owns 32 of the tokens and one of the G query heads of
 // the kv head, so each K/V tile is read once into LDS for all of them (4 waves:
-// 32 tokens for G = 4, 64 and 128 for G = 2 and 1; 8 waves for G = 8).  Tiles of 64 keys
+// 32 tokens for G = 4, 64 and 128 for G = 2 and 1; 8 waves for G = 8, or two
+// workgroups of four, by the length of the tables).  Tiles of 64 keys
 // go through four LDS stages: two tiles' loads are in flight beside the tile
 // whose scores and the one whose softmax are computed.  Per tile a wave computes S^T = K Q^T with
 // 32x32 MFMAs (bf16 queries: the fp8 MFMA 32x32x64 on the K bytes as they
@@ -330,8 +331,8 @@ __device__ __forceinline__ void pf_make_q(const u32x4 (&w)[2][4], PfQOperand<QDT
 }
 
 // Two waves per SIMD: at most 256 VGPRs + AGPRs per lane.
-// G: query heads per kv head; WHOLE: a tile lies in one page (page % 64 == 0),
-// else its 16-key groups are looked up one by one.
+// G: query heads of one kv head per workgroup; WHOLE: a tile lies in one page
+// (page % 64 == 0), else its 16-key groups are looked up one by one.
 constexpr int pf_waves(int g) { return g <= 4 ? 4 : 8; }
 constexpr int pf_qtile(int g) { return kPfCols * pf_waves(g) / g; }
 
@@ -355,14 +356,21 @@ paged_prefill_kernel(const PrefillArgs a) {
     }
   }
   if (!found) return;
-  const int seq = uniform_int(work.seq), qblock = uniform_int(work.qblock), h = uniform_int(work.head);
+  const int seq = uniform_int(work.seq), qblock = uniform_int(work.qblock);
+  // two workgroups of a kv head (G is half its group) are kv_heads apart: with 8 kv heads on one XCD
+  int h = uniform_int(work.head), qhead0 = h * G;
+  if (G == 4 && a.groups == 8) {
+    const int kv_heads = a.num_heads / 8, upper = h >= kv_heads;
+    h -= upper * kv_heads;
+    qhead0 = h * 8 + upper * G;
+  }
   const int split = uniform_int(work.split), splits = uniform_int(work.splits);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);  // uniform: SGPR arithmetic below
   const int lane = tid % 64;
   const int c = lane % 32;
   const int g = lane / 32;
-  const int qhead = h * G + wave % G;
+  const int qhead = qhead0 + wave % G;
 
   // sequence metadata in SGPRs: every branch on it below is uniform
   const int qs = __builtin_amdgcn_readfirstlane(a.cu_q[seq]);
@@ -843,24 +851,35 @@ __global__ void __launch_bounds__(256) paged_prefill_merge_kernel(const PrefillA
   dst[1] = (QDT == PRISM_DTYPE_F16) ? f32_to_f16_bits(o1 * inv) : f32_to_bf16_bits(o1 * inv);
 }
 
+// Query heads per workgroup: all of a kv head's, but 4 of 8 where the tables
+// hold few keys.  Eight waves fill a CU, so that a workgroup's lookup, loads
+// and output lie bare between its tiles; two of four waves hide each other's
+// and read the keys twice.  64 / 8 heads, pages of 256: a prompt of 16 tokens
+// 15.0 us with eight and 11.4 with four, 80 of 100 188 and 153, 4 of 2048 375
+// and 353, 300 tokens behind 1000 (16 sequences) 261 and 258; behind 2000 405
+// and 407, without scales 397 and 415; 4 x 2048 behind 8000 2290 and 2323,
+// without scales 2235 and 2360.
+constexpr int64_t kPfHalfKeys = 2048;
+int heads_per_wg(int groups, int64_t capacity) { return groups == 8 && capacity <= kPfHalfKeys ? 4 : groups; }
+
 // Query blocks that the launch provides for: every sequence may end in a
 // partial block.
-int64_t block_bound(int total_q, int batch, int groups) { return ceil_div(total_q, pf_qtile(groups)) + batch; }
+int64_t block_bound(int total_q, int batch, int g) { return ceil_div(total_q, pf_qtile(g)) + batch; }
 
 // Workgroups that the chip holds at once: the kernel fits eight waves on a CU.
-int64_t chip_slots(int groups) { return static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(groups); }
+int64_t chip_slots(int g) { return static_cast<int64_t>(device_cu_count()) * 8 / pf_waves(g); }
 
 // Most workgroups per (block, kv head), for the fewest blocks that total_q rows
 // make: where these leave slots free, parts of at least 4 tiles of the longest
 // context the tables can hold; 1 where no number of parts pays even for that
 // one (shorter contexts gain less).  The kernel chooses by the real blocks.
 int split_count(int total_q, int num_heads, int num_kv_heads, int64_t capacity) {
-  const int groups = num_heads / num_kv_heads;
-  const int64_t slots = chip_slots(groups), wgs = ceil_div(total_q, pf_qtile(groups)) * num_kv_heads;
+  const int g = heads_per_wg(num_heads / num_kv_heads, capacity);
+  const int64_t slots = chip_slots(g), wgs = ceil_div(total_q, pf_qtile(g)) * (num_heads / g);
   const int most = static_cast<int>(std::min<int64_t>({slots / wgs, capacity / (4 * kPfKT), 64}));
   const int tiles = static_cast<int>(std::min<int64_t>(ceil_div(capacity, kPfKT), 1 << 24));
   auto cost = [&](int s) {  // (two parts or more: few workgroups, and so few rows)
-    return split_cost(s, tiles, static_cast<int>(wgs), pf_waves(groups), static_cast<int>(slots), total_q * num_heads);
+    return split_cost(s, tiles, static_cast<int>(wgs), pf_waves(g), static_cast<int>(slots), total_q * num_heads);
   };
   for (int s = 2; s <= most; ++s)
     if (cost(s) < cost(1)) return most;
@@ -896,8 +915,8 @@ int launch_prefill(const PrefillArgs& a, bool scaled, hipStream_t stream) {
 }
 
 template <int QDT>
-int dispatch_groups(const PrefillArgs& a, bool scaled, hipStream_t stream) {
-  switch (a.groups) {
+int dispatch_groups(const PrefillArgs& a, int g, bool scaled, hipStream_t stream) {
+  switch (g) {
     case 1: return launch_prefill<QDT, 1>(a, scaled, stream);
     case 2: return launch_prefill<QDT, 2>(a, scaled, stream);
     case 4: return launch_prefill<QDT, 4>(a, scaled, stream);
@@ -1023,8 +1042,10 @@ extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t 
   a.report = report;
   a.out_vec = aligned(out, 8) && out_strides[0] % 4 == 0 && out_strides[1] % 4 == 0;
   a.total_q = total_q;
-  a.slots = static_cast<int>(chip_slots(num_heads / num_kv_heads));
-  a.splits = split_count(total_q, num_heads, num_kv_heads, static_cast<int64_t>(width) * page_size);
+  const int64_t capacity = static_cast<int64_t>(width) * page_size;
+  const int g = heads_per_wg(a.groups, capacity);
+  a.slots = static_cast<int>(chip_slots(g));
+  a.splits = split_count(total_q, num_heads, num_kv_heads, capacity);
   // without scratch for the partials the keys are not split
   if (a.splits > 1 &&
       (workspace == nullptr || !aligned(workspace, 16) || workspace_bytes < split_workspace(a.splits, total_q, num_heads)))
@@ -1033,8 +1054,8 @@ extern "C" int prism_paged_prefill_ws(const void* q, int q_dtype, const int64_t 
   a.part = a.splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kPfPartOffset) : nullptr;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   const bool scaled = k_scale != nullptr;
-  if (q_dtype == PRISM_DTYPE_F16) return dispatch_groups<PRISM_DTYPE_F16>(a, scaled, stream);
-  return dispatch_groups<PRISM_DTYPE_BF16>(a, scaled, stream);
+  if (q_dtype == PRISM_DTYPE_F16) return dispatch_groups<PRISM_DTYPE_F16>(a, g, scaled, stream);
+  return dispatch_groups<PRISM_DTYPE_BF16>(a, g, scaled, stream);
 }
 
 extern "C" int prism_paged_prefill(const void* q, int q_dtype, const int64_t q_strides[3], const void* k_cache,

@@ -104,3 +104,21 @@ def test_parts_follow_the_contexts_and_not_the_tables():
         _both(c, f"context {context}")
         chosen[context] = parts[0]
     assert chosen[100] == 1 and 1 < chosen[600] < chosen[4700], chosen
+
+
+@pytest.mark.parametrize("qdtype,scaled,page", [(torch.bfloat16, True, 64), (torch.float16, True, 16),
+                                                (torch.bfloat16, False, 32), (torch.float16, False, 128)])
+@pytest.mark.parametrize("kv", [1, 3, 8])
+def test_eight_heads_a_kv_head_by_four_and_by_eight(kv, qdtype, scaled, page):
+    """Tables of up to 2048 keys give a workgroup four of the eight heads, wider ones all of them."""
+
+    require_gpu()
+    from test_gpu_prefill import _check
+    seqs = [(33, 2000), (1, 1), (64, 64), (17, 900)]
+    c = _case(20270500 + kv, seqs, num_heads=8 * kv, num_kv_heads=kv, qdtype=qdtype, scaled=scaled, page=page)
+    for width in (2048 // page, 2048 // page + 1):
+        wide = torch.full((len(seqs), width), -1, dtype=torch.int32)
+        n = min(width, c["tables"].shape[1])
+        wide[:, :n] = c["tables"][:, :n]
+        _check(dict(c, tables=wide), f"{width} pages of {page}")
+        _both(dict(c, tables=wide), f"{width} pages of {page}")
