@@ -384,7 +384,10 @@ template <int IN_DTYPE, int OUT_DTYPE>
 int launch_rows(const void* key, const void* value, int64_t k_tok_bytes, int64_t v_tok_bytes, void* k_cache,
                 void* v_cache, const int32_t* slots, int64_t num_tokens, int chunks, int64_t num_slots,
                 hipStream_t stream) {
-  // four tokens per block; one where the tokens alone would leave most CUs without a block
+  // Four tokens per block; one where the tokens alone would leave most CUs
+  // without a block.  One and four: 8 x 128 float32, 256 tokens 3.1 and 3.8 us,
+  // 1023 5.2 and 5.4, 2048 8.8 and 8.7; bf16, up to 1023 tokens within 0.2 us,
+  // 2048 5.2 and 4.6, 3001 6.3 and 5.6; 1 x 128, 8192 tokens 5.0 and 4.1.
   const int waves = num_tokens >= 1024 ? 4 : 1;
   const int64_t blocks = ceil_div(num_tokens, waves);
   if (blocks > INT32_MAX) {

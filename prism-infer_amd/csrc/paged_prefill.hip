@@ -443,7 +443,7 @@ paged_prefill_kernel(const PrefillArgs a) {
                  : : "v"(off), "s"(uniform_ptr(base)), "s"(lds) : "memory", "m0");
   };
   // Starts tile t's loads into stage st; returns whether all of a full tile's
-  // loads were issued.
+  // loads were issued (wait_tiles counts on their number).
   auto issue_tile = [&](int t, uint8_t* st) -> bool {
     constexpr int kGroups = WHOLE ? 1 : kPfKT / 16;  // table lookups per tile
     constexpr int kGroupRows = kPfKT / kGroups;
@@ -515,8 +515,10 @@ paged_prefill_kernel(const PrefillArgs a) {
   // place, while the tile before it is computed: a score times its entry is
   // the exponent.
   auto scale_slot = [&](uint32_t st) { return reinterpret_cast<float*>(stages + st + 2 * kPayload) + lane; };
-  // Waits for this wave's loads but those of the last tile issued (`full`: it
-  // issued all of them; else for all).
+  // Waits for this wave's loads but those of the last tile issued.  They are
+  // counted: a wave issues exactly kLoads loads for a tile, waves 0 and 1 one
+  // more for its scales, whenever issue_tile returns true (`full`); otherwise,
+  // and where no tile was issued, it waits for all.
   auto wait_tiles = [&](bool full) {
     constexpr int kLoads = 2 * kPfKT / 8 / NW;
     if (!full) __builtin_amdgcn_s_waitcnt(0xF70);                              // vmcnt(0)

@@ -9,10 +9,12 @@ source slot ``src[i]`` held before the call -- all reads precede all writes,
 so overlapping in-place plans are safe.  Payload and scale caches are moved
 by separate calls, exactly as the reference's caller does.
 
-The native side first detects on the device whether any destination aliases
-another entry's source; only then does it stage through the workspace (two
-passes), otherwise it moves each slot once.  Every dtype goes through the
-same byte-moving kernels on the GPU.  A CPU cache is compacted with torch
+Plans whose entries fit a workgroup's registers (2048 token rows of 1 KB, 8192
+scale rows) move in one launch that reads everything before it writes.  For
+larger plans the native side first detects on the device whether any
+destination aliases another entry's source; only then does it stage through
+the workspace (two passes), otherwise it moves each slot once.  Every dtype
+goes through the same byte-moving kernels on the GPU.  A CPU cache is compacted with torch
 index ops over a byte view of the cache (the reference uses index ops for CPU
 and non-FP8 caches, :105-112).
 """
