@@ -30,6 +30,7 @@
 #include <atomic>
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "fp8_mfma.h"
@@ -165,10 +166,20 @@ __device__ __forceinline__ void store_out8(const Args& a, int64_t idx, const flo
 struct TileRegs {
   u32x4 k[2][2];   // [half][part]: 32 bytes of K row (c + 16 * half), dims 32g..32g+31
   u32x2 v[8];      // V rows of tokens {4g+i, 16+4g+i}, dims 8c..8c+7
-  float scale;     // lanes 0..31: k scale of token t0 + lane, lanes 32..63: v scales
+  float scale;     // lane (g, c): the k scale (c < 8) or v scale of slot c % 8's token
   uint32_t kvalid; // bit e: token of slot e is attended
   int base;        // first cache slot of the tile (a tile in one page; INT_MIN: absent block)
 };
+
+// v of lanes FIRST .. FIRST + 7 of the lane's 16-lane row.
+template <int FIRST, int... E>
+__device__ __forceinline__ void row_bcast_each(float v, float (&out)[8], std::integer_sequence<int, E...>) {
+  ((out[E] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + FIRST + E, 0xF, 0xF, false))), ...);  // row_newbcast
+}
+template <int FIRST>
+__device__ __forceinline__ void row_bcast8(float v, float (&out)[8]) {
+  row_bcast_each<FIRST>(v, out, std::make_integer_sequence<int, 8>{});
+}
 
 // Token order of the 8 per-lane "slots": e < 4 -> 4g + e; e >= 4 -> 16 + 4g + (e - 4).
 __device__ __forceinline__ int slot_token(int g, int e) { return (e < 4) ? (4 * g + e) : (16 + 4 * g + e - 4); }
@@ -196,13 +207,12 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
       r.k[hh][0] = p[0];
       r.k[hh][1] = p[1];
     }
-    // the tile's 64 scales in one load: lane l < 32 token l's k scale, lane
-    // 32 + l its v scale (one load per token a lane weighs was 16 of the 28
-    // loads of a tile)
+    // the tile's 64 scales in one load, each in the 16 lanes that weigh its
+    // token (one load per token a lane weighs was 16 of the 28 loads of a tile)
     r.scale = 1.f;
     if (SCALED) {
-      const int64_t tok = off0 + (c + 16 * (g & 1));
-      r.scale = g < 2 ? a.ks[blk * a.ks_sblk + tok * a.ks_stok + h * a.ks_sh]
+      const int64_t tok = off0 + slot_token(g, c & 7);
+      r.scale = c < 8 ? a.ks[blk * a.ks_sblk + tok * a.ks_stok + h * a.ks_sh]
                       : a.vs[blk * a.vs_sblk + tok * a.vs_stok + h * a.vs_sh];
     }
 #pragma unroll
@@ -215,13 +225,13 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
     // Tiles may straddle pages: resolve every row separately.
     r.scale = SCALED ? 0.f : 1.f;
     if (SCALED) {
-      const int tok = t0 + c + 16 * (g & 1);
+      const int tok = t0 + slot_token(g, c & 7);
       if (tok < t_end) {
         const int page = tok / a.page_size;
         const int64_t off = tok - page * a.page_size;
         const int32_t blk = bt_row[page * a.bt_sn];
         if (blk >= 0 && blk < a.num_blocks)
-          r.scale = g < 2 ? a.ks[blk * a.ks_sblk + off * a.ks_stok + h * a.ks_sh]
+          r.scale = c < 8 ? a.ks[blk * a.ks_sblk + off * a.ks_stok + h * a.ks_sh]
                           : a.vs[blk * a.vs_sblk + off * a.vs_stok + h * a.vs_sh];
       }
     }
@@ -507,7 +517,6 @@ paged_decode_split_kernel(const DecodeArgs a) {
   const int c_end = min(c_begin + a.split, n_eff);
   const int n_live = (n_eff + a.split - 1) / a.split;  // chunks with attended tokens (>= 1)
 
-  __shared__ __attribute__((aligned(16))) float s_scale[kSplitWaves][64];
   floatx4 acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -621,8 +630,8 @@ paged_decode_split_kernel(const DecodeArgs a) {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             if (v_group && e == ve) cur.v[e] = vq;
-          if (lane == t) cur.scale = ks;
-          if (lane == 32 + t) cur.scale = vs;
+          if (v_group && c == ve) cur.scale = ks;
+          if (v_group && c == 8 + ve) cur.scale = vs;
         }
       }
     };
@@ -633,15 +642,6 @@ paged_decode_split_kernel(const DecodeArgs a) {
         const uint64_t hit = __builtin_amdgcn_ballot_w64(slot_l >= cur.base && slot_l < cur.base + kTile);
         if (hit != 0) patch(cur, hit);
       }
-      // The scales change hands through the wave's own LDS (no barrier: only
-      // this wave reads them, in order behind its write).
-      float ksc[8], vsc[8];
-      if constexpr (CB == 1 && SCALED) {
-        __builtin_amdgcn_wave_barrier();
-        s_scale[wv][lane] = cur.scale;
-        __builtin_amdgcn_wave_barrier();
-      }
-
       // ---- QK
       floatx4 sc[2];
 #pragma unroll
@@ -673,14 +673,14 @@ paged_decode_split_kernel(const DecodeArgs a) {
         sc[hh] = accs;
       }
 
+      // Slot e's scales are in lanes e and 8 + e of every 16-lane row: broadcast
+      // by DPP.  (Through the wave's LDS, written in front of QK: 11.2 us for 1
+      // x 1800 tokens, 36 layers cold 12.2;
+      // a load per token 10.8 and 11.8; here 10.45.)
+      float ksc[8], vsc[8];
       if constexpr (CB == 1 && SCALED) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const floatx4 kq = *reinterpret_cast<const floatx4*>(&s_scale[wv][16 * q + 4 * g]);
-          const floatx4 vq = *reinterpret_cast<const floatx4*>(&s_scale[wv][32 + 16 * q + 4 * g]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) ksc[4 * q + i] = kq[i], vsc[4 * q + i] = vq[i];
-        }
+        row_bcast8<0>(cur.scale, ksc);
+        row_bcast8<8>(cur.scale, vsc);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) ksc[e] = vsc[e] = 1.f;

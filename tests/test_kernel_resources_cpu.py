@@ -42,3 +42,16 @@ def test_main_path_kernels_do_not_spill():
     spilled = {name: k[".vgpr_spill_count"] for name, k in kernels.items()
                if k[".vgpr_spill_count"] and not any(part in name for part in MAY_SPILL)}
     assert not spilled
+
+
+def test_split_decode_passes_scales_between_lanes_without_lds():
+    """Scales that went through LDS in front of the scores cost a decode of one tile per wave 0.4 us of 11."""
+
+    if not _native.available():
+        pytest.skip("the library is not built")
+    lds = {}
+    for name, k in _kernels().items():
+        if "paged_decode_split_kernel" in name:
+            lds.setdefault("Lb1E" if "paged_decode_split_kernelILi1ELb1E" in name else "other", set()).add(
+                k[".group_segment_fixed_size"])
+    assert lds["Lb1E"] and lds["Lb1E"] <= lds["other"], lds
