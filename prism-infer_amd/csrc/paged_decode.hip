@@ -674,9 +674,8 @@ paged_decode_split_kernel(const DecodeArgs a) {
       }
 
       // Slot e's scales are in lanes e and 8 + e of every 16-lane row: broadcast
-      // by DPP.  (Through the wave's LDS, written in front of QK: 11.2 us for 1
-      // x 1800 tokens, 36 layers cold 12.2;
-      // a load per token 10.8 and 11.8; here 10.45.)
+      // by DPP.  1 x 1800 tokens 10.45 us; through the wave's LDS, written in
+      // front of QK, 11.2; with a load per token 10.8.
       float ksc[8], vsc[8];
       if constexpr (CB == 1 && SCALED) {
         row_bcast8<0>(cur.scale, ksc);

@@ -7,6 +7,7 @@ kernel).  A spill is a round trip to memory in the inner loop or behind a prolog
 
 from __future__ import annotations
 
+import re
 import struct
 
 import pytest
@@ -49,9 +50,6 @@ def test_split_decode_passes_scales_between_lanes_without_lds():
 
     if not _native.available():
         pytest.skip("the library is not built")
-    lds = {}
-    for name, k in _kernels().items():
-        if "paged_decode_split_kernel" in name:
-            lds.setdefault("Lb1E" if "paged_decode_split_kernelILi1ELb1E" in name else "other", set()).add(
-                k[".group_segment_fixed_size"])
-    assert lds["Lb1E"] and lds["Lb1E"] <= lds["other"], lds
+    lds = {scaled: {k[".group_segment_fixed_size"] for name, k in _kernels().items()
+                    if re.search(rf"paged_decode_split_kernelILi\dELb{scaled}E", name)} for scaled in (0, 1)}
+    assert lds[1] and lds[1] <= lds[0], lds
