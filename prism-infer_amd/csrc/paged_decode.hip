@@ -3837,13 +3837,20 @@ int decode_call(
     // The store joins the split-K kernel in its main forms: scaled FP8 or a
     // 16-bit cache of the query's dtype, tiles within a page, aligned dense
     // rows, at most one slot per lane, and the contiguous cache that the store
-    // addresses by slot.  Everything else takes two launches.
+    // addresses by slot.  Everything else takes two launches, and so do grids
+    // of more than a workgroup per CU where each wave has one tile: the second
+    // round waits for what the store adds to the first (33 sequences of 200
+    // tokens, 8 kv heads: 16.3 us against 14.7 in two launches, 24 x 500 20.0
+    // and 19.05, 33 x 1000 with 2 kv heads 19.8 and 18.5; at one round, 32 x 200,
+    // 9.3 and 10.1; with several tiles, 9 x 2500 of 4000, 21.4 and 22.9).
     const int64_t tok = static_cast<int64_t>(num_kv_heads) * kHeadDim;
     auto canonical = [&](const int64_t* st) { return st[0] == tok * page_size && st[1] == tok && st[2] == kHeadDim; };
     auto canonical_scales = [&](const int64_t* st) {
       return st[0] == static_cast<int64_t>(num_kv_heads) * page_size && st[1] == num_kv_heads && st[2] == 1;
     };
-    step->taken = geo.fast && !use_stream && page_aligned && args.q_vec && batch <= 64 &&
+    const bool rounds = static_cast<int64_t>(batch) * num_kv_heads * geo.max_splits > device_cu_count() &&
+                        geo.split <= kSplitWaves * kTile;
+    step->taken = geo.fast && !use_stream && !rounds && page_aligned && args.q_vec && batch <= 64 &&
                   (q_dtype == PRISM_DTYPE_BF16 || q_dtype == PRISM_DTYPE_F16) &&
                   (k_scale ? canonical_scales(ks_strides) && canonical_scales(vs_strides) : cache_dtype == q_dtype) &&
                   canonical(k_strides) && canonical(v_strides) && num_blocks * page_size <= INT32_MAX &&

@@ -1,7 +1,7 @@
 """The decode step's one launch (store inside the split-K kernel) against the two ops, byte for byte.
 
 Forms: scaled FP8 and 16-bit caches, bf16 and f16, GQA groups 1 to 16, pages of 32 to 256 tokens, batches up to the
-64 slots a wave holds and above (two launches); contexts that end on a tile's first and last row, one-token and empty
+64 slots a wave holds and grids up to a workgroup per CU, and above (two launches); contexts that end on a tile's first and last row, one-token and empty
 ones; slots that are skipped (-1, past the cache), that lie in another sequence's pages (which must then see the new
 row, as after a store) and in nobody's.  Old bytes under the new rows are NaN codes, so a row taken from memory too
 early cannot pass unnoticed.  The split-K family is forced, the native call must take the step, and a captured step
@@ -49,7 +49,7 @@ class _MustTake:
         return call
 
 
-def _check(batch, hkv, groups, page, width, dtype, scaled, lens, odd_slots=False, view=False):
+def _check(batch, hkv, groups, page, width, dtype, scaled, lens, odd_slots=False, view=False, launches=1):
     from prism_infer import _native
     from prism_infer.engine import decode_attention
     from prism_infer.engine.decode_attention import PagedKVDecodeAttention, pack_decode_metadata
@@ -100,7 +100,7 @@ def _check(batch, hkv, groups, page, width, dtype, scaled, lens, odd_slots=False
                 with pytest.MonkeyPatch.context() as m:
                     m.setattr(decode_attention, "_HOST", _MustTake(decode_attention._HOST))
                     out = layer(q, new_k, new_v, meta)
-                assert _launches(lambda: layer(q, new_k, new_v, meta)) == (1 if batch <= 64 else 2)
+                assert _launches(lambda: layer(q, new_k, new_v, meta)) == launches
             else:
                 out = layer(q, new_k, new_v, meta)
         else:
@@ -126,11 +126,14 @@ def test_fused_step_forms(dtype, scaled, hkv, groups, page):
     _check(len(lens), hkv, groups, page, width, dtype, scaled, lens, odd_slots=True, view=True)
 
 
-@pytest.mark.parametrize("batch", [1, 2, 63, 64, 65])
-def test_fused_step_batches(batch):
+@pytest.mark.parametrize("batch,hkv,width,launches", [
+    (1, 8, 5, 1), (2, 8, 5, 1), (63, 2, 5, 1), (64, 2, 5, 1), (65, 2, 5, 2),
+    (16, 8, 5, 1), (17, 8, 5, 2),  # chunks of a tile per wave: up to a workgroup per CU (of 256), and above
+    (9, 8, 33, 1)])                # more than that, with several tiles per wave
+def test_fused_step_batches(batch, hkv, width, launches):
     require_gpu()
-    lens = [1 + (37 * b) % 300 for b in range(batch)]
-    _check(batch, 8, 4, 64, 5, torch.bfloat16, True, lens, odd_slots=batch > 4)
+    lens = [1 + (37 * b) % 300 + 1700 * (width > 5) for b in range(batch)]
+    _check(batch, hkv, 4, 64, width, torch.bfloat16, True, lens, odd_slots=batch > 4, launches=launches)
 
 
 def test_fused_step_long_contexts_and_replay():
