@@ -166,9 +166,20 @@ __device__ __forceinline__ void store_out8(const Args& a, int64_t idx, const flo
 struct TileRegs {
   u32x4 k[2][2];   // [half][part]: 32 bytes of K row (c + 16 * half), dims 32g..32g+31
   u32x2 v[8];      // V rows of tokens {4g+i, 16+4g+i}, dims 8c..8c+7
-  float scale;     // lane (g, c): the k scale (c < 8) or v scale of slot c % 8's token
+  float scale;     // a k or v scale of the tile (ScaleLane)
   uint32_t kvalid; // bit e: token of slot e is attended
   int base;        // first cache slot of the tile (a tile in one page; INT_MIN: absent block)
+};
+
+// Which scale a lane loads.  ROWS: lane (g, c) slot c % 8's k scale (c < 8) or
+// v scale, so that every 16-lane row holds those it weighs; else lane t < 32
+// token t's k scale, lane 32 + t its v scale.
+template <bool ROWS>
+struct ScaleLane {
+  int token;
+  bool k;
+  __device__ ScaleLane(int c, int g)
+      : token(ROWS ? (c & 4) * 4 + 4 * g + (c & 3) : c + 16 * (g & 1)), k(ROWS ? c < 8 : g < 2) {}
 };
 
 // v of lanes FIRST .. FIRST + 7 of the lane's 16-lane row.
@@ -184,7 +195,7 @@ __device__ __forceinline__ void row_bcast8(float v, float (&out)[8]) {
 // Token order of the 8 per-lane "slots": e < 4 -> 4g + e; e >= 4 -> 16 + 4g + (e - 4).
 __device__ __forceinline__ int slot_token(int g, int e) { return (e < 4) ? (4 * g + e) : (16 + 4 * g + e - 4); }
 
-template <bool SCALED, bool PAGE_ALIGNED>
+template <bool SCALED, bool PAGE_ALIGNED, bool ROWS>
 __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int g, int c, int t0, int t_end,
                                           TileRegs& r, int32_t blk_pre = -1, bool use_pre = false) {
   const int32_t* bt_row = a.bt + static_cast<int64_t>(b) * a.bt_sb;
@@ -207,12 +218,13 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
       r.k[hh][0] = p[0];
       r.k[hh][1] = p[1];
     }
-    // the tile's 64 scales in one load, each in the 16 lanes that weigh its
-    // token (one load per token a lane weighs was 16 of the 28 loads of a tile)
+    // the tile's 64 scales in one load (one load per token a lane weighs was 16
+    // of the 28 loads of a tile)
     r.scale = 1.f;
     if (SCALED) {
-      const int64_t tok = off0 + slot_token(g, c & 7);
-      r.scale = c < 8 ? a.ks[blk * a.ks_sblk + tok * a.ks_stok + h * a.ks_sh]
+      const ScaleLane<ROWS> of(c, g);
+      const int64_t tok = off0 + of.token;
+      r.scale = of.k ? a.ks[blk * a.ks_sblk + tok * a.ks_stok + h * a.ks_sh]
                       : a.vs[blk * a.vs_sblk + tok * a.vs_stok + h * a.vs_sh];
     }
 #pragma unroll
@@ -225,13 +237,14 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, int b, int h, int
     // Tiles may straddle pages: resolve every row separately.
     r.scale = SCALED ? 0.f : 1.f;
     if (SCALED) {
-      const int tok = t0 + slot_token(g, c & 7);
+      const ScaleLane<ROWS> of(c, g);
+      const int tok = t0 + of.token;
       if (tok < t_end) {
         const int page = tok / a.page_size;
         const int64_t off = tok - page * a.page_size;
         const int32_t blk = bt_row[page * a.bt_sn];
         if (blk >= 0 && blk < a.num_blocks)
-          r.scale = c < 8 ? a.ks[blk * a.ks_sblk + off * a.ks_stok + h * a.ks_sh]
+          r.scale = of.k ? a.ks[blk * a.ks_sblk + off * a.ks_stok + h * a.ks_sh]
                           : a.vs[blk * a.vs_sblk + off * a.vs_stok + h * a.vs_sh];
       }
     }
@@ -517,6 +530,8 @@ paged_decode_split_kernel(const DecodeArgs a) {
   const int c_end = min(c_begin + a.split, n_eff);
   const int n_live = (n_eff + a.split - 1) / a.split;  // chunks with attended tokens (>= 1)
 
+  constexpr bool kRowScales = !STORE;  // how a tile's scales change lanes: within 16-lane rows, or through LDS
+  __shared__ __attribute__((aligned(16))) float s_scale[kRowScales ? 1 : kSplitWaves][64];
   floatx4 acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -527,7 +542,7 @@ paged_decode_split_kernel(const DecodeArgs a) {
     // First tile's loads go out before the query is read and converted.
     Tile ta, tb;
     auto load = [&](int t, Tile& r, int32_t pre, bool use_pre) {
-      if constexpr (CB == 1) load_tile<SCALED, PAGE_ALIGNED>(a, b, h, g, c, t, c_end, r, pre, use_pre);
+      if constexpr (CB == 1) load_tile<SCALED, PAGE_ALIGNED, kRowScales>(a, b, h, g, c, t, c_end, r, pre, use_pre);
       else load_tile16<PAGE_ALIGNED>(a, b, h, g, c, t, c_end, r, pre, use_pre);
     };
     load(t0, ta, blk0, true);
@@ -630,8 +645,8 @@ paged_decode_split_kernel(const DecodeArgs a) {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             if (v_group && e == ve) cur.v[e] = vq;
-          if (v_group && c == ve) cur.scale = ks;
-          if (v_group && c == 8 + ve) cur.scale = vs;
+          if (lane == t) cur.scale = ks;
+          if (lane == 32 + t) cur.scale = vs;
         }
       }
     };
@@ -642,6 +657,13 @@ paged_decode_split_kernel(const DecodeArgs a) {
         const uint64_t hit = __builtin_amdgcn_ballot_w64(slot_l >= cur.base && slot_l < cur.base + kTile);
         if (hit != 0) patch(cur, hit);
       }
+      // (no barrier: only this wave reads them, in order behind its write)
+      if constexpr (CB == 1 && SCALED && !kRowScales) {
+        __builtin_amdgcn_wave_barrier();
+        s_scale[wv][lane] = cur.scale;
+        __builtin_amdgcn_wave_barrier();
+      }
+
       // ---- QK
       floatx4 sc[2];
 #pragma unroll
@@ -675,11 +697,21 @@ paged_decode_split_kernel(const DecodeArgs a) {
 
       // Slot e's scales are in lanes e and 8 + e of every 16-lane row: broadcast
       // by DPP.  1 x 1800 tokens 10.45 us; through the wave's LDS, written in
-      // front of QK, 11.2; with a load per token 10.8.
+      // front of QK, 11.2; with a load per token 10.8.  With the store in the
+      // launch LDS is no slower for 8 kv heads (11.05 us) and faster for 2 (10.7
+      // against 11.05).
       float ksc[8], vsc[8];
-      if constexpr (CB == 1 && SCALED) {
+      if constexpr (CB == 1 && SCALED && kRowScales) {
         row_bcast8<0>(cur.scale, ksc);
         row_bcast8<8>(cur.scale, vsc);
+      } else if constexpr (CB == 1 && SCALED) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const floatx4 kq = *reinterpret_cast<const floatx4*>(&s_scale[wv][16 * q + 4 * g]);
+          const floatx4 vq = *reinterpret_cast<const floatx4*>(&s_scale[wv][32 + 16 * q + 4 * g]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ksc[4 * q + i] = kq[i], vsc[4 * q + i] = vq[i];
+        }
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) ksc[e] = vsc[e] = 1.f;

@@ -51,5 +51,5 @@ def test_split_decode_passes_scales_between_lanes_without_lds():
     if not _native.available():
         pytest.skip("the library is not built")
     lds = {scaled: {k[".group_segment_fixed_size"] for name, k in _kernels().items()
-                    if re.search(rf"paged_decode_split_kernelILi\dELb{scaled}E", name)} for scaled in (0, 1)}
+                    if re.search(rf"paged_decode_split_kernelILi\dELb{scaled}E.*ELb0EEE", name)} for scaled in (0, 1)}
     assert lds[1] and lds[1] <= lds[0], lds
