@@ -32,15 +32,19 @@
 // Few, long blocks (a short chunk behind a long prefix) leave most CUs idle:
 // the keys of a block are then split over several workgroups, which write
 // fp32 partials (max, sum, unnormalised output), merged by a second kernel
-// (330 tokens behind 12000-token prefixes, 32 / 8 heads: 371 us on 88
-// workgroups, 110 + 9.6 us on 440).
+// (267 tokens behind 12000-token prefixes, 32 / 8 heads: 371 us on 88
+// workgroups, 79 + 9.7 us split).
 //
-// Bound by VALU issue beside the MFMAs: per 32 x 32 scores of a wave the MFMAs
-// take 512 cycles (4 fp8 and 8 bf16) and the softmax, the
-// scales and the V conversion about 140 instructions.  With 16x16 MFMAs (four
-// lane groups per score column, outputs as query rows) the same work took
-// 193: 4 x 2048 tokens behind 8192, 32 / 8 heads, 1585 us against 1390 here
-// (890 TFLOP/s); 6 prompts of 61 to 1900 tokens, kernel 219 against 182 us.
+// Bound by VALU issue and dependency beside the MFMAs (busy 61% and 52% of the
+// cycles): per 32 x 32 scores of a wave the MFMAs take 512 cycles (4 fp8 and 8
+// bf16) and the softmax, the scales and the V conversion about 120
+// instructions.  With 16x16 MFMAs (four lane groups per score column, outputs
+// as query rows) the same work took 193: 4 x 2048 tokens behind 8192, 32 / 8
+// heads, 1585 us; 1390 with this layout, and 1120 to 1190 (1040 to 1100
+// TFLOP/s) with the next tile's scores spread over the softmax; 6 prompts of
+// 61 to 1900 tokens 219 and 166 us.  Workgroups of one or two tiles spend most
+// of their time on the lookup, the first loads and the masked tile, which costs
+// 2.2 settled ones: 80 prompts of 100 tokens take 81 us, 68 with 16x16 MFMAs.
 //
 // Metadata stays on the device: each workgroup finds its sequence and query
 // block from cu_seqlens_q with wave reductions, longest blocks first.
